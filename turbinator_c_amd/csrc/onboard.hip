@@ -36,10 +36,8 @@
 //     landing / standard / inversion / BWB laws, cannon) run in a second
 //     kernel from the parked scan results, both on one quad of lanes per
 //     environment (lane a evaluates arm a and a quarter of the independent
-//     transcendental calls).  The controller's long register-heavy chain is
-//     kept apart from the scan so both keep their occupancy, except where
-//     the batch is one round of 64-environment workgroups over most CUs
-//     (the onboard entry from 10,240 to 16,384 environments): there one
+//     transcendental calls), except where the workgroups of 64 environments
+//     fill the chip (the onboard entry from 8,192 environments): there one
 //     kernel does both, each workgroup scanning its own environments into
 //     LDS before their controller runs, which saves the second launch and
 //     the parked results' round trip.  The angles
@@ -63,6 +61,7 @@
 #include <type_traits>
 
 #include "turbinator/training/hip_features.h"
+#include "onboard_math.h"
 #include "recip_range.h"
 #include "xcd_order.h"
 
@@ -82,10 +81,9 @@ constexpr int kListRounds = kListCap / 64;
 constexpr unsigned kMaxBlocks = 1u << 20;
 constexpr int kStreamThreads = 1024;  // actor plane kernel: one workgroup per environment
 constexpr unsigned kScanBlocks = 256 * 4;   // persistent scan grid: 4 per CU
-// Controller grid cap: 4,096 workgroups of 64 environments.  One workgroup is
-// resident per CU (205 VGPRs), so the cap is 16 full rounds of the chip and
-// larger batches stride; a 16,384-environment call launches 256.
-constexpr unsigned kControlBlocks = 4096;
+// Widest row of the control kernel's grid; larger batches take more rows (a
+// launch's x extent is limited to 2^32 threads).
+constexpr unsigned kControlGridX = 1u << 20;
 constexpr size_t kMaxBatch = 0x7fffffffu;
 constexpr float kPi = 3.14159265358979323846f;
 
@@ -103,50 +101,54 @@ __device__ __forceinline__ float div_const(float x, float c) {
     return (float)((double)x * (1.0 / (double)c));
 }
 
-// onboard_features.cuh:6-22
+// onboard_features.cuh:6-22.  The tests are formed before the selects, so
+// they stay selects: as nested conditionals each became two branches.
+// TAME (onboard_math.h): no value is infinite or NaN.
+template <bool TAME = false>
 __device__ __forceinline__ float ob_clamp(float x, float lo, float hi) {
-    if (__builtin_isnan(x)) return x;
-    return fminf(hi, fmaxf(lo, x));
+    const float y = fminf(hi, fmaxf(lo, x));
+    if constexpr (TAME) return y;
+    const bool nan = __builtin_isnan(x);
+    return nan ? x : y;
 }
+__device__ __forceinline__ float finite_as(float x, float limit) {
+    const bool nan = __builtin_isnan(x), inf = __builtin_isinf(x);
+    const float y = inf ? copysignf(limit, x) : x;
+    return nan ? 0.0f : y;
+}
+template <bool TAME = false>
 __device__ __forceinline__ float ob_obs(float x) {
-    return __builtin_isnan(x) ? 0.0f : (__builtin_isinf(x) ? copysignf(1000.0f, x) : x);
+    return TAME ? x : finite_as(x, 1000.0f);
 }
+template <bool TAME = false>
 __device__ __forceinline__ float ob_mission(float x) {
-    return __builtin_isnan(x) ? 0.0f : (__builtin_isinf(x) ? copysignf(1.0f, x) : x);
+    return TAME ? x : finite_as(x, 1.0f);
 }
-// sinf and cosf of one argument through sincosf: one argument reduction
-// instead of two, and the same bits as the separate calls for every float
-// (checked over all 2^32 inputs on gfx950 by tests/csrc/check_sincos.hip).
-struct SinCos {
-    float s, c;
-};
-__device__ __forceinline__ SinCos sin_cos(float x) {
-    SinCos r;
-    sincosf(x, &r.s, &r.c);
-    return r;
-}
-// atan2 rounded correctly, for the angles that reach an angle wrap (yaw,
-// the goal and course bearings, the cannon azimuths, the outer gimbals).
-// ob_wrap is discontinuous where its two angles differ by pi, and that is
-// reached exactly by angles such as -3pi/4 and pi/4 (from equal or zero
-// components), or pi and a yaw of +-0: there one ulp of either angle flips
-// the wrapped error between about -pi and +pi and the controller's torques
-// with it.  The single-precision atan2f can be an ulp from the correctly
-// rounded value on such arguments; the host libm's atan2f, which the oracle
-// calls, is correctly rounded on them (equal, opposite and zero components,
-// results near +-pi: tests/csrc/check_atan2.hip), and so is the double
-// evaluation rounded once.  Elsewhere either libm may be an ulp off, which
-// moves the angles continuously.  The tactical terms and the wrap's own
-// atan2 depend on their angles continuously and keep atan2f.
+// atan2 and the angle wrap.  ob_wrap is discontinuous where its two angles
+// differ by pi, and that is reached exactly by angles such as -3pi/4 and pi/4
+// (from equal or zero components), or pi and a yaw of +-0: there one ulp of
+// either angle flips the wrapped error between about -pi and +pi and the
+// controller's torques with it.  The single-precision atan2f can be an ulp
+// from the correctly rounded value on such arguments; the host libm's
+// atan2f, which the oracle calls, is correctly rounded on them (equal,
+// opposite and zero components, results near +-pi: tests/csrc/
+// check_atan2.hip), and so is atan2_float (check_onboard_math.hip).
+// Elsewhere either may be an ulp off, which moves the angles continuously.
+template <bool TAME>
 __device__ __forceinline__ float ob_atan2(float y, float x) {
-    return (float)atan2((double)y, (double)x);
+    return onboard_math::atan2_float<TAME>(y, x);
 }
+template <bool TAME>
 __device__ __forceinline__ float ob_wrap(float target, float current) {
-    const SinCos d = sin_cos(target - current);
-    return atan2f(d.s, d.c);
+    return onboard_math::wrap_angle<TAME>(target - current);
 }
+template <bool TAME>
 __device__ __forceinline__ float ob_norm3(float x, float y, float z) {
-    return sqrtf(x * x + y * y + z * z);
+    return onboard_math::square_root<TAME>(x * x + y * y + z * z);
+}
+template <bool TAME>
+__device__ __forceinline__ float ob_hypot(float x, float y) {
+    return onboard_math::hypotenuse<TAME>(x, y);
 }
 
 // Normalised, sign-fixed attitude quaternion (onboard_features.cuh:105-109)
@@ -158,13 +160,14 @@ struct Attitude {
 
 __device__ __forceinline__ Attitude attitude_of(float o6, float o7, float o8, float o9) {
     Attitude a;
-    float qnorm = fmaxf(ob_norm3(o6, o7, o8), 0.0f);
+    float qnorm = fmaxf(sqrtf(o6 * o6 + o7 * o7 + o8 * o8), 0.0f);
     qnorm = fmaxf(sqrtf(qnorm * qnorm + o9 * o9), 1.0e-8f);
     const float sign = o6 < 0.0f ? -1.0f : 1.0f;
-    a.qw = sign * o6 / qnorm;
-    a.qx = sign * o7 / qnorm;
-    a.qy = sign * o8 / qnorm;
-    a.qz = sign * o9 / qnorm;
+    const onboard_math::Divisor over(qnorm);  // the IEEE quotients
+    a.qw = over(sign * o6);
+    a.qx = over(sign * o7);
+    a.qy = over(sign * o8);
+    a.qz = over(sign * o9);
     const float qw = a.qw, qx = a.qx, qy = a.qy, qz = a.qz;
     a.r[0] = 1.0f - 2.0f * (qy * qy + qz * qz);
     a.r[1] = 2.0f * (qx * qy - qw * qz);
@@ -640,29 +643,93 @@ __device__ __forceinline__ Quad4 quad_all(float v) {
     return Quad4{{quad_lane<0>(v), quad_lane<1>(v), quad_lane<2>(v), quad_lane<3>(v)}};
 }
 
-// Quad lane a's choice among four values.
+// Quad lane a's choice among four values: three plain selects (as a nested
+// conditional it became branches with the values' computation inside).
 __device__ __forceinline__ float quad_pick(int a, float v0, float v1, float v2, float v3) {
-    return a == 0 ? v0 : (a == 1 ? v1 : (a == 2 ? v2 : v3));
+    const bool odd = (a & 1) != 0, high = (a & 2) != 0;
+    const float lo = odd ? v1 : v0;
+    const float hi = odd ? v3 : v2;
+    return high ? hi : lo;
+}
+
+// The staged inputs that a lane of the control kernel's two chains reads,
+// taken from LDS all at once: an empty asm on each value keeps the compiler
+// from sinking its read to the first use, where every read would cost the
+// chain its own LDS round trip.  `head` is obs[0..12], `arm` the lane's arm's
+// four values obs[16 + 4 k + a], `tail` obs[40], obs[41], obs[44..47].
+struct ChainInputs {
+    float head[13], arm[4], tail[6], m[10];
+};
+
+__device__ __forceinline__ ChainInputs chain_inputs(const float *obs, const float *mission, int a) {
+    ChainInputs in;
+#pragma unroll
+    for (int i = 0; i < 13; ++i) in.head[i] = obs[i];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) in.arm[k] = obs[16 + 4 * k + a];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) in.tail[k] = obs[k < 2 ? 40 + k : 42 + k];
+#pragma unroll
+    for (int i = 0; i < 10; ++i) in.m[i] = mission[i];
+#pragma unroll
+    for (int i = 0; i < 13; ++i) asm volatile("" : "+v"(in.head[i]));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(in.arm[k]));
+#pragma unroll
+    for (int k = 0; k < 6; ++k) asm volatile("" : "+v"(in.tail[k]));
+#pragma unroll
+    for (int i = 0; i < 10; ++i) asm volatile("" : "+v"(in.m[i]));
+    return in;
+}
+
+// Whether every value the active lanes read is finite and below
+// onboard_math::kTameMax: the sum of their squares is below its square.
+__device__ __forceinline__ bool tame_inputs(const ChainInputs &in) {
+    float s = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 13; ++i) s = __builtin_fmaf(in.head[i], in.head[i], s);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s = __builtin_fmaf(in.arm[k], in.arm[k], s);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s = __builtin_fmaf(in.tail[k], in.tail[k], s);
+#pragma unroll
+    for (int i = 0; i < 10; ++i) s = __builtin_fmaf(in.m[i], in.m[i], s);
+    return __builtin_amdgcn_ballot_w64(
+               !(s < onboard_math::kTameMax * onboard_math::kTameMax)) == 0;
+}
+
+// The inputs as the controller reads them (onboard_features.cuh:12-22, 95-99).
+__device__ __forceinline__ void controller_inputs(ChainInputs &in) {
+#pragma unroll
+    for (int i = 0; i < 13; ++i) in.head[i] = ob_obs(in.head[i]);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) in.arm[k] = ob_obs(in.arm[k]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) in.tail[k] = ob_obs(in.tail[k]);
+#pragma unroll
+    for (int i = 0; i < 10; ++i) in.m[i] = ob_mission(in.m[i]);
 }
 
 // onboard_features.cuh:25-86 on the four lanes of a quad: lane a evaluates
 // arm a's thrust terms, and the independent calls of one function are spread
-// over the quad and broadcast (the three atanhf of the mission offsets; yaw
-// and the target bearing; the two hypotf and the two atan2f of the aim;
-// eight tanhf in two calls), so a lane makes 11 library calls instead of
-// the 25 of the per-environment chain.  Every call takes the arguments the
-// reference's code gives it, and the arm sums are formed in its order from
-// the broadcasts, so each feature is the value that code forms.  Lane a
-// returns features 6a .. 6a + 5 in t, mapped as the reference maps them
-// (NaN -> 0, +-inf -> +-1).
-__device__ void tactical_quad(const float *o, const float *m, int a, float (&t)[6]) {
+// over the quad and broadcast (the three atanh of the mission offsets; the
+// directions of yaw and of the target bearing; the two hypotenuses and the
+// two atan2f of the aim; eight tanhf in two calls), so a lane makes 8 calls
+// instead of the 25 of the per-environment chain.  Every call takes the
+// arguments the reference's code gives it, and the arm sums are formed in
+// its order from the broadcasts.  Lane a returns features 6a .. 6a + 5 in t,
+// mapped as the reference maps them (NaN -> 0, +-inf -> +-1).
+template <bool TAME>
+__device__ __forceinline__ void tactical_quad(const ChainInputs &in, int a, float (&t)[6]) {
     const float pi = kPi;
-    const float spool_a = ob_clamp(o[16 + a], 0.0f, 1.0f);
+    const float *o = in.head, *m = in.m;
+    const float o44 = in.tail[2], o45 = in.tail[3], o46 = in.tail[4], o47 = in.tail[5];
+    const float spool_a = ob_clamp<TAME>(in.arm[0], 0.0f, 1.0f);
     const float thrust_a = 0.036f + 0.964f * spool_a;
-    const float ci_a = cosf(o[28 + a]);
+    const float ci_a = onboard_math::cos_float<TAME>(in.arm[3]);
     const Quad4 spool = quad_all(spool_a);
-    const Quad4 fz = quad_all(thrust_a * o[24 + a] * ci_a);
-    const Quad4 tz = quad_all(thrust_a * o[20 + a] * ci_a);
+    const Quad4 fz = quad_all(thrust_a * in.arm[2] * ci_a);
+    const Quad4 tz = quad_all(thrust_a * in.arm[1] * ci_a);
     float tau_z = 0.0f, spool_mean = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -680,22 +747,41 @@ __device__ void tactical_quad(const float *o, const float *m, int a, float (&t)[
     const float qw = o[6], qx = o[7], qy = o[8], qz = o[9];
     const float bz_x = 2.0f * (qx * qz + qw * qy);
     const float bz_y = 2.0f * (qy * qz - qw * qx);
-    const float ct = ob_clamp(1.0f - 2.0f * (qx * qx + qy * qy), -1.0f, 1.0f);
+    const float ct = ob_clamp<TAME>(1.0f - 2.0f * (qx * qx + qy * qy), -1.0f, 1.0f);
     const float bx_x = 1.0f - 2.0f * (qy * qy + qz * qz);
     const float bx_y = 2.0f * (qx * qy + qw * qz);
     // rx, ry, rz on lanes 0, 1, 2 (lane 3 repeats rz).
-    const float r_a = atanhf(ob_clamp(m[7 + (a < 2 ? a : 2)], -0.995f, 0.995f)) * 20.0f;
+    const float r_a = onboard_math::atanh_float(ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]),
+                                                               -0.995f, 0.995f)) * 20.0f;
     const float rx = quad_lane<0>(r_a), ry = quad_lane<1>(r_a), rz = quad_lane<2>(r_a);
-    // yaw on lane 0, the target bearing atan2f(ry, rx) on the others.
-    const float at_a = atan2f(a == 0 ? bx_y : ry, a == 0 ? bx_x : rx);
-    const float yaw = quad_lane<0>(at_a), bearing = quad_lane<1>(at_a);
-    const SinCos yaw_sc = sin_cos(yaw);
-    const float cy = yaw_sc.c, sy = yaw_sc.s;
+    // Sine and cosine of yaw = atan2(bx_y, bx_x) on lane 0 and of the target
+    // bearing atan2(ry, rx) on the others, from their components; the angles
+    // themselves are used nowhere else.
+    const float ty_a = a == 0 ? bx_y : ry, tx_a = a == 0 ? bx_x : rx;
+    onboard_math::Direction at_a = onboard_math::direction(ty_a, tx_a);
+    if constexpr (!TAME) {
+        // Where a value that they multiply or come from is not finite, they
+        // are those of the rounded angle, as the reference forms them: an
+        // infinity times the sine of a float near pi is an infinity, times
+        // an exact zero it would be NaN.  (The sum of magnitudes may
+        // overflow; such a row takes that form too.)
+        const float reach = (fabsf(ty_a) + fabsf(tx_a)) + (fabsf(o[3]) + fabsf(o[4])) +
+                            (fabsf(bz_x) + fabsf(bz_y));
+        const bool odd = !(reach < __builtin_huge_valf());
+        if (__builtin_amdgcn_ballot_w64(odd)) {
+            float s, c;
+            sincosf(atan2f(ty_a, tx_a), &s, &c);
+            at_a.s = odd ? s : at_a.s;
+            at_a.c = odd ? c : at_a.c;
+        }
+    }
+    const float cy = quad_lane<0>(at_a.c), sy = quad_lane<0>(at_a.s);
+    const float cb = quad_lane<1>(at_a.c), sb = quad_lane<1>(at_a.s);
     v[8] = cy * bz_y - sy * bz_x;
     v[9] = -sy * bz_y - cy * bz_x;
     v[10] = ct;
     v[11] = ct < 0.20f ? 1.0f : 0.0f;
-    const float dist = fmaxf(ob_norm3(rx, ry, rz), 1.0f);
+    const float dist = fmaxf(ob_norm3<TAME>(rx, ry, rz), 1.0f);
     const float flight = div_const(dist, 20.0f);
     const float wx = rx - o[3] * 0.5f * flight;
     const float wy = ry - o[4] * 0.5f * flight;
@@ -707,14 +793,14 @@ __device__ void tactical_quad(const float *o, const float *m, int a, float (&t)[
     const float bx = wx + 2.0f * (uy * cz - uz * cyq);
     const float by = wy + 2.0f * (uz * cx - ux * cz);
     const float bz = wz + 2.0f * (ux * cyq - uy * cx);
-    // hypotf(rx, ry) on lane 0, hypotf(bx, by) on the others; then the aim's
-    // azimuth on lane 0 and elevation on the others.
-    const float hy_a = hypotf(a == 0 ? rx : bx, a == 0 ? ry : by);
+    // The hypotenuse of (rx, ry) on lane 0, of (bx, by) on the others; then
+    // the aim's azimuth on lane 0 and elevation on the others.
+    const float hy_a = ob_hypot<TAME>(a == 0 ? rx : bx, a == 0 ? ry : by);
     const float h_rxy = quad_lane<0>(hy_a), h_bxy = quad_lane<1>(hy_a);
     const float aim_a = atan2f(a == 0 ? by : bz, a == 0 ? bx : fmaxf(h_bxy, 0.2f));
-    const float az = ob_clamp(quad_lane<0>(aim_a), pi / 12.0f, pi * 5.0f / 12.0f);
-    const float el = ob_clamp(quad_lane<1>(aim_a), -pi / 6.0f, pi / 6.0f);
-    const float err = hypotf(az - o[44], el - o[45]);
+    const float az = ob_clamp<TAME>(quad_lane<0>(aim_a), pi / 12.0f, pi * 5.0f / 12.0f);
+    const float el = ob_clamp<TAME>(quad_lane<1>(aim_a), -pi / 6.0f, pi / 6.0f);
+    const float err = ob_hypot<TAME>(az - o44, el - o45);
     const float th1 = tanhf(quad_pick(a, (cy * rx + sy * ry) * 0.08f, (-sy * rx + cy * ry) * 0.08f,
                                       rz * 0.12f, h_rxy * 0.05f));
     const float th2 = tanhf(quad_pick(a, (cy * o[3] + sy * o[4]) * 0.15f,
@@ -729,33 +815,81 @@ __device__ void tactical_quad(const float *o, const float *m, int a, float (&t)[
     v[18] = expf(-fmaxf(o[2] - 0.62f, 0.0f));
     v[19] = div_const(az - pi * 0.25f, pi / 6.0f);
     v[20] = div_const(el, pi / 6.0f);
-    v[22] = (o[46] <= 0.02f && o[47] > 0.01f && err < 0.26f && dist < 34.0f) ? 1.0f : -1.0f;
-    v[23] = sinf(bearing - pi * 0.25f - yaw);
+    const bool ready = (int)(o46 <= 0.02f) & (int)(o47 > 0.01f) & (int)(err < 0.26f) &
+                       (int)(dist < 34.0f);
+    v[22] = ready ? 1.0f : -1.0f;
+    // sin(bearing - pi/4 - yaw) by the addition theorem.
+    v[23] = ((sb * cy - cb * sy) - (cb * cy + sb * sy)) * 0x1.6a09e6p-1f;  // 1 / sqrt 2
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
         const float x = quad_pick(a, v[k], v[6 + k], v[12 + k], v[18 + k]);
-        t[k] = __builtin_isnan(x) ? 0.0f : (__builtin_isinf(x) ? copysignf(1.0f, x) : x);
+        t[k] = TAME ? x : finite_as(x, 1.0f);
     }
 }
 
-// One lane's share of the prior features: its arm's throttle, outer and
-// inner commands, and (identical in the four lanes) cannon azimuth,
-// elevation and fire.
-struct ArmOutputs {
-    float throttle, outer, inner, az, el, fire;
+// The mission's flags (onboard_features.cuh:107-109, 126-136, 433-437).
+struct MissionFlags {
+    bool landing, cargo, inversion, turbine_out, lateral, slalom, dodge, arena;
+    bool bwb_arena, bwb_endurance, bwb;
 };
 
-// onboard_features.cuh:88-513 with the LiDAR passes replaced by `scan`, on
-// the four lanes of a quad: lane a evaluates arm a's terms (the two per-arm
-// loops, :114-125 and :376-391) and the four lanes repeat the shared chain,
-// except that independent calls of one function are spread over the quad
-// (four atan2, four atanh, four sine/cosine pairs, four angle wraps) and
-// their results broadcast.  The arm sums and the running maximum are formed
-// in the reference's order from quad broadcasts, so every value is the one
-// the per-environment code forms.  The statements are reordered only where
-// a value is needed earlier for such a group.
-__device__ ArmOutputs prior_features(const float *input_obs, const float *input_mission,
-                                     const ScanResult &scan, int a) {
+__device__ __forceinline__ MissionFlags mission_flags(const float (&m)[10]) {
+    MissionFlags f;
+    f.landing = m[1] > 0.75f;
+    f.cargo = m[2] > 0.75f;
+    f.inversion = (int)(m[3] > 0.75f) & (int)(m[0] < -0.25f);
+    f.turbine_out = (int)(m[3] > 0.75f) & (int)(m[2] < -0.25f);
+    f.lateral = (int)(m[4] > 0.75f) & (int)(m[5] > 0.25f);
+    f.slalom = (int)(m[4] > 0.75f) & (int)!f.lateral;
+    f.dodge = m[5] > 0.75f;
+    f.arena = m[6] > 0.75f;
+    f.bwb_arena = (int)f.arena & (int)(m[4] < -0.25f);
+    const bool cruise = (int)(m[4] > 0.75f) & (int)(m[2] > 0.25f);
+    f.bwb_endurance = (int)cruise & (int)(m[0] > 0.25f);
+    f.bwb = (int)f.bwb_arena | (int)cruise | ((int)f.arena & (int)(m[5] > 0.60f));
+    return f;
+}
+
+// The goal's position (onboard_features.cuh:157-172, before the arena's
+// stand-off) from the mission offsets.
+struct Goal {
+    float x, y, z;
+};
+
+__device__ __forceinline__ Goal goal_of(const MissionFlags &f, float px, float py, float pz,
+                                        float relx, float rely, float relz) {
+    const bool chase = (int)f.arena | (int)f.lateral;
+    Goal g;
+    g.x = chase ? px + relx : 0.0f;
+    g.x = f.cargo ? 15.0f : g.x;
+    g.x = f.slalom ? 36.0f : g.x;
+    g.y = chase ? py + rely : 0.0f;
+    g.z = f.landing ? 0.60f : 8.0f;
+    g.z = f.inversion ? 14.0f : g.z;
+    g.z = (int)f.cargo | (int)f.arena ? pz + relz : g.z;
+    return g;
+}
+
+// One lane's share of the flight controls: its arm's throttle, outer and
+// inner commands.
+struct ArmOutputs {
+    float throttle, outer, inner;
+};
+
+// The flight controller: onboard_features.cuh:88-432 without the cannon, with
+// the LiDAR passes replaced by `scan`, on the four lanes of a quad: lane a
+// evaluates arm a's terms (the two per-arm loops, :114-125 and :376-391) and
+// the four lanes repeat the shared chain, except that independent calls of
+// one function are spread over the quad (three atan2, three atanh, two
+// directions) and their results broadcast.  The arm sums and the running
+// maximum are formed in the reference's order from quad broadcasts, so every
+// value is the one the per-environment code forms.  The cannon and the BWB
+// law share nothing with this chain but its inputs: gunnery_quad forms them
+// on the waves of the tactical features, which are done far earlier.
+template <bool TAME>
+__device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, const MissionFlags &f,
+                                                  const ScanResult &scan, int a) {
+    using onboard_math::quotient;
     const float pi = kPi;
     const float max_installed = 294.2f * 0.85f;
     const float idle_frac = 0.08f;
@@ -764,33 +898,326 @@ __device__ ArmOutputs prior_features(const float *input_obs, const float *input_
     const float outer_limit = 2.0f;
     const float inner_limit = pi / 4.0f;
     const float cannon_az_ctr = pi / 4.0f;
+    const float *o = in.head, *m = in.m;
+    const float px = o[0], py = o[1], pz = o[2], vx = o[3], vy = o[4], vz = o[5];
+    const Attitude att = attitude_of(o[6], o[7], o[8], o[9]);
+    const float qw = att.qw, qx = att.qx, qy = att.qy, qz = att.qz;
+    const float ux = -qx, uy = -qy, uz = -qz;
+    const float r00 = att.r[0], r10 = att.r[3], r22 = att.r[8];
+    const float ox = o[10], oy = o[11], oz = o[12];
+    const float omega_norm = ob_norm3<TAME>(ox, oy, oz);
+
+    // Arm a of the four (this lane's); the quad exchanges the arm forces.
+    const float spool = ob_clamp<TAME>(in.arm[0], 0.0f, 1.0f);
+    const float thrust = max_installed * (idle_frac + (1.0f - idle_frac) * spool);
+    const float outer = ob_atan2<TAME>(in.arm[1], in.arm[2]);
+    const onboard_math::Direction o_sc = onboard_math::direction(in.arm[1], in.arm[2]);
+    const float c_inner = onboard_math::cos_float<TAME>(in.arm[3]);
+    const Quad4 fz = quad_all(thrust * o_sc.c * c_inner), ft = quad_all(thrust * o_sc.s * c_inner);
+    float total_fz = 0.0f, jammed_yaw_ft = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        total_fz += fz.v[i];
+        jammed_yaw_ft += ft.v[i];
+    }
+    const float fuel = ob_clamp<TAME>(in.tail[0], 0.0f, 1.0f) * 9.0f;
+    const float ammo_mass = ob_clamp<TAME>(in.tail[5], 0.0f, 4.0f) * 6.0f;
+    const bool payload = in.tail[1] > 0.5f;
+    const float mass = (f.arena ? 40.0f : 43.0f) + fuel + ammo_mass + (payload ? 30.0f : 0.0f);
+    const float weight = mass * gravity;
+    const float body_z_x = 2.0f * (qx * qz + qw * qy);
+    const float body_z_y = 2.0f * (qy * qz - qw * qx);
+    const float ct = ob_clamp<TAME>(r22, -1.0f, 1.0f);
+    const float tau_x_actual = fz.v[1] - fz.v[3];
+    const float tau_y_actual = fz.v[2] - fz.v[0];
+    const float az_actual = quotient<TAME>(total_fz * ct - weight, mass);
+    const bool heavy_cargo = (int)f.cargo & (int)payload;
+    const bool landing_like = (int)f.landing | (int)heavy_cargo;
+
+    // The mission offsets, one per lane; then yaw, the opponent bearing and
+    // the goal bearing.
+    const Quad4 offsets = quad_all(onboard_math::atanh_float(
+        ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]), -0.9995f, 0.9995f)));
+    const float relx = offsets.v[0] * 20.0f;
+    const float rely = offsets.v[1] * 20.0f;
+    const float relz = offsets.v[2] * 20.0f;
+    const Goal goal = goal_of(f, px, py, pz, relx, rely, relz);
+    const float tx = goal.x, ty = goal.y, tz = goal.z;
+    const float dx_opp = tx - px, dy_opp = ty - py;
+    const Quad4 angles = quad_all(ob_atan2<TAME>(quad_pick(a, r10, m[1], dy_opp, dy_opp),
+                                                 quad_pick(a, r00, m[2], dx_opp, dx_opp)));
+    const float yaw = angles.v[0], opp_bearing = angles.v[1], raw_bearing = angles.v[2];
+
+    float ex = tx, ey = ty, ez = tz;
+    const float dxy = ob_hypot<TAME>(dx_opp, dy_opp);
+    const bool valid_d = dxy > 1.0e-3f;
+    const onboard_math::Divisor over_d(valid_d ? dxy : 1.0f);
+    const bool intercept = (int)f.arena & (int)(m[0] > 0.75f) & (int)(m[5] < -0.25f);
+    const float desired_range = intercept ? 8.5f : 12.5f;
+    const float stand_x = tx - over_d(dx_opp) * desired_range;
+    const float stand_y = ty - over_d(dy_opp) * desired_range;
+    float ax = valid_d ? stand_x : tx;
+    float ay = valid_d ? stand_y : ty;
+    const float scale =
+        fminf(quotient<TAME>(16.0f, fmaxf(ob_hypot<TAME>(ax, ay), 1.0e-3f)), 1.0f);
+    ax *= scale;
+    ay *= scale;
+    const float pull =
+        ob_clamp<TAME>(div_const(ob_hypot<TAME>(px, py) - 21.0f, 10.0f), 0.0f, 1.0f);
+    ax *= 1.0f - pull;
+    ay *= 1.0f - pull;
+    const bool low_or_sinking = (int)(pz < 8.0f) | (int)(vz < -1.0f);
+    const float tz_held = ob_clamp<TAME>(tz, 8.5f, 12.2f);
+    const float az_t = low_or_sinking ? 12.2f : tz_held;
+    ex = f.arena ? ax : ex;
+    ey = f.arena ? ay : ey;
+    ez = f.arena ? az_t : ez;
+    const float errx = ex - px, erry = ey - py;
+    const float horiz_dist = ob_hypot<TAME>(errx, erry);
+
+    // Sine and cosine of yaw and of the closest return's bearing from their
+    // components (a rotation's rows; a range inside the window), and the sine
+    // of the slalom hill phase.
+    const onboard_math::Direction sc = onboard_math::direction(a == 0 ? r10 : scan.min_r_dy,
+                                                               a == 0 ? r00 : scan.min_r_dx);
+    const float cyaw = quad_lane<0>(sc.c), syaw = quad_lane<0>(sc.s);
+    const float hill = ob_clamp<TAME>(div_const(px - 6.0f, 30.0f), 0.0f, 1.0f);
+    const float hill_sin = onboard_math::sin_half_turn(hill);
+
+    const bool avoid = (int)f.dodge & (int)(scan.min_r < 7.5f);
+    const float away_x = -quad_lane<1>(sc.s) * 2.2f, away_y = quad_lane<1>(sc.c) * 2.2f;
+    const float avoid_x = avoid ? away_x : 0.0f, avoid_y = avoid ? away_y : 0.0f;
+    const float min_dx_c = scan.min_dx_c;
+    const int cluster_count = scan.cluster_count;
+    // Its sign alone is used, and the divisor is positive.
+    const float cluster_y = scan.cluster_y_sum;
+    const bool has_slalom_obs = (int)f.slalom & (int)(horiz_dist > 2.5f) & (int)(min_dx_c < 10.2f) &
+                                (int)(cluster_count > 0);
+    const float nearest_dx = has_slalom_obs ? min_dx_c : 30.0f;
+    const float side_y = cluster_y >= 0.0f ? -1.85f : 1.85f;
+    ey = has_slalom_obs ? side_y : ey;
+    const float lane_err = fabsf(py - ey);
+    float speed_limit = lane_err > 0.55f ? 2.75f : 4.10f;
+    speed_limit = lane_err > 1.05f ? 1.55f : speed_limit;
+    const bool open_road = (int)(min_dx_c >= 6.6f) & (int)(px > 4.0f);
+    speed_limit = open_road ? 3.10f : speed_limit;
+    const float slalom_speed = has_slalom_obs ? speed_limit : 3.8f;
+    const bool over_hill = (int)f.slalom & (int)(horiz_dist > 3.5f);
+    const float hill_z = 2.5f * hill_sin + 8.0f;
+    ez = over_hill ? hill_z : ez;
+    const float upx = ex - px, upy = ey - py, upz = ez - pz;
+    const float up_horiz = ob_hypot<TAME>(upx, upy);
+    const bool active_slalom =
+        (int)f.slalom & (int)(nearest_dx < 10.2f) & (int)(horiz_dist > 3.0f);
+
+    const float pad_z = fmaxf(ez, 0.60f), above_pad = pz - pad_z;
+    const float horiz_speed = ob_hypot<TAME>(vx, vy);
+    const float transit_cap = heavy_cargo ? 2.65f : 3.4f;
+    const float near_cap = heavy_cargo ? 1.25f : 1.6f;
+    const float low_cap = above_pad < 1.2f ? 0.55f : near_cap;
+    const float max_vxy_land = up_horiz > 1.8f ? transit_cap : low_cap;
+    const float kp_land = heavy_cargo ? 0.75f : 1.05f;
+    const float des_vx_land = ob_clamp<TAME>(kp_land * upx, -max_vxy_land, max_vxy_land);
+    const float des_vy_land = ob_clamp<TAME>(kp_land * upy, -max_vxy_land, max_vxy_land);
+    const float vz_land_touch = pz > 0.635f ? -0.16f : 0.0f;
+    const float vz_land_cargo = ob_clamp<TAME>(1.6f * (0.64f - pz), -0.30f, 0.18f);
+    const float vz_land_low = f.cargo ? vz_land_cargo : vz_land_touch;
+    const float max_desc = f.cargo ? -0.82f : -1.4f;
+    const float vz_land_mid = ob_clamp<TAME>(-0.70f * above_pad, max_desc, -0.25f);
+    const float vz_land_align = ob_clamp<TAME>(1.2f * (pad_z + 0.90f - pz), -0.30f, 0.60f);
+    const float heavy_transit = fmaxf(1.2f + 0.28f * up_horiz, 2.0f);
+    const float transit_z = heavy_cargo ? heavy_transit : 2.0f;
+    const float max_desc_trans = heavy_cargo ? -1.05f : -1.6f;
+    const float vz_land_trans = ob_clamp<TAME>(1.3f * (transit_z - pz), max_desc_trans, 1.4f);
+    float des_vz_land = above_pad > 1.05f ? vz_land_mid : vz_land_low;
+    const bool align = ((int)(up_horiz > 0.85f) | (int)(horiz_speed > 0.65f)) &
+                       (int)(above_pad < 0.95f);
+    des_vz_land = align ? vz_land_align : des_vz_land;
+    des_vz_land = up_horiz > 1.8f ? vz_land_trans : des_vz_land;
+    const float max_axy_land = heavy_cargo ? 2.2f : 2.6f;
+    const float des_ax_land = ob_clamp<TAME>(2.4f * (des_vx_land - vx), -max_axy_land, max_axy_land);
+    const float des_ay_land = ob_clamp<TAME>(2.4f * (des_vy_land - vy), -max_axy_land, max_axy_land);
+    const float kp_az_land = heavy_cargo ? 5.0f : 4.5f;
+    const float kd_az_land = heavy_cargo ? 1.0f : 0.80f;
+    const float min_az_land = heavy_cargo ? -1.8f : -2.8f;
+    const float des_az_land = ob_clamp<TAME>(
+        kp_az_land * (des_vz_land - vz) - kd_az_land * az_actual, min_az_land, 5.5f);
+
+    const bool dash = (int)(up_horiz > 9.0f) & (int)(fabsf(upz) < 2.5f) & (int)(ct > 0.90f);
+    const float inv_max_v = dash ? 6.2f : 4.2f;
+    const float lat_vx = fabsf(upy) > 1.35f ? 1.45f : 3.8f;
+    float max_vx = f.arena ? 3.2f : 3.0f;
+    max_vx = f.inversion ? inv_max_v : max_vx;
+    float max_vy = f.lateral ? 3.4f : max_vx;
+    max_vx = f.lateral ? lat_vx : max_vx;
+    max_vx = f.slalom ? 3.5f : max_vx;
+    max_vx = active_slalom ? slalom_speed : max_vx;
+    max_vy = active_slalom ? 3.2f : max_vy;
+    const bool climb_fast = (int)(vz < -2.0f) | (int)f.inversion;
+    const float max_vz = climb_fast ? 6.5f : 2.6f;
+    const float kp_side = f.lateral ? 0.95f : 0.90f;
+    const float kp_xy = f.inversion ? 0.85f : kp_side;
+    const float kp_vx = active_slalom ? 1.25f : kp_xy;
+    const float kp_vy_calm = f.lateral ? 1.05f : kp_xy;
+    const float kp_vy = active_slalom ? 1.45f : kp_vy_calm;
+    const float des_vx = ob_clamp<TAME>(kp_vx * upx + avoid_x, -max_vx, max_vx);
+    const float des_vy = ob_clamp<TAME>(kp_vy * upy + avoid_y, -max_vy, max_vy);
+    float des_vz = ob_clamp<TAME>(1.25f * upz, -2.6f, max_vz);
+    const bool recover = ((int)f.inversion | (int)f.arena) & (int)(vz < -1.0f);
+    const float des_vz_up = fmaxf(des_vz, 0.8f);
+    des_vz = recover ? des_vz_up : des_vz;
+    const float kp_ax = active_slalom ? 3.0f : 2.4f;
+    const float kp_ay = active_slalom ? 3.0f : 2.6f;
+    const float des_ax_std = ob_clamp<TAME>(kp_ax * (des_vx - vx), -3.8f, 3.8f);
+    const float des_ay_std = ob_clamp<TAME>(kp_ay * (des_vy - vy), -3.8f, 3.8f);
+    const bool pull_up = (int)(vz < -1.8f) | (int)f.inversion;
+    const float max_az = pull_up ? 14.0f : 6.5f;
+    const float des_az_std =
+        ob_clamp<TAME>(3.8f * (des_vz - vz) - 0.80f * az_actual, -4.0f, max_az);
+    const float des_ax = landing_like ? des_ax_land : des_ax_std;
+    const float des_ay = landing_like ? des_ay_land : des_ay_std;
+    const float des_az = landing_like ? des_az_land : des_az_std;
+
+    const float tilt = acosf(ct);
+    const bool need_headroom = (int)f.inversion | (int)f.arena | (int)(ct < 0.88f);
+    const bool urgent_climb = (int)f.arena & ((int)(pz < 8.5f) | (int)(vz < -1.2f)) &
+                              (int)(ct > 0.58f);
+    const float room = ob_clamp<TAME>(3.95f - 0.90f * omega_norm - 1.30f * tilt, 2.55f, 3.95f);
+    const float calm_coll = need_headroom ? room : 3.95f;
+    const float max_coll = urgent_climb ? 3.95f : calm_coll;
+    const float fz_des = ob_clamp<TAME>(quotient<TAME>(weight + mass * des_az, fmaxf(ct, 0.45f)),
+                                        0.10f * weight, max_coll * max_installed);
+    const float tilt_scale_h =
+        ob_clamp<TAME>(1.0f - 1.5f * fmaxf(tilt - 0.15f, 0.0f), 0.0f, 1.0f);
+    const float calm_scale = need_headroom ? tilt_scale_h : 1.0f;
+    const float horiz_scale = urgent_climb ? 0.0f : calm_scale;
+    const float tilt_comp = f.turbine_out ? 0.65f : 0.0f;
+    const float damp_v = active_slalom ? 0.8f : 0.4f;
+    const float fx_world =
+        (mass * des_ax + damp_v * vx - tilt_comp * total_fz * body_z_x) * horiz_scale;
+    const float fy_world =
+        (mass * des_ay + damp_v * vy - tilt_comp * total_fz * body_z_y) * horiz_scale;
+    const float std_fh = heavy_cargo ? 52.0f : 80.0f;
+    const float lat_fh = f.lateral ? 125.0f : std_fh;
+    const float max_fh = active_slalom ? 105.0f : lat_fh;
+    const float fx_body = ob_clamp<TAME>(cyaw * fx_world + syaw * fy_world, -max_fh, max_fh);
+    const float fy_body = ob_clamp<TAME>(-syaw * fx_world + cyaw * fy_world, -max_fh, max_fh);
+
+    const float cw_x = body_z_y, cw_y = -body_z_x;
+    const float tt_x = 2.0f * (-uz * cw_y), tt_y = 2.0f * (uz * cw_x);
+    const float tt_z = 2.0f * (ux * cw_y - uy * cw_x);
+    const float te_x = cw_x + qw * tt_x + (uy * tt_z - uz * tt_y);
+    const float te_y = cw_y + qw * tt_y + (uz * tt_x - ux * tt_z);
+    const float te_z = qw * tt_z + (ux * tt_y - uy * tt_x);
+    const float te_norm = ob_norm3<TAME>(te_x, te_y, te_z);
+    const float per_te = quotient<TAME>(tilt, fmaxf(te_norm, 1.0e-5f));
+    const float tilt_scale = te_norm > 1.0e-5f ? per_te : 0.0f;
+    const float e_rx = te_x * tilt_scale, e_ry = te_y * tilt_scale;
+
+    const bool inv_hold_yaw = ((int)f.inversion | (int)f.arena) &
+                              ((int)(pz < 6.0f) | (int)(vz < -0.5f) | (int)(ct < 0.88f));
+    const bool opp_bearing_valid = (int)f.arena & (int)(fabsf(m[1]) + fabsf(m[2]) > 0.1f);
+    const float target_bearing = opp_bearing_valid ? opp_bearing : raw_bearing;
+    const bool face = (int)f.arena & (int)(horiz_dist > 1.0f) & (int)!inv_hold_yaw;
+    const float held_yaw = inv_hold_yaw ? yaw : 0.0f;
+    const float facing_yaw = target_bearing - cannon_az_ctr;
+    const float desired_yaw = face ? facing_yaw : held_yaw;
+    const float yaw_err = ob_wrap<TAME>(desired_yaw, yaw);
+
+    const float parasite_scale = f.turbine_out ? 0.35f : 1.0f;
+    const float tau_x_par = -0.1625f * fy_body * parasite_scale;
+    const float tau_y_par = 0.1625f * fx_body * parasite_scale;
+    const float tau_x_net = tau_x_actual + tau_x_par;
+    const float tau_y_net = tau_y_actual + tau_y_par;
+    const float max_txy = heavy_cargo ? 120.0f : 260.0f;
+    const float tau_x_cmd = ob_clamp<TAME>(
+        95.0f * e_rx - 64.0f * ox - 0.90f * tau_x_net - tau_x_par, -max_txy, max_txy);
+    const float tau_y_cmd = ob_clamp<TAME>(
+        95.0f * e_ry - 64.0f * oy - 0.90f * tau_y_net - tau_y_par, -max_txy, max_txy);
+    const float tau_z_cmd = ob_clamp<TAME>(22.0f * yaw_err - 18.0f * oz, -70.0f, 70.0f);
+    // {q - ty, q + tx, q + ty, q - tx}[a]; q - t and q + (-t) are the same
+    // IEEE operation.
+    const float half_tx = tau_x_cmd * 0.5f, half_ty = tau_y_cmd * 0.5f;
+    const float fz_cmd = 0.25f * fz_des + quad_pick(a, -half_ty, half_tx, half_ty, -half_tx);
+    const float yaw_ft = (tau_z_cmd - 0.40f * jammed_yaw_ft) * 0.25f;
+    const float fx_outer = ft.v[3] - ft.v[1];
+    const float fy_outer = ft.v[0] - ft.v[2];
+    const float fx_rem = fx_body - fx_outer, fy_rem = fy_body - fy_outer;
+    const float std_sin = heavy_cargo ? 0.22f : 0.32f;
+    const float road_sin = active_slalom ? 0.42f : std_sin;
+    const float max_sin_inner = f.lateral ? 0.44f : road_sin;
+    const float std_gain = heavy_cargo ? 4.5f : 2.4f;
+    const float spool_gain = f.turbine_out ? 10.5f : std_gain;
+    const bool land_idle = (int)f.landing & (int)(pz <= 0.638f) & (int)(up_horiz < 0.85f) &
+                           (int)(fabsf(vz) < 0.20f);
+    const float sin_alpha =
+        ob_clamp<TAME>(quotient<TAME>(yaw_ft, fmaxf(thrust, 30.0f)), -0.35f, 0.35f);
+    const float yaw_alpha = asinf(sin_alpha);
+    float outer_cmd =
+        ob_clamp<TAME>(6.5f * ob_wrap<TAME>(yaw_alpha, outer), -outer_limit, outer_limit);
+    const float urx = quad_pick(a, 1.0f, 0.0f, -1.0f, 0.0f);
+    const float ury = quad_pick(a, 0.0f, 1.0f, 0.0f, -1.0f);
+    const float fr_req = 0.5f * (fx_rem * urx + fy_rem * ury);
+    const float sin_in = ob_clamp<TAME>(quotient<TAME>(fr_req, fmaxf(thrust, 40.0f)),
+                                        -max_sin_inner, max_sin_inner);
+    float inner_cmd = ob_clamp<TAME>(asinf(sin_in), -inner_limit * 0.90f, inner_limit * 0.90f);
+    // cos(yaw_alpha) cos(inner_cmd), both arcsines (|sin_in| <= 0.44, so the
+    // limit on inner_cmd is never met): one square root of the product of
+    // the two squared cosines, which is at least 0.70.
+    const float nominal_cos =
+        fmaxf(__builtin_amdgcn_sqrtf(__builtin_fmaf(-sin_alpha, sin_alpha, 1.0f) *
+                                     __builtin_fmaf(-sin_in, sin_in, 1.0f)), 0.70f);
+    const float lift_thrust = quotient<TAME>(fmaxf(fz_cmd, 0.0f), nominal_cos);
+    const float idle_thrust = 0.15f * weight * 0.25f;
+    const float target_thrust = land_idle ? idle_thrust : lift_thrust;
+    const float u_des = ob_clamp<TAME>(
+        div_const(target_thrust - min_thrust, max_installed - min_thrust), 0.0f, 1.0f);
+    const float u_raw = u_des + spool_gain * (u_des - spool);
+    // The reference's running maximum over arms 0..3, from -inf.
+    const Quad4 u_all = quad_all(u_raw);
+    float max_raw = -__builtin_huge_valf();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) max_raw = fmaxf(max_raw, u_all.v[i]);
+    const float excess = ob_clamp<TAME>(max_raw - 1.0f, 0.0f, urgent_climb ? 0.10f : 0.45f);
+    float throttle = ob_clamp<TAME>(u_raw - (need_headroom ? excess : 0.0f), 0.0f, 1.0f);
+    const bool inv_mode = ct < 0.20f;
+    const float inv_rx = te_norm > 1.0e-5f ? e_rx : tilt;
+    const float tx_inv = 130.0f * inv_rx - 52.0f * ox;
+    const float ty_inv = 130.0f * e_ry - 52.0f * oy;
+    const float arm_mom = quad_pick(a, -ty_inv, tx_inv, ty_inv, -tx_inv);
+    const float inv_throttle = arm_mom > 12.0f ? 0.58f : 0.0f;
+    const float inv_outer = ob_clamp<TAME>(-outer * 6.0f, -outer_limit, outer_limit);
+    throttle = inv_mode ? inv_throttle : throttle;
+    outer_cmd = inv_mode ? inv_outer : outer_cmd;
+    inner_cmd = inv_mode ? 0.0f : inner_cmd;
+    ArmOutputs out;
+    out.throttle = ob_clamp<TAME>(throttle * 2.0f - 1.0f, -1.0f, 1.0f);
+    out.outer = ob_clamp<TAME>(outer_cmd * (1.0f / outer_limit), -1.0f, 1.0f);
+    out.inner = ob_clamp<TAME>(div_const(inner_cmd, inner_limit), -1.0f, 1.0f);
+    return out;
+}
+
+// The cannon (onboard_features.cuh:393-430) and, for BWB missions, the BWB
+// law, which replaces every prior value (:433-510): the cannon's azimuth,
+// elevation and fire (identical in the four lanes) and, for a BWB mission,
+// lane a's arm commands.
+struct GunOutputs {
+    float az, el, fire;
+    ArmOutputs arm;  // BWB missions only
+};
+
+template <bool TAME>
+__device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, const MissionFlags &f,
+                                                   int a) {
+    using onboard_math::quotient;
+    const float pi = kPi;
+    const float gravity = 9.80665f;
+    const float inner_limit = pi / 4.0f;
+    const float cannon_az_ctr = pi / 4.0f;
     const float cannon_az_half = pi / 6.0f;
     const float cannon_el_lim = pi / 6.0f;
-    float o[48], m[10];
-#pragma unroll
-    for (int i = 0; i < 48; ++i) o[i] = input_obs[i];
-#pragma unroll
-    for (int i = 0; i < 10; ++i) m[i] = input_mission[i];
-    // The staged inputs the chain reads are all taken from LDS here, at
-    // once: an empty asm on each value keeps the compiler from sinking its
-    // read to the first use, where every read cost the chain its own LDS
-    // round trip (51 waits on LDS in the kernel before, 29 after).
-    float arm_in[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) arm_in[k] = input_obs[16 + 4 * k + a];
-    {
-        constexpr int kUsed[] = {0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 40, 41, 44, 45, 46, 47};
-#pragma unroll
-        for (int i : kUsed) asm volatile("" : "+v"(o[i]));
-#pragma unroll
-        for (int i = 0; i < 10; ++i) asm volatile("" : "+v"(m[i]));
-#pragma unroll
-        for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(arm_in[k]));
-    }
-#pragma unroll
-    for (int i = 0; i < 48; ++i) o[i] = ob_obs(o[i]);
-#pragma unroll
-    for (int i = 0; i < 10; ++i) m[i] = ob_mission(m[i]);
+    const float *o = in.head, *m = in.m;
+    const float o44 = in.tail[2], o45 = in.tail[3], o46 = in.tail[4], o47 = in.tail[5];
     const float px = o[0], py = o[1], pz = o[2], vx = o[3], vy = o[4], vz = o[5];
     const Attitude att = attitude_of(o[6], o[7], o[8], o[9]);
     const float qw = att.qw, qx = att.qx, qy = att.qy, qz = att.qz;
@@ -798,97 +1225,16 @@ __device__ ArmOutputs prior_features(const float *input_obs, const float *input_
     const float r00 = att.r[0], r01 = att.r[1], r02 = att.r[2];
     const float r10 = att.r[3], r11 = att.r[4], r12 = att.r[5];
     const float r20 = att.r[6], r21 = att.r[7], r22 = att.r[8];
-    const float ox = o[10], oy = o[11], oz = o[12];
-    const float omega_norm = ob_norm3(ox, oy, oz);
+    const float ct = ob_clamp<TAME>(r22, -1.0f, 1.0f);
+    const bool inv_mode = ct < 0.20f;
 
-    // Arm a of the four (this lane's); the quad exchanges the arm forces.
-    const float spool = ob_clamp(ob_obs(arm_in[0]), 0.0f, 1.0f);
-    const float thrust = max_installed * (idle_frac + (1.0f - idle_frac) * spool);
-    const float outer = ob_atan2(ob_obs(arm_in[1]), ob_obs(arm_in[2]));
-    const SinCos o_sc = sin_cos(outer);
-    const float c_inner = cosf(ob_obs(arm_in[3]));
-    const float fz_a = thrust * o_sc.c * c_inner;
-    const float ft_a = thrust * o_sc.s * c_inner;
-    const Quad4 fz = quad_all(fz_a), ft = quad_all(ft_a);
-    float total_fz = 0.0f, jammed_yaw_ft = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        total_fz += fz.v[i];
-        jammed_yaw_ft += ft.v[i];
-    }
-    const bool landing = m[1] > 0.75f;
-    const bool cargo = m[2] > 0.75f;
-    const bool inversion = m[3] > 0.75f && m[0] < -0.25f;
-    const bool turbine_out = m[3] > 0.75f && m[2] < -0.25f;
-    const bool lateral = m[4] > 0.75f && m[5] > 0.25f;
-    const bool slalom = m[4] > 0.75f && !lateral;
-    const bool dodge = m[5] > 0.75f;
-    const bool arena = m[6] > 0.75f;
-    const bool bwb_arena = m[6] > 0.75f && m[4] < -0.25f;
-    const bool bwb_cruise = m[4] > 0.75f && m[2] > 0.25f;
-    const bool bwb_intercept = m[6] > 0.75f && m[5] > 0.60f;
-    const bool bwb_endurance = bwb_cruise && m[0] > 0.25f;
-    const bool bwb = bwb_arena || bwb_cruise || bwb_intercept;
-    const float fuel = ob_clamp(o[40], 0.0f, 1.0f) * 9.0f;
-    const float ammo_mass = ob_clamp(o[47], 0.0f, 4.0f) * 6.0f;
-    const bool payload = o[41] > 0.5f;
-    const float mass = (arena ? 40.0f : 43.0f) + fuel + ammo_mass + (payload ? 30.0f : 0.0f);
-    const float weight = mass * gravity;
-    const float body_z_x = 2.0f * (qx * qz + qw * qy);
-    const float body_z_y = 2.0f * (qy * qz - qw * qx);
-    const float ct = ob_clamp(r22, -1.0f, 1.0f);
-    const float tau_x_actual = fz.v[1] - fz.v[3];
-    const float tau_y_actual = fz.v[2] - fz.v[0];
-    const float az_actual = (total_fz * ct - weight) / mass;
-    const bool heavy_cargo = cargo && payload;
-    const bool landing_like = landing || heavy_cargo;
-
-    // Independent calls of one function, one per lane of the quad: yaw, the
-    // opponent bearing, the BWB roll and ground-track angles; the mission
-    // offsets (atanh at the standard clamp, and the first at the BWB clamp).
-    const Quad4 angles = quad_all(ob_atan2(quad_pick(a, r10, m[1], r21, vy),
-                                         quad_pick(a, r00, m[2], r22, vx)));
-    const float yaw = angles.v[0], opp_bearing = angles.v[1];
-    const float roll_right = angles.v[2], track_yaw = angles.v[3];
-    const Quad4 offsets = quad_all(atanhf(quad_pick(
-        a, ob_clamp(m[7], -0.9995f, 0.9995f), ob_clamp(m[8], -0.9995f, 0.9995f),
-        ob_clamp(m[9], -0.9995f, 0.9995f), ob_clamp(m[7], -0.9999f, 0.9999f))));
-
-    const float relx = offsets.v[0] * 20.0f;
-    const float rely = offsets.v[1] * 20.0f;
-    const float relz = offsets.v[2] * 20.0f;
-    float tx = (arena || lateral) ? px + relx : 0.0f;
-    if (cargo) tx = 15.0f;
-    if (slalom) tx = 36.0f;
-    const float ty = (arena || lateral) ? py + rely : 0.0f;
-    float tz = 8.0f;
-    if (landing) tz = 0.60f;
-    if (inversion) tz = 14.0f;
-    if (cargo || arena) tz = pz + relz;
-    float ex = tx, ey = ty, ez = tz;
-    const float dx_opp = tx - px, dy_opp = ty - py;
-    const float dxy = hypotf(dx_opp, dy_opp);
-    const bool valid_d = dxy > 1.0e-3f;
-    const float safe_d = valid_d ? dxy : 1.0f;
-    const bool intercept = arena && m[0] > 0.75f && m[5] < -0.25f;
-    const float desired_range = intercept ? 8.5f : 12.5f;
-    float ax = valid_d ? tx - (dx_opp / safe_d) * desired_range : tx;
-    float ay = valid_d ? ty - (dy_opp / safe_d) * desired_range : ty;
-    const float scale = fminf(16.0f / fmaxf(hypotf(ax, ay), 1.0e-3f), 1.0f);
-    ax *= scale;
-    ay *= scale;
-    const float pull = ob_clamp(div_const(hypotf(px, py) - 21.0f, 10.0f), 0.0f, 1.0f);
-    ax *= 1.0f - pull;
-    ay *= 1.0f - pull;
-    const float az_t = pz < 8.0f || vz < -1.0f ? 12.2f : ob_clamp(tz, 8.5f, 12.2f);
-    if (arena) { ex = ax; ey = ay; ez = az_t; }
-    const float errx = ex - px, erry = ey - py;
-    const float horiz_dist = hypotf(errx, erry);
-
-    // Cannon aim point in the body frame (formed here so that its two
-    // angles join the quad's next atan2 round).
-    const float to_x = tx - px, to_y = ty - py, to_z = tz - pz;
-    const float dist = fmaxf(ob_norm3(to_x, to_y, to_z), 1.0f);
+    const Quad4 offsets = quad_all(onboard_math::atanh_float(
+        ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]), -0.9995f, 0.9995f)));
+    const Goal goal = goal_of(f, px, py, pz, offsets.v[0] * 20.0f, offsets.v[1] * 20.0f,
+                              offsets.v[2] * 20.0f);
+    // The aim point in the body frame.
+    const float to_x = goal.x - px, to_y = goal.y - py, to_z = goal.z - pz;
+    const float dist = fmaxf(ob_norm3<TAME>(to_x, to_y, to_z), 1.0f);
     const float flight = div_const(dist, 20.0f);
     const float aim_x = to_x - vx * (0.65f * flight);
     const float aim_y = to_y - vy * (0.65f * flight);
@@ -899,309 +1245,120 @@ __device__ ArmOutputs prior_features(const float *input_obs, const float *input_
     const float aim_bx = aim_x + 2.0f * (uy * cz - uz * cyq);
     const float aim_by = aim_y + 2.0f * (uz * cx - ux * cz);
     const float aim_bz = aim_z + 2.0f * (ux * cyq - uy * cx);
-    const Quad4 bearings = quad_all(ob_atan2(
-        quad_pick(a, ty - py, scan.min_r_dy, aim_by, aim_bz),
-        quad_pick(a, tx - px, scan.min_r_dx, aim_bx, fmaxf(hypotf(aim_bx, aim_by), 0.2f))));
-    const float raw_bearing = bearings.v[0], min_az = bearings.v[1];
+    // The aim's azimuth and elevation, and for the BWB law roll and course
+    // (the ground track above 2.5 m/s, else yaw).
+    const float gs = ob_hypot<TAME>(vx, vy);
+    const float course_y = gs > 2.5f ? vy : r10, course_x = gs > 2.5f ? vx : r00;
+    const Quad4 angles = quad_all(ob_atan2<TAME>(
+        quad_pick(a, aim_by, aim_bz, r21, course_y),
+        quad_pick(a, aim_bx, fmaxf(ob_hypot<TAME>(aim_bx, aim_by), 0.2f), r22, course_x)));
     const float des_cannon_az =
-        ob_clamp(bearings.v[2], cannon_az_ctr - cannon_az_half, cannon_az_ctr + cannon_az_half);
-    const float des_cannon_el = ob_clamp(bearings.v[3], -cannon_el_lim, cannon_el_lim);
+        ob_clamp<TAME>(angles.v[0], cannon_az_ctr - cannon_az_half, cannon_az_ctr + cannon_az_half);
+    const float des_cannon_el = ob_clamp<TAME>(angles.v[1], -cannon_el_lim, cannon_el_lim);
+    const float roll_right = angles.v[2], course_yaw = angles.v[3];
 
-    // Sine and cosine of yaw, of the closest return's bearing, of the BWB
-    // roll, and of the slalom hill phase.
-    const float hill = ob_clamp(div_const(px - 6.0f, 30.0f), 0.0f, 1.0f);
-    const SinCos sc = sin_cos(quad_pick(a, yaw, min_az, roll_right, pi * hill));
-    const Quad4 sines = quad_all(sc.s), cosines = quad_all(sc.c);
-    const float cyaw = cosines.v[0], syaw = sines.v[0];
+    const float aim_err = ob_hypot<TAME>(ob_wrap<TAME>(des_cannon_az, o44), des_cannon_el - o45);
+    const bool loaded = (int)f.arena & (int)(o46 <= 0.02f) & (int)(o47 > 0.01f);
+    const bool fire =
+        (int)loaded & (int)!inv_mode & (int)(aim_err < 0.28f) & (int)(dist < 34.0f);
+    const bool cannon = (int)f.arena & (int)!inv_mode;
+    const float aimed_az =
+        ob_clamp<TAME>(div_const(des_cannon_az - cannon_az_ctr, cannon_az_half), -1.0f, 1.0f);
+    const float aimed_el = ob_clamp<TAME>(div_const(des_cannon_el, cannon_el_lim), -1.0f, 1.0f);
+    GunOutputs out;
+    out.az = cannon ? aimed_az : 0.0f;
+    out.az = inv_mode ? -1.0f : out.az;
+    out.el = cannon ? aimed_el : 0.0f;
+    out.fire = fire ? 0.8f : -0.8f;
+    out.arm = ArmOutputs{0.0f, 0.0f, 0.0f};
+    if (!f.bwb) return out;
 
-    float avoid_x = 0.0f, avoid_y = 0.0f, slalom_speed = 3.8f, nearest_dx = 30.0f;
-    if (dodge && scan.min_r < 7.5f) {
-        avoid_x = -sines.v[1] * 2.2f;
-        avoid_y = cosines.v[1] * 2.2f;
-    }
-    const float min_dx_c = scan.min_dx_c;
-    const int cluster_count = scan.cluster_count;
-    const float cluster_y = scan.cluster_y_sum / fmaxf((float)cluster_count, 1.0f);
-    const bool has_slalom_obs = slalom && horiz_dist > 2.5f && min_dx_c < 10.2f &&
-                                cluster_count > 0;
-    if (has_slalom_obs) {
-        nearest_dx = min_dx_c;
-        ey = cluster_y >= 0.0f ? -1.85f : 1.85f;
-    }
-    const float lane_err = fabsf(py - ey);
-    float speed_limit = lane_err > 0.55f ? 2.75f : 4.10f;
-    if (lane_err > 1.05f) speed_limit = 1.55f;
-    if (min_dx_c >= 6.6f && px > 4.0f) speed_limit = 3.10f;
-    if (has_slalom_obs) slalom_speed = speed_limit;
-    if (slalom && horiz_dist > 3.5f) ez = 2.5f * sines.v[3] + 8.0f;
-    const float upx = ex - px, upy = ey - py, upz = ez - pz;
-    const float up_horiz = hypotf(upx, upy);
-    const bool active_slalom = slalom && nearest_dx < 10.2f && horiz_dist > 3.0f;
+    const float vb_x = r00 * vx + r10 * vy + r20 * vz;
+    const float vb_y = r01 * vx + r11 * vy + r21 * vz;
+    const Quad4 b_offsets = quad_all(onboard_math::atanh_float(
+        ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]), -0.9999f, 0.9999f)));
+    const float brx = b_offsets.v[0] * 20.0f;
+    const float bry = b_offsets.v[1] * 20.0f;
+    const float brz = b_offsets.v[2] * 20.0f;
+    float btx = px + brx;
+    float bty = py + bry;
+    float btz = pz + brz;
+    const float rxy = ob_hypot<TAME>(px, py);
+    const float pull_b = ob_clamp<TAME>(div_const(rxy - 235.0f, 45.0f), 0.0f, 0.85f);
+    const bool fenced = (int)f.arena & (int)(rxy > 235.0f);
+    const float in_x = btx * (1.0f - pull_b), in_y = bty * (1.0f - pull_b);
+    btx = fenced ? in_x : btx;
+    bty = fenced ? in_y : bty;
+    const float in_z = ob_clamp<TAME>(btz, 28.0f, 135.0f);
+    btz = f.arena ? in_z : btz;
+    const float gx = btx - px, gy = bty - py;
+    const float gz = btz - pz;
+    const float gdist = fmaxf(ob_norm3<TAME>(gx, gy, gz), 1.0f);
+    const float climb_des = ob_clamp<TAME>(0.42f * gz, -5.0f, 5.0f);
+    const float oppx = brx - vx * 0.10f, oppy = bry - vy * 0.10f, oppz = brz - vz * 0.10f;
+    const float bdist = fmaxf(ob_norm3<TAME>(oppx, oppy, oppz), 1.0f);
+    const bool head_on = (int)f.bwb_arena & (int)(btx * px + bty * py < -800.0f) &
+                         (int)(bdist > 45.0f);
+    const float head_closing = 75.0f + 2.0f * fmaxf(vb_x, 0.0f);
+    const float closing = head_on ? head_closing : 75.0f;
+    const float bflight = quotient<TAME>(bdist, closing);
+    const float bax = oppx, bay = oppy;
+    const float sink = -vz * (0.85f * bflight);
+    const float baz = oppz + (head_on ? sink : 0.0f) + 0.50f * gravity * bflight * bflight;
+    const float bbx = r00 * bax + r10 * bay + r20 * baz;
+    const float bby = r01 * bax + r11 * bay + r21 * baz;
+    const float bbz = r02 * bax + r12 * bay + r22 * baz;
+    const Quad4 b_angles = quad_all(ob_atan2<TAME>(
+        quad_pick(a, gy, climb_des, bby, bbz),
+        quad_pick(a, gx, fmaxf(gs, 14.0f), fmaxf(bbx, 0.2f),
+                  fmaxf(ob_hypot<TAME>(bbx, bby), 0.2f))));
+    const float desired_yaw_b = b_angles.v[0], gamma_des = b_angles.v[1];
+    const float b_az = ob_clamp<TAME>(b_angles.v[2], -pi / 6.0f, pi / 6.0f);
+    const float b_el = ob_clamp<TAME>(b_angles.v[3], -cannon_el_lim, cannon_el_lim);
 
-    const float pad_z = fmaxf(ez, 0.60f), above_pad = pz - pad_z;
-    const float horiz_speed = hypotf(vx, vy);
-    const float transit_cap = heavy_cargo ? 2.65f : 3.4f;
-    const float low_cap = above_pad < 1.2f ? 0.55f : (heavy_cargo ? 1.25f : 1.6f);
-    const float max_vxy_land = up_horiz > 1.8f ? transit_cap : low_cap;
-    const float kp_land = heavy_cargo ? 0.75f : 1.05f;
-    const float des_vx_land = ob_clamp(kp_land * upx, -max_vxy_land, max_vxy_land);
-    const float des_vy_land = ob_clamp(kp_land * upy, -max_vxy_land, max_vxy_land);
-    const float vz_land_touch = pz > 0.635f ? -0.16f : 0.0f;
-    const float vz_land_cargo = ob_clamp(1.6f * (0.64f - pz), -0.30f, 0.18f);
-    const float vz_land_low = cargo ? vz_land_cargo : vz_land_touch;
-    const float max_desc = cargo ? -0.82f : -1.4f;
-    const float vz_land_mid = ob_clamp(-0.70f * above_pad, max_desc, -0.25f);
-    const float vz_land_align = ob_clamp(1.2f * (pad_z + 0.90f - pz), -0.30f, 0.60f);
-    const float transit_z = heavy_cargo ? fmaxf(1.2f + 0.28f * up_horiz, 2.0f) : 2.0f;
-    const float max_desc_trans = heavy_cargo ? -1.05f : -1.6f;
-    const float vz_land_trans = ob_clamp(1.3f * (transit_z - pz), max_desc_trans, 1.4f);
-    float des_vz_land = above_pad > 1.05f ? vz_land_mid : vz_land_low;
-    if ((up_horiz > 0.85f || horiz_speed > 0.65f) && above_pad < 0.95f)
-        des_vz_land = vz_land_align;
-    if (up_horiz > 1.8f) des_vz_land = vz_land_trans;
-    const float max_axy_land = heavy_cargo ? 2.2f : 2.6f;
-    const float des_ax_land = ob_clamp(2.4f * (des_vx_land - vx), -max_axy_land, max_axy_land);
-    const float des_ay_land = ob_clamp(2.4f * (des_vy_land - vy), -max_axy_land, max_axy_land);
-    const float kp_az_land = heavy_cargo ? 5.0f : 4.5f;
-    const float kd_az_land = heavy_cargo ? 1.0f : 0.80f;
-    const float min_az_land = heavy_cargo ? -1.8f : -2.8f;
-    const float des_az_land = ob_clamp(kp_az_land * (des_vz_land - vz) - kd_az_land * az_actual,
-                                       min_az_land, 5.5f);
-
-    const float inv_max_v = up_horiz > 9.0f && fabsf(upz) < 2.5f && ct > 0.90f ? 6.2f : 4.2f;
-    const float lat_vx = fabsf(upy) > 1.35f ? 1.45f : 3.8f;
-    float max_vx = arena ? 3.2f : 3.0f;
-    if (inversion) max_vx = inv_max_v;
-    float max_vy = max_vx;
-    if (lateral) { max_vx = lat_vx; max_vy = 3.4f; }
-    if (slalom) max_vx = 3.5f;
-    if (active_slalom) { max_vx = slalom_speed; max_vy = 3.2f; }
-    const float max_vz = vz < -2.0f || inversion ? 6.5f : 2.6f;
-    const float kp_xy = inversion ? 0.85f : (lateral ? 0.95f : 0.90f);
-    const float kp_vx = active_slalom ? 1.25f : kp_xy;
-    const float kp_vy = active_slalom ? 1.45f : (lateral ? 1.05f : kp_xy);
-    const float des_vx = ob_clamp(kp_vx * upx + avoid_x, -max_vx, max_vx);
-    const float des_vy = ob_clamp(kp_vy * upy + avoid_y, -max_vy, max_vy);
-    float des_vz = ob_clamp(1.25f * upz, -2.6f, max_vz);
-    if ((inversion || arena) && vz < -1.0f) des_vz = fmaxf(des_vz, 0.8f);
-    const float kp_ax = active_slalom ? 3.0f : 2.4f;
-    const float kp_ay = active_slalom ? 3.0f : 2.6f;
-    const float des_ax_std = ob_clamp(kp_ax * (des_vx - vx), -3.8f, 3.8f);
-    const float des_ay_std = ob_clamp(kp_ay * (des_vy - vy), -3.8f, 3.8f);
-    const float max_az = vz < -1.8f || inversion ? 14.0f : 6.5f;
-    const float des_az_std = ob_clamp(3.8f * (des_vz - vz) - 0.80f * az_actual, -4.0f, max_az);
-    const float des_ax = landing_like ? des_ax_land : des_ax_std;
-    const float des_ay = landing_like ? des_ay_land : des_ay_std;
-    const float des_az = landing_like ? des_az_land : des_az_std;
-
-    const float tilt = acosf(ct);
-    const bool need_headroom = inversion || arena || ct < 0.88f;
-    const bool urgent_climb = arena && (pz < 8.5f || vz < -1.2f) && ct > 0.58f;
-    const float max_coll =
-        urgent_climb ? 3.95f
-                     : (need_headroom
-                            ? ob_clamp(3.95f - 0.90f * omega_norm - 1.30f * tilt, 2.55f, 3.95f)
-                            : 3.95f);
-    const float fz_des = ob_clamp((weight + mass * des_az) / fmaxf(ct, 0.45f), 0.10f * weight,
-                                  max_coll * max_installed);
-    const float horiz_scale =
-        urgent_climb ? 0.0f
-                     : (need_headroom
-                            ? ob_clamp(1.0f - 1.5f * fmaxf(tilt - 0.15f, 0.0f), 0.0f, 1.0f)
-                            : 1.0f);
-    const float tilt_comp = turbine_out ? 0.65f : 0.0f;
-    const float damp_v = active_slalom ? 0.8f : 0.4f;
-    const float fx_world =
-        (mass * des_ax + damp_v * vx - tilt_comp * total_fz * body_z_x) * horiz_scale;
-    const float fy_world =
-        (mass * des_ay + damp_v * vy - tilt_comp * total_fz * body_z_y) * horiz_scale;
-    const float max_fh =
-        active_slalom ? 105.0f : (lateral ? 125.0f : (heavy_cargo ? 52.0f : 80.0f));
-    const float fx_body = ob_clamp(cyaw * fx_world + syaw * fy_world, -max_fh, max_fh);
-    const float fy_body = ob_clamp(-syaw * fx_world + cyaw * fy_world, -max_fh, max_fh);
-
-    const float cw_x = body_z_y, cw_y = -body_z_x;
-    const float tt_x = 2.0f * (-uz * cw_y), tt_y = 2.0f * (uz * cw_x);
-    const float tt_z = 2.0f * (ux * cw_y - uy * cw_x);
-    const float te_x = cw_x + qw * tt_x + (uy * tt_z - uz * tt_y);
-    const float te_y = cw_y + qw * tt_y + (uz * tt_x - ux * tt_z);
-    const float te_z = qw * tt_z + (ux * tt_y - uy * tt_x);
-    const float te_norm = ob_norm3(te_x, te_y, te_z);
-    const float tilt_scale = te_norm > 1.0e-5f ? tilt / fmaxf(te_norm, 1.0e-5f) : 0.0f;
-    const float e_rx = te_x * tilt_scale, e_ry = te_y * tilt_scale;
-
-    const bool inv_hold_yaw = (inversion || arena) && (pz < 6.0f || vz < -0.5f || ct < 0.88f);
-    const bool opp_bearing_valid = arena && fabsf(m[1]) + fabsf(m[2]) > 0.1f;
-    const float target_bearing = opp_bearing_valid ? opp_bearing : raw_bearing;
-    const float desired_yaw = arena && horiz_dist > 1.0f && !inv_hold_yaw
-                                  ? target_bearing - cannon_az_ctr
-                                  : (inv_hold_yaw ? yaw : 0.0f);
-
-    // BWB geometry (onboard_features.cuh:437-510), up to the angles its two
-    // wraps need; the control law follows after the shared part.
-    float vb_x = 0.0f, vb_y = 0.0f, brx = 0.0f, bry = 0.0f, btx = 0.0f, bty = 0.0f, gz = 0.0f;
-    float gdist = 0.0f, gamma_des = 0.0f, bdist = 0.0f, bbx = 0.0f;
-    float desired_yaw_b = 0.0f, course_yaw = 0.0f, b_az = 0.0f, b_el = 0.0f;
-    if (bwb) {
-        vb_x = r00 * vx + r10 * vy + r20 * vz;
-        vb_y = r01 * vx + r11 * vy + r21 * vz;
-        brx = offsets.v[3] * 20.0f;
-        const Quad4 b_offsets = quad_all(atanhf(quad_pick(a, ob_clamp(m[8], -0.9999f, 0.9999f),
-                                                          ob_clamp(m[9], -0.9999f, 0.9999f),
-                                                          0.0f, 0.0f)));
-        bry = b_offsets.v[0] * 20.0f;
-        const float brz = b_offsets.v[1] * 20.0f;
-        btx = px + brx;
-        bty = py + bry;
-        float btz = pz + brz;
-        const float rxy = hypotf(px, py);
-        const float pull_b = ob_clamp(div_const(rxy - 235.0f, 45.0f), 0.0f, 0.85f);
-        if (arena && rxy > 235.0f) { btx *= 1.0f - pull_b; bty *= 1.0f - pull_b; }
-        if (arena) btz = ob_clamp(btz, 28.0f, 135.0f);
-        const float gx = btx - px, gy = bty - py;
-        gz = btz - pz;
-        gdist = fmaxf(ob_norm3(gx, gy, gz), 1.0f);
-        const float gs = hypotf(vx, vy);
-        course_yaw = gs > 2.5f ? track_yaw : yaw;
-        const float climb_des = ob_clamp(0.42f * gz, -5.0f, 5.0f);
-        const float oppx = brx - vx * 0.10f, oppy = bry - vy * 0.10f, oppz = brz - vz * 0.10f;
-        bdist = fmaxf(ob_norm3(oppx, oppy, oppz), 1.0f);
-        const bool head_on = bwb_arena && btx * px + bty * py < -800.0f && bdist > 45.0f;
-        const float closing = head_on ? 75.0f + 2.0f * fmaxf(vb_x, 0.0f) : 75.0f;
-        const float bflight = bdist / closing;
-        const float bax = oppx, bay = oppy;
-        const float baz =
-            oppz + (head_on ? -vz * (0.85f * bflight) : 0.0f) + 0.50f * gravity * bflight * bflight;
-        bbx = r00 * bax + r10 * bay + r20 * baz;
-        const float bby = r01 * bax + r11 * bay + r21 * baz;
-        const float bbz = r02 * bax + r12 * bay + r22 * baz;
-        const Quad4 b_angles = quad_all(ob_atan2(
-            quad_pick(a, gy, climb_des, bby, bbz),
-            quad_pick(a, gx, fmaxf(gs, 14.0f), fmaxf(bbx, 0.2f), fmaxf(hypotf(bbx, bby), 0.2f))));
-        desired_yaw_b = b_angles.v[0];
-        gamma_des = b_angles.v[1];
-        b_az = ob_clamp(b_angles.v[2], -pi / 6.0f, pi / 6.0f);
-        b_el = ob_clamp(b_angles.v[3], -cannon_el_lim, cannon_el_lim);
-    }
-
-    // The four angle wraps, one per lane: yaw error, cannon azimuth error,
-    // BWB course error, BWB cannon azimuth error.
-    const Quad4 wraps = quad_all(ob_wrap(quad_pick(a, desired_yaw, des_cannon_az, desired_yaw_b,
-                                                   b_az),
-                                         quad_pick(a, yaw, o[44], course_yaw, o[44])));
-    const float yaw_err = wraps.v[0];
-
-    const float parasite_scale = turbine_out ? 0.35f : 1.0f;
-    const float tau_x_par = -0.1625f * fy_body * parasite_scale;
-    const float tau_y_par = 0.1625f * fx_body * parasite_scale;
-    const float tau_x_net = tau_x_actual + tau_x_par;
-    const float tau_y_net = tau_y_actual + tau_y_par;
-    const float max_txy = heavy_cargo ? 120.0f : 260.0f;
-    const float tau_x_cmd = ob_clamp(95.0f * e_rx - 64.0f * ox - 0.90f * tau_x_net - tau_x_par,
-                                     -max_txy, max_txy);
-    const float tau_y_cmd = ob_clamp(95.0f * e_ry - 64.0f * oy - 0.90f * tau_y_net - tau_y_par,
-                                     -max_txy, max_txy);
-    const float tau_z_cmd = ob_clamp(22.0f * yaw_err - 18.0f * oz, -70.0f, 70.0f);
-    // {q - ty, q + tx, q + ty, q - tx}[a]; q - t and q + (-t) are the same
-    // IEEE operation.
-    const float half_tx = tau_x_cmd * 0.5f, half_ty = tau_y_cmd * 0.5f;
-    const float fz_cmd = 0.25f * fz_des + quad_pick(a, -half_ty, half_tx, half_ty, -half_tx);
-    const float yaw_ft = (tau_z_cmd - 0.40f * jammed_yaw_ft) * 0.25f;
-    float outer_cmd, inner_cmd, throttle;
-    const float fx_outer = ft.v[3] - ft.v[1];
-    const float fy_outer = ft.v[0] - ft.v[2];
-    const float fx_rem = fx_body - fx_outer, fy_rem = fy_body - fy_outer;
-    const float max_sin_inner =
-        lateral ? 0.44f : (active_slalom ? 0.42f : (heavy_cargo ? 0.22f : 0.32f));
-    const float spool_gain = turbine_out ? 10.5f : (heavy_cargo ? 4.5f : 2.4f);
-    const bool land_idle = landing && pz <= 0.638f && up_horiz < 0.85f && fabsf(vz) < 0.20f;
-    const float yaw_alpha = asinf(ob_clamp(yaw_ft / fmaxf(thrust, 30.0f), -0.35f, 0.35f));
-    outer_cmd = ob_clamp(6.5f * ob_wrap(yaw_alpha, outer), -outer_limit, outer_limit);
-    const float urx = quad_pick(a, 1.0f, 0.0f, -1.0f, 0.0f);
-    const float ury = quad_pick(a, 0.0f, 1.0f, 0.0f, -1.0f);
-    const float fr_req = 0.5f * (fx_rem * urx + fy_rem * ury);
-    const float sin_in = ob_clamp(fr_req / fmaxf(thrust, 40.0f), -max_sin_inner, max_sin_inner);
-    inner_cmd = ob_clamp(asinf(sin_in), -inner_limit * 0.90f, inner_limit * 0.90f);
-    const float nominal_cos = fmaxf(cosf(yaw_alpha) * cosf(inner_cmd), 0.70f);
-    float target_thrust = fmaxf(fz_cmd, 0.0f) / nominal_cos;
-    if (land_idle) target_thrust = 0.15f * weight * 0.25f;
-    const float u_des =
-        ob_clamp(div_const(target_thrust - min_thrust, max_installed - min_thrust), 0.0f, 1.0f);
-    const float u_raw = u_des + spool_gain * (u_des - spool);
-    // The reference's running maximum over arms 0..3, from -inf.
-    const Quad4 u_all = quad_all(u_raw);
-    float max_raw = -__builtin_huge_valf();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) max_raw = fmaxf(max_raw, u_all.v[i]);
-    const float excess = ob_clamp(max_raw - 1.0f, 0.0f, urgent_climb ? 0.10f : 0.45f);
-    throttle = ob_clamp(u_raw - (need_headroom ? excess : 0.0f), 0.0f, 1.0f);
-    const bool inv_mode = ct < 0.20f;
-    if (inv_mode) {
-        const float inv_rx = te_norm > 1.0e-5f ? e_rx : tilt;
-        const float tx_inv = 130.0f * inv_rx - 52.0f * ox;
-        const float ty_inv = 130.0f * e_ry - 52.0f * oy;
-        const float arm_mom = quad_pick(a, -ty_inv, tx_inv, ty_inv, -tx_inv);
-        throttle = arm_mom > 12.0f ? 0.58f : 0.0f;
-        outer_cmd = ob_clamp(-outer * 6.0f, -outer_limit, outer_limit);
-        inner_cmd = 0.0f;
-    }
-
-    const float aim_err = hypotf(wraps.v[1], des_cannon_el - o[45]);
-    const bool fire = arena && !inv_mode && o[46] <= 0.02f && o[47] > 0.01f && aim_err < 0.28f &&
-                      dist < 34.0f;
-    const bool cannon = arena && !inv_mode;
-    float norm_az =
-        cannon ? ob_clamp(div_const(des_cannon_az - cannon_az_ctr, cannon_az_half), -1.0f, 1.0f) : 0.0f;
-    if (inv_mode) norm_az = -1.0f;
-    float norm_el = cannon ? ob_clamp(div_const(des_cannon_el, cannon_el_lim), -1.0f, 1.0f) : 0.0f;
-    float norm_fire = fire ? 0.8f : -0.8f;
-
-    if (bwb) {
-        const float course_err = wraps.v[2];
-        const float desired_speed =
-            bwb_endurance ? 18.5f : (arena ? (gdist > 38.0f ? 26.0f : 24.0f) : 22.4f);
-        const float speed_err = desired_speed - vb_x;
-        const float u_coll = ob_clamp((bwb_endurance ? 0.36f : 0.44f) + 0.065f * speed_err +
-                                          0.018f * gz, 0.12f, 0.90f);
-        const float desired_roll = ob_clamp(-1.35f * course_err, -0.55f, 0.55f);
-        const float diff_u =
-            ob_clamp(0.90f * (desired_roll - roll_right) - 0.34f * ox, -0.45f, 0.45f);
-        const float u0 = ob_clamp(u_coll + diff_u, 0.05f, 1.0f);
-        const float u1 = ob_clamp(u_coll - diff_u, 0.05f, 1.0f);
-        throttle = (a & 1) ? u1 : u0;
-        const float pitch_up = asinf(ob_clamp(r20, -1.0f, 1.0f));
-        const float climb_des = ob_clamp(0.42f * gz, -5.0f, 5.0f);
-        const float climb_err = climb_des - vz;
-        const float cos_bank = cosines.v[2], sin_bank = sines.v[2];
-        float desired_pitch = ob_clamp(0.062831853f + 0.75f * gamma_des + 0.035f * climb_err +
-                                           0.09f * (1.0f - fmaxf(cos_bank, 0.5f)),
-                                       -0.15f, 0.25f);
-        if (vb_x < 15.5f) desired_pitch = fminf(desired_pitch, 0.02f);
-        const float theta_dot = 2.20f * (desired_pitch - pitch_up);
-        const float psi_dot = (gravity / fmaxf(vb_x, 12.0f)) *
-                                  tanf(ob_clamp(-roll_right, -0.75f, 0.75f)) +
-                              0.35f * course_err;
-        const float q_up = cos_bank * theta_dot - sin_bank * psi_dot;
-        const float r_left = sin_bank * theta_dot + cos_bank * psi_dot;
-        const float gimbal = pi / 6.0f;
-        const float inner0 = ob_clamp(0.85f * (q_up + oy) + 0.03f, -gimbal, gimbal);
-        const float inner1 = ob_clamp(-0.65f * (r_left - oz) - 0.025f * vb_y, -gimbal, gimbal);
-        inner_cmd = quad_pick(a, inner0, inner1, 0.0f, 0.0f);
-        outer_cmd = 0.0f;
-        const float b_err = hypotf(wraps.v[3], b_el - o[45]);
-        const bool b_fire = arena && o[46] <= 0.02f && o[47] > 0.01f && b_err < 0.045f &&
-                            bdist < 165.0f && bbx > 0.0f;
-        norm_az = arena ? ob_clamp(div_const(b_az, pi / 6.0f), -1.0f, 1.0f) : 0.0f;
-        norm_el = arena ? ob_clamp(div_const(b_el, cannon_el_lim), -1.0f, 1.0f) : 0.0f;
-        norm_fire = b_fire ? 0.8f : -0.8f;
-    }
-    ArmOutputs out;
-    out.throttle = ob_clamp(throttle * 2.0f - 1.0f, -1.0f, 1.0f);
-    out.outer = ob_clamp(outer_cmd / outer_limit, -1.0f, 1.0f);
-    out.inner = ob_clamp(div_const(inner_cmd, inner_limit), -1.0f, 1.0f);
-    out.az = norm_az;
-    out.el = norm_el;
-    out.fire = norm_fire;
+    const float course_err = ob_wrap<TAME>(desired_yaw_b, course_yaw);
+    const float arena_speed = gdist > 38.0f ? 26.0f : 24.0f;
+    const float free_speed = f.arena ? arena_speed : 22.4f;
+    const float desired_speed = f.bwb_endurance ? 18.5f : free_speed;
+    const float speed_err = desired_speed - vb_x;
+    const float u_coll = ob_clamp<TAME>((f.bwb_endurance ? 0.36f : 0.44f) + 0.065f * speed_err +
+                                            0.018f * gz, 0.12f, 0.90f);
+    const float desired_roll = ob_clamp<TAME>(-1.35f * course_err, -0.55f, 0.55f);
+    const float diff_u = ob_clamp<TAME>(0.90f * (desired_roll - roll_right) - 0.34f * o[10],
+                                        -0.45f, 0.45f);
+    const float u0 = ob_clamp<TAME>(u_coll + diff_u, 0.05f, 1.0f);
+    const float u1 = ob_clamp<TAME>(u_coll - diff_u, 0.05f, 1.0f);
+    const float throttle = (a & 1) ? u1 : u0;
+    const float pitch_up = asinf(ob_clamp<TAME>(r20, -1.0f, 1.0f));
+    const float climb_err = climb_des - vz;
+    const onboard_math::Direction bank = onboard_math::direction(r21, r22);
+    const float cos_bank = bank.c, sin_bank = bank.s;
+    float desired_pitch = ob_clamp<TAME>(0.062831853f + 0.75f * gamma_des + 0.035f * climb_err +
+                                             0.09f * (1.0f - fmaxf(cos_bank, 0.5f)),
+                                         -0.15f, 0.25f);
+    const float slow_pitch = fminf(desired_pitch, 0.02f);
+    desired_pitch = vb_x < 15.5f ? slow_pitch : desired_pitch;
+    const float theta_dot = 2.20f * (desired_pitch - pitch_up);
+    const float psi_dot = quotient<TAME>(gravity, fmaxf(vb_x, 12.0f)) *
+                              onboard_math::tan_float(ob_clamp<TAME>(-roll_right, -0.75f, 0.75f)) +
+                          0.35f * course_err;
+    const float q_up = cos_bank * theta_dot - sin_bank * psi_dot;
+    const float r_left = sin_bank * theta_dot + cos_bank * psi_dot;
+    const float gimbal = pi / 6.0f;
+    const float inner0 = ob_clamp<TAME>(0.85f * (q_up + o[11]) + 0.03f, -gimbal, gimbal);
+    const float inner1 = ob_clamp<TAME>(-0.65f * (r_left - o[12]) - 0.025f * vb_y, -gimbal, gimbal);
+    const float inner_cmd = quad_pick(a, inner0, inner1, 0.0f, 0.0f);
+    const float b_err = ob_hypot<TAME>(ob_wrap<TAME>(b_az, o44), b_el - o45);
+    const bool b_fire = (int)loaded & (int)(b_err < 0.045f) & (int)(bdist < 165.0f) &
+                        (int)(bbx > 0.0f);
+    const float b_norm_az = ob_clamp<TAME>(div_const(b_az, pi / 6.0f), -1.0f, 1.0f);
+    const float b_norm_el = ob_clamp<TAME>(div_const(b_el, cannon_el_lim), -1.0f, 1.0f);
+    out.az = f.arena ? b_norm_az : 0.0f;
+    out.el = f.arena ? b_norm_el : 0.0f;
+    out.fire = b_fire ? 0.8f : -0.8f;
+    out.arm.throttle = ob_clamp<TAME>(throttle * 2.0f - 1.0f, -1.0f, 1.0f);
+    out.arm.outer = 0.0f;
+    out.arm.inner = ob_clamp<TAME>(div_const(inner_cmd, inner_limit), -1.0f, 1.0f);
     return out;
 }
 
@@ -1397,15 +1554,13 @@ constexpr unsigned kPoolBlocks = 256;     // one workgroup per CU
 // workgroup holds at most a few environments whose mission uses the scan).
 constexpr size_t kPoolMinBatch = 2560;
 // The onboard entry's batches that take the one-kernel form (each
-// workgroup scans its own 64 environments, then runs their controller):
-// those that fill at least 160 of the 256 CUs with one round of 64-
-// environment workgroups.  Measured on one box (two kernels -> one, us):
-// 8,192 envs 20.6 -> 21.4, 10,240 21.95 -> 21.65, 12,288 23.3 -> 21.8,
-// 14,336 24.4 -> 22.1, 16,384 25.4 -> 22.4; with a second round it loses
-// (18,432 36.3 -> 38.8, 65,536 79.4 -> 82.2), as it does with fewer
-// workgroups than CUs (4,096 18.3 -> 21.1): the two-kernel form spreads the
-// scan over every CU.
-constexpr size_t kFusedMinBatch = 160 * 64, kFusedMaxBatch = 256 * 64;
+// workgroup scans its own 64 environments, then runs their controller).
+// Two of its workgroups fit a CU, so one's scan overlaps the other's
+// controller; below kFusedMinBatch the workgroups are fewer than the CUs and
+// the two-kernel form spreads the scan over all of them.  Measured on one
+// box (two kernels -> one, us): 4,000 envs 15.2 -> 16.3, 8,000 17.4 -> 17.0,
+// 20,000 28.2 -> 24.7, 39,999 46.5 -> 42.8, 65,000 60.1 -> 50.3.
+constexpr size_t kFusedMinBatch = 8192;
 struct PoolEntry {
     unsigned env;  // kMaxBatch < 2^31
     int need;
@@ -1544,12 +1699,23 @@ struct ControlStage {
 
 // Phase 2: the tactical features and the controller, from the parked scan
 // result (FUSED: from the workgroup's own scan, phase 1 and 2 in one
-// kernel).  A workgroup covers 64 environments: waves 0..3 run the
-// controller and waves 4..7 the tactical features, each on one quad of lanes
-// per environment (16 per wave), so every SIMD holds one wave of each.
-// Both are long scalar chains and few waves exist per launch, so splitting
-// the work shortens the chains and spreads them over more SIMDs.  For the
-// actor's inputs (SCALARS) each tactical wave then writes the symlog
+// kernel).  A workgroup covers 64 environments: waves 0..3 run the flight
+// controller, waves 4..7 the tactical features, the cannon and the BWB law,
+// each on one quad of lanes per environment (16 per wave), so every SIMD
+// holds one wave of each.  The time of the chains is their instruction
+// count (onboard_math.h), so they are written without branches (conditions
+// are formed first and values selected; as nested conditionals they became
+// 130 branches, with the computation inside and five instructions of mask
+// handling each), take short forms of the functions, and have a form for
+// tame inputs without the reference's checks for infinities and NaN.
+// Cycles of a workgroup's chains at 1,000 environments, before these and
+// after: 16,800 in the flight wave that held BWB missions (13,700 in the
+// others) and 4,800 in the tactical waves -> 7,000 and 11,600.
+//   * One pass per workgroup, without a grid-stride loop: in a loop the
+//     compiler kept 64-bit coefficients and literals in registers across it,
+//     256 of them; without it the chains fit in 128, and two workgroups in a
+//     CU.
+// For the actor's inputs (SCALARS) each tactical wave then writes the symlog
 // scalars and mission values of its 16 environments, one row per store (on
 // the scan waves they cost the scan kernel 6 µs and the plane kernel of the
 // next call 6 µs more).
@@ -1560,15 +1726,6 @@ struct ControlStage {
 //   * Values are formed in registers and then stored to each destination
 //     (the tactical / prior rows and, for the actor, their copies in
 //     proprio and mission_vec).
-// Whether an environment's staged mission selects the BWB law
-// (onboard_features.cuh:433-437, on the values the controller forms).
-__device__ __forceinline__ bool bwb_mission(const float *raw) {
-    const float m2 = ob_mission(raw[2]), m4 = ob_mission(raw[4]), m5 = ob_mission(raw[5]),
-                m6 = ob_mission(raw[6]);
-    return (m6 > 0.75f && m4 < -0.25f) || (m4 > 0.75f && m2 > 0.25f) ||
-           (m6 > 0.75f && m5 > 0.60f);
-}
-
 // FUSED: the workgroup also scans its own environments (the onboard
 // entry's one-kernel form), from a pool in LDS over its eight waves, and the
 // results go straight into the stage.
@@ -1681,11 +1838,10 @@ __device__ __forceinline__ void fused_scan(const OnboardRows &rows, size_t base,
 }
 
 template <bool SCALARS, bool FUSED>
-__global__ __launch_bounds__(kControlThreads) void onboard_control_kernel(OnboardRows rows) {
+__global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void onboard_control_kernel(OnboardRows rows) {
     constexpr int CW = kControlWaves, N = 64, kThreads = kControlThreads;
     __shared__ ControlStage stage;
-    // Per controller wave: the workgroup's environments, BWB missions first.
-    __shared__ unsigned char order[CW][N];
     __shared__ std::conditional_t<FUSED, FusedScanLds, char> fused;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1697,193 +1853,177 @@ __global__ __launch_bounds__(kControlThreads) void onboard_control_kernel(Onboar
             fused.rays.d[2][i] = kRayDir[i * 3 + 2];
         }
     }
-    for (size_t base = (size_t)blockIdx.x * N; base < rows.batch;
-         base += (size_t)gridDim.x * N) {
-        // Rows past the batch end re-read the last row; nothing uses them.
-        auto row_of = [&](int e) {
-            const size_t env = base + (size_t)e;
-            return env < rows.batch ? env : rows.batch - 1;
-        };
-        constexpr int kObsLoads = (N * kStageObs + kThreads - 1) / kThreads;
-        constexpr int kMissionLoads = (N * 10 + kThreads - 1) / kThreads;
-        constexpr int kScanLoads = (N * 7 + kThreads - 1) / kThreads;
-        // Every thread issues all its loads unconditionally (an index past
-        // the stage re-reads the stage's last value), so they leave at once.
-        float vo[kObsLoads], vm[kMissionLoads], vs[kScanLoads], vt = 0.0f;
+    const size_t base = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * N;
+    if (base >= rows.batch) return;
+    // Rows past the batch end re-read the last row; nothing uses them.
+    auto row_of = [&](int e) {
+        const size_t env = base + (size_t)e;
+        return env < rows.batch ? env : rows.batch - 1;
+    };
+    constexpr int kObsLoads = (N * kStageObs + kThreads - 1) / kThreads;
+    constexpr int kMissionLoads = (N * 10 + kThreads - 1) / kThreads;
+    constexpr int kScanLoads = (N * 7 + kThreads - 1) / kThreads;
+    // Every thread issues all its loads unconditionally (an index past
+    // the stage re-reads the stage's last value), so they leave at once.
+    float vo[kObsLoads], vm[kMissionLoads], vs[kScanLoads], vt = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kObsLoads; ++k) {
-            const int idx = min(tid + kThreads * k, N * kStageObs - 1);
-            const int e = idx / kStageObs, i = idx - kStageObs * e;
-            vo[k] = reinterpret_cast<const float *>(rows.obs + row_of(e) * rows.obs_stride)[i];
-        }
-#pragma unroll
-        for (int k = 0; k < kMissionLoads; ++k) {
-            const int idx = min(tid + kThreads * k, N * 10 - 1);
-            const int e = idx / 10, i = idx - 10 * e;
-            vm[k] = reinterpret_cast<const float *>(rows.mission + row_of(e) * rows.mission_stride)[i];
-        }
-#pragma unroll
-        for (int k = 0; k < kScanLoads; ++k) {
-            const int idx = min(tid + kThreads * k, N * 7 - 1);
-            const int e = idx / 7, i = idx - 7 * e;
-            vs[k] = FUSED ? 0.0f : rows.prior[row_of(e) * 15 + i];
-        }
-        if (SCALARS) {
-            const int idx = min(tid, N * 4 - 1);
-            const int e = idx / 4;
-            vt = reinterpret_cast<const float *>(
-                rows.obs + row_of(e) * rows.obs_stride)[4144 + idx - 4 * e];
-        }
-#pragma unroll
-        for (int k = 0; k < kObsLoads; ++k) {
-            const int idx = tid + kThreads * k;
-            const int e = idx / kStageObs;
-            if (idx < N * kStageObs) stage.obs[e][idx - kStageObs * e] = vo[k];
-        }
-#pragma unroll
-        for (int k = 0; k < kMissionLoads; ++k) {
-            const int idx = tid + kThreads * k;
-            const int e = idx / 10;
-            if (idx < N * 10) stage.mission[e][idx - 10 * e] = vm[k];
-        }
-#pragma unroll
-        for (int k = 0; k < kScanLoads; ++k) {
-            const int idx = tid + kThreads * k;
-            const int e = idx / 7;
-            if (!FUSED && idx < N * 7) stage.scan[e][idx - 7 * e] = vs[k];
-        }
-        if (SCALARS && tid < N * 4) stage.tail[tid / 4][tid % 4] = vt;
-        __syncthreads();
-        if constexpr (FUSED) fused_scan(rows, base, stage, fused, w, lane);
-
-        // The controller waves take the workgroup's environments BWB
-        // missions first, so that all but about one wave of them have no
-        // BWB environment and skip the BWB blocks, which a wave runs when
-        // any of its quads needs them.  (18% of the benchmark's missions are
-        // BWB, and 96% of 16-environment waves held one: 34.47 -> 34.06 us
-        // for the entry.  The wave that keeps BWB environments still runs
-        // the whole chain, and its SIMD sets the time; with the BWB blocks
-        // removed from every wave the entry would take 1.4 us less.)  Each
-        // controller wave ranks the 64 environments itself (lane e ranks
-        // environment e) into its own table and reads back its quads'
-        // environments.  Every environment's values are the same in any
-        // order.
-        // Tactical waves: environment 16 (w - 4) + lane / 4.
-        int slot = 16 * (w - CW) + (lane >> 2);
-        if (w < CW) {
-            const bool b = bwb_mission(stage.mission[lane]);
-            const uint64_t bm = __builtin_amdgcn_ballot_w64(b);
-            const unsigned nb = (unsigned)__builtin_popcountll(bm);
-            const uint64_t mine = b ? bm : ~bm;
-            const unsigned below = __builtin_amdgcn_mbcnt_hi(
-                (unsigned)(mine >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0u));
-            order[w][b ? below : nb + below] = (unsigned char)lane;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            slot = order[w][16 * w + (lane >> 2)];
-        }
-
-        const size_t env = base + (size_t)slot;
-        if (env < rows.batch) {
-            const float *obs = stage.obs[slot];
-            const float *mission = stage.mission[slot];
-            if (w >= CW) {
-                // Lane a of the quad writes features 6a .. 6a + 5.
-                float t[6];
-                tactical_quad(obs, mission, a, t);
-                float *tac = rows.tactical + env * 24 + 6 * a;
-#pragma unroll
-                for (int i = 0; i < 6; ++i) tac[i] = t[i];
-                if (rows.proprio) {
-                    float *p = rows.proprio + env * 91 + 52 + 6 * a,
-                          *mv = rows.mission_vec + env * 49 + 10 + 6 * a;
-#pragma unroll
-                    for (int i = 0; i < 6; ++i) {
-                        p[i] = t[i];
-                        mv[i] = t[i];
-                    }
-                }
-            } else {
-                const float *sc = stage.scan[slot];
-                ScanResult s;
-                s.min_r = sc[0];
-                s.min_r_dx = sc[1];
-                s.min_r_dy = sc[2];
-                s.min_dx_c = sc[3];
-                s.cluster_y_sum = sc[4];
-                s.min_ray = __float_as_int(sc[5]);
-                s.cluster_count = __float_as_int(sc[6]);
-                // Read from LDS before the chain, like the other inputs.
-                asm volatile("" : "+v"(s.min_r), "+v"(s.min_r_dx), "+v"(s.min_r_dy), "+v"(s.min_dx_c),
-                             "+v"(s.cluster_y_sum), "+v"(s.min_ray), "+v"(s.cluster_count));
-                const ArmOutputs n = prior_features(obs, mission, s, a);
-                // The parked result was staged before the chain; each lane
-                // now writes its arm's three values, lane 0 the cannon's.
-                float *prior = rows.prior + env * 15;
-                prior[a] = n.throttle;
-                prior[4 + a] = n.outer;
-                prior[8 + a] = n.inner;
-                if (a == 0) {
-                    prior[12] = n.az;
-                    prior[13] = n.el;
-                    prior[14] = n.fire;
-                }
-                if (rows.proprio) {
-                    float *p = rows.proprio + env * 91 + 76, *mv = rows.mission_vec + env * 49 + 34;
-                    p[a] = n.throttle;
-                    p[4 + a] = n.outer;
-                    p[8 + a] = n.inner;
-                    mv[a] = n.throttle;
-                    mv[4 + a] = n.outer;
-                    mv[8 + a] = n.inner;
-                    if (a == 0) {
-                        p[12] = n.az;
-                        p[13] = n.el;
-                        p[14] = n.fire;
-                        mv[12] = n.az;
-                        mv[13] = n.el;
-                        mv[14] = n.fire;
-                    }
-                }
-                if (rows.diag && a == 0) {
-                    float *d = rows.diag + env * 5;
-                    d[0] = s.min_r;
-                    d[1] = (float)s.min_ray;
-                    d[2] = s.min_dx_c;
-                    d[3] = (float)s.cluster_count;
-                    d[4] = s.cluster_y_sum;
-                }
-            }
-        }
-        if (SCALARS && w >= CW) {
-            // Lane l's input: obs[l] (l < 48), obs[4144 + l - 48] (l < 52),
-            // mission[l - 52] (l < 62).
-            const int lo = min(lane, kStageObs - 1), lt = min(max(lane - 48, 0), 3),
-                      lm = min(max(lane - 52, 0), 9);
-            // All 16 inputs are read first, so the 16 chains are
-            // independent; rows past the batch end (staged as copies of the
-            // last row) store nothing.
-            float raw[16];
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int e = 16 * (w - CW) + j;
-                raw[j] = lane < 48 ? stage.obs[e][lo]
-                                   : (lane < 52 ? stage.tail[e][lt] : stage.mission[e][lm]);
-            }
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const size_t env = base + (size_t)(16 * (w - CW) + j);
-                const bool valid = env < rows.batch;
-                const size_t row = valid ? env : base;
-                actor_scalars(raw[j], lane, rows.proprio + row * 91, rows.mission_vec + row * 49,
-                              valid);
-            }
-        }
-
-        // The stage is reused by this workgroup's next 64 environments.
-        if (base + (size_t)gridDim.x * N < rows.batch) __syncthreads();
+    for (int k = 0; k < kObsLoads; ++k) {
+        const int idx = min(tid + kThreads * k, N * kStageObs - 1);
+        const int e = idx / kStageObs, i = idx - kStageObs * e;
+        vo[k] = reinterpret_cast<const float *>(rows.obs + row_of(e) * rows.obs_stride)[i];
     }
+#pragma unroll
+    for (int k = 0; k < kMissionLoads; ++k) {
+        const int idx = min(tid + kThreads * k, N * 10 - 1);
+        const int e = idx / 10, i = idx - 10 * e;
+        vm[k] = reinterpret_cast<const float *>(rows.mission + row_of(e) * rows.mission_stride)[i];
+    }
+#pragma unroll
+    for (int k = 0; k < kScanLoads; ++k) {
+        const int idx = min(tid + kThreads * k, N * 7 - 1);
+        const int e = idx / 7, i = idx - 7 * e;
+        vs[k] = FUSED ? 0.0f : rows.prior[row_of(e) * 15 + i];
+    }
+    if (SCALARS) {
+        const int idx = min(tid, N * 4 - 1);
+        const int e = idx / 4;
+        vt = reinterpret_cast<const float *>(
+            rows.obs + row_of(e) * rows.obs_stride)[4144 + idx - 4 * e];
+    }
+#pragma unroll
+    for (int k = 0; k < kObsLoads; ++k) {
+        const int idx = tid + kThreads * k;
+        const int e = idx / kStageObs;
+        if (idx < N * kStageObs) stage.obs[e][idx - kStageObs * e] = vo[k];
+    }
+#pragma unroll
+    for (int k = 0; k < kMissionLoads; ++k) {
+        const int idx = tid + kThreads * k;
+        const int e = idx / 10;
+        if (idx < N * 10) stage.mission[e][idx - 10 * e] = vm[k];
+    }
+#pragma unroll
+    for (int k = 0; k < kScanLoads; ++k) {
+        const int idx = tid + kThreads * k;
+        const int e = idx / 7;
+        if (!FUSED && idx < N * 7) stage.scan[e][idx - 7 * e] = vs[k];
+    }
+    if (SCALARS && tid < N * 4) stage.tail[tid / 4][tid % 4] = vt;
+    __syncthreads();
+    if constexpr (FUSED) fused_scan(rows, base, stage, fused, w, lane);
+
+    const int slot = 16 * (w & (CW - 1)) + (lane >> 2);
+    const size_t env = base + (size_t)slot;
+    if (env < rows.batch) {
+        ChainInputs in = chain_inputs(stage.obs[slot], stage.mission[slot], a);
+        const bool tame = tame_inputs(in);
+        float *const prior = rows.prior + env * 15;
+        float *const p = rows.proprio ? rows.proprio + env * 91 + 52 : nullptr;
+        float *const mv = rows.proprio ? rows.mission_vec + env * 49 + 10 : nullptr;
+        auto store_arm = [&](const ArmOutputs &n) {
+            prior[a] = n.throttle;
+            prior[4 + a] = n.outer;
+            prior[8 + a] = n.inner;
+            if (p) {
+                p[24 + a] = n.throttle;
+                p[28 + a] = n.outer;
+                p[32 + a] = n.inner;
+                mv[24 + a] = n.throttle;
+                mv[28 + a] = n.outer;
+                mv[32 + a] = n.inner;
+            }
+        };
+        if (w >= CW) {
+            // Lane a of the quad writes features 6a .. 6a + 5.
+            float t[6];
+            if (tame) tactical_quad<true>(in, a, t);
+            else tactical_quad<false>(in, a, t);
+            float *tac = rows.tactical + env * 24 + 6 * a;
+#pragma unroll
+            for (int i = 0; i < 6; ++i) tac[i] = t[i];
+            if (p) {
+#pragma unroll
+                for (int i = 0; i < 6; ++i) {
+                    p[6 * a + i] = t[i];
+                    mv[6 * a + i] = t[i];
+                }
+            }
+            if (!tame) controller_inputs(in);
+            const MissionFlags f = mission_flags(in.m);
+            const GunOutputs g = tame ? gunnery_quad<true>(in, f, a) : gunnery_quad<false>(in, f, a);
+            if (f.bwb) store_arm(g.arm);
+            if (a == 0) {
+                prior[12] = g.az;
+                prior[13] = g.el;
+                prior[14] = g.fire;
+                if (p) {
+                    p[36] = g.az;
+                    p[37] = g.el;
+                    p[38] = g.fire;
+                    mv[36] = g.az;
+                    mv[37] = g.el;
+                    mv[38] = g.fire;
+                }
+            }
+        } else {
+            const float *sc = stage.scan[slot];
+            ScanResult s;
+            s.min_r = sc[0];
+            s.min_r_dx = sc[1];
+            s.min_r_dy = sc[2];
+            s.min_dx_c = sc[3];
+            s.cluster_y_sum = sc[4];
+            s.min_ray = __float_as_int(sc[5]);
+            s.cluster_count = __float_as_int(sc[6]);
+            // Read from LDS before the chain, like the other inputs.
+            asm volatile("" : "+v"(s.min_r), "+v"(s.min_r_dx), "+v"(s.min_r_dy), "+v"(s.min_dx_c),
+                         "+v"(s.cluster_y_sum), "+v"(s.min_ray), "+v"(s.cluster_count));
+            if (!tame) controller_inputs(in);
+            const MissionFlags f = mission_flags(in.m);
+            const ArmOutputs n =
+                tame ? flight_quad<true>(in, f, s, a) : flight_quad<false>(in, f, s, a);
+            if (!f.bwb) store_arm(n);  // a BWB mission's are the other waves'
+            if (rows.diag && a == 0) {
+                float *d = rows.diag + env * 5;
+                d[0] = s.min_r;
+                d[1] = (float)s.min_ray;
+                d[2] = s.min_dx_c;
+                d[3] = (float)s.cluster_count;
+                d[4] = s.cluster_y_sum;
+            }
+        }
+    }
+    if (SCALARS && w >= CW) {
+        // Lane l's input: obs[l] (l < 48), obs[4144 + l - 48] (l < 52),
+        // mission[l - 52] (l < 62).
+        const int lo = min(lane, kStageObs - 1), lt = min(max(lane - 48, 0), 3),
+                  lm = min(max(lane - 52, 0), 9);
+        // All 16 inputs are read first, so the 16 chains are
+        // independent; rows past the batch end (staged as copies of the
+        // last row) store nothing.
+        float raw[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const int e = 16 * (w - CW) + j;
+            raw[j] = lane < 48 ? stage.obs[e][lo]
+                               : (lane < 52 ? stage.tail[e][lt] : stage.mission[e][lm]);
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            const size_t env = base + (size_t)(16 * (w - CW) + j);
+            const bool valid = env < rows.batch;
+            const size_t row = valid ? env : base;
+            actor_scalars(raw[j], lane, rows.proprio + row * 91, rows.mission_vec + row * 49,
+                          valid);
+        }
+    }
+}
+
+// One workgroup per 64 environments.
+dim3 control_grid(size_t batch) {
+    const size_t want = (batch + 63) / 64;
+    return dim3((unsigned)(want < kControlGridX ? want : kControlGridX),
+                (unsigned)((want + kControlGridX - 1) / kControlGridX));
 }
 
 // `pooled` selects the pooled scan, which holds a whole CU per workgroup:
@@ -1891,7 +2031,6 @@ __global__ __launch_bounds__(kControlThreads) void onboard_control_kernel(Onboar
 int launch_onboard(const OnboardRows &rows, hipStream_t s, bool pooled) {
     const size_t scan_want = (rows.batch + kWavesPerBlock - 1) / kWavesPerBlock;
     const unsigned scan_blocks = scan_want > kScanBlocks ? kScanBlocks : (unsigned)scan_want;
-    const size_t ctrl_want = (rows.batch + 63) / 64;
     if (rows.lidar) {
         onboard_scan_kernel<true><<<scan_blocks, kBlockThreads, 0, s>>>(rows);
     } else if (pooled) {
@@ -1903,11 +2042,11 @@ int launch_onboard(const OnboardRows &rows, hipStream_t s, bool pooled) {
     } else {
         onboard_scan_kernel<false><<<scan_blocks, kBlockThreads, 0, s>>>(rows);
     }
-    const unsigned ctrl_blocks = ctrl_want > kControlBlocks ? kControlBlocks : (unsigned)ctrl_want;
+    const dim3 ctrl = control_grid(rows.batch);
     if (rows.proprio)
-        onboard_control_kernel<true, false><<<ctrl_blocks, kControlThreads, 0, s>>>(rows);
+        onboard_control_kernel<true, false><<<ctrl, kControlThreads, 0, s>>>(rows);
     else
-        onboard_control_kernel<false, false><<<ctrl_blocks, kControlThreads, 0, s>>>(rows);
+        onboard_control_kernel<false, false><<<ctrl, kControlThreads, 0, s>>>(rows);
     return hipGetLastError() == hipSuccess;
 }
 
@@ -1931,10 +2070,9 @@ extern "C" int tb_hip_onboard_tactical_prior_device(const float *obs, const floa
     rows.lidar = nullptr;
     rows.batch = batch_size;
     (void)hipGetLastError();
-    if (batch_size >= kFusedMinBatch && batch_size <= kFusedMaxBatch) {
-        // One round of 64-environment workgroups, one per CU.
+    if (batch_size >= kFusedMinBatch) {
         onboard_control_kernel<false, true>
-            <<<(unsigned)((batch_size + 63) / 64), kControlThreads, 0,
+            <<<control_grid(batch_size), kControlThreads, 0,
                reinterpret_cast<hipStream_t>(stream)>>>(rows);
         return hipGetLastError() == hipSuccess;
     }
