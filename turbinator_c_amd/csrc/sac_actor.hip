@@ -175,69 +175,101 @@ struct PackArgs {
     unsigned *out;  // the packed buffer as 32-bit words
 };
 
-// The scale exponent of packed row n of layer l: the row's weights times
-// 2^s lie below 2^15 in magnitude.
-__device__ int row_scale(const PackArgs &a, int l, int n) {
-    if (n >= a.n[l]) return 0;
-    const float *row = a.w[l] + (size_t)(l == 2 ? raw_row(n) : n) * a.k[l];
-    unsigned m = 0;
-    for (int k = 0; k < a.k[l]; ++k) {
-        const unsigned b = __float_as_uint(row[k]) & 0x7fffffffu;
-        m = b > m ? b : m;
-    }
-    return row_exponent(m);
-}
+// Packs one output tile (16 rows of one layer): workgroup b is tile b of the
+// three layers' tiles in order.  The rows are read once, 16 threads each with
+// every load of a thread issued before any is used; their magnitudes are
+// reduced over those 16 lanes to the row's scale, the scaled rows pass
+// through LDS, and each thread writes whole 16-byte vectors (one lane's
+// eight positions of a chunk) of both pieces.  The first layer's workgroups
+// also write their rows of the fp32 copy, and the last tile of a layer (and
+// of the copy) the zero padding up to the next section.
+// What bounds it is one round trip for the rows and one for the stores; a
+// kernel with one thread per packed word, each scanning its row for the
+// scale, took 25.6 us at hidden 256 (kernel trace), this one 4.2.
+constexpr int kPackThreads = 256;
+constexpr int kRowLanes = kPackThreads / 16;  // threads per row
 
-// The packed weight piece pair at byte offset `e` of layer l's weight
-// section: two fp16 values of one piece, chunk positions i0 and i0 + 1.
-__device__ unsigned packed_weight_pair(const PackArgs &a, int l, size_t e) {
-    const size_t block = e / kBlockBytes;
-    const int within = (int)(e % kBlockBytes);
-    const int piece = within / 1024, lane = (within % 1024) / 16, i0 = (within % 16) / 2;
-    const int tile = (int)(block / a.kc[l]), c = (int)(block % a.kc[l]);
-    const int n = 16 * tile + (lane & 15);
-    const int scale = row_scale(a, l, n);
-    f32x2 v = {0.0f, 0.0f};
+__global__ __launch_bounds__(kPackThreads) void sac_pack_kernel(PackArgs a) {
+    __shared__ float rows[16][kMaxHidden + 1];
+    __shared__ int scales[16];
+    const int tid = threadIdx.x;
+    int l = 0, tile = blockIdx.x;
+    while (tile >= a.nt[l]) tile -= a.nt[l++];  // the grid is the sum of nt[]
+    const int kl = a.k[l];
+    {
+        const int r = tid / kRowLanes, j = tid % kRowLanes, n = 16 * tile + r;
+        const bool live = n < a.n[l];
+        const float *row = a.w[l] + (size_t)(live ? (l == 2 ? raw_row(n) : n) : 0) * kl;
+        float v[kMaxHidden / kRowLanes];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int k = chunk_input(l, c, 8 * (lane >> 4) + i0 + h);
-        if (n < a.n[l] && k < a.k[l])
-            v[h] = __builtin_amdgcn_ldexpf(
-                a.w[l][(size_t)(l == 2 ? raw_row(n) : n) * a.k[l] + k], scale);
-    }
-    unsigned p[kPieces];
-    split_pair(v, p[0], p[1]);
-    return p[piece];
-}
-
-// One thread per packed 32-bit word.
-__global__ __launch_bounds__(256) void sac_pack_kernel(PackArgs a) {
-    const size_t words = a.layout.total / 4;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < words;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const size_t byte = 4 * i;
-        unsigned v = 0;
-        for (int l = 0; l < 3; ++l) {
-            const size_t wsize = (size_t)a.nt[l] * a.kc[l] * kBlockBytes;
-            if (byte >= a.layout.w[l] && byte < a.layout.w[l] + wsize) {
-                v = packed_weight_pair(a, l, byte - a.layout.w[l]);
-            } else if (byte >= a.layout.b[l] &&
-                       byte < a.layout.b[l] + (size_t)a.nt[l] * kTileScaleBytes) {
-                // Tile block: biases of rows 16 t .. +15, then the exponents
-                // that undo the row scale (and the hidden inputs' 2^14).
-                const int e = (int)((byte - a.layout.b[l]) / 4);
-                const int n = 16 * (e / 32) + (e % 16);
-                if (n < a.n[l]) {
-                    if (e % 32 < 16)
-                        v = __float_as_uint(a.b[l][l == 2 ? raw_row(n) : n]);
-                    else
-                        v = (unsigned)(-row_scale(a, l, n) - (l == 0 ? 0 : kHiddenScale));
-                }
-            }
+        for (int i = 0; i < kMaxHidden / kRowLanes; ++i) {
+            const int k = j + kRowLanes * i;
+            v[i] = live && k < kl ? row[k] : 0.0f;
         }
-        if (byte >= a.layout.w0 && byte < a.layout.w0 + (size_t)a.hidden * kFeatures * 4)
-            v = __float_as_uint(a.w[0][(byte - a.layout.w0) / 4]);
-        a.out[i] = v;
+        unsigned m = 0;
+#pragma unroll
+        for (int i = 0; i < kMaxHidden / kRowLanes; ++i) {
+            const unsigned b = __float_as_uint(v[i]) & 0x7fffffffu;
+            m = b > m ? b : m;
+        }
+#pragma unroll
+        for (int d = 1; d < kRowLanes; d <<= 1) {
+            const unsigned o = (unsigned)__shfl_xor((int)m, d);
+            m = o > m ? o : m;
+        }
+        // The row's weights times 2^scale lie below 2^15 in magnitude.
+        const int scale = live ? row_exponent(m) : 0;
+        if (j == 0) scales[r] = scale;
+#pragma unroll
+        for (int i = 0; i < kMaxHidden / kRowLanes; ++i) {
+            const int k = j + kRowLanes * i;
+            rows[r][k] = __builtin_amdgcn_ldexpf(v[i], scale);
+            if (l == 0 && live && k < kl)
+                a.out[a.layout.w0 / 4 + (size_t)n * kFeatures + k] = __float_as_uint(v[i]);
+        }
+    }
+    __syncthreads();
+    // Lane vectors of the tile: chunk c, lane x, both pieces.
+    u32x4 *block = reinterpret_cast<u32x4 *>(a.out + (a.layout.w[l] + (size_t)tile * a.kc[l] * kBlockBytes) / 4);
+    for (int e = tid; e < a.kc[l] * 64; e += kPackThreads) {
+        const int c = e / 64, x = e % 64;
+        u32x4 hi, lo;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            f32x2 v;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int k = chunk_input(l, c, 8 * (x >> 4) + 2 * i + h);
+                v[h] = k < kl ? rows[x & 15][k] : 0.0f;
+            }
+            unsigned p0, p1;
+            split_pair(v, p0, p1);
+            hi[i] = p0;
+            lo[i] = p1;
+        }
+        block[c * (kBlockBytes / 16) + x] = hi;
+        block[c * (kBlockBytes / 16) + 64 + x] = lo;
+    }
+    // The tile's biases, and the exponents that undo the row scale (and the
+    // hidden inputs' 2^14).
+    unsigned *const out = a.out;
+    if (tid < 32) {
+        const int n = 16 * tile + tid % 16;
+        unsigned v = 0;
+        if (n < a.n[l])
+            v = tid < 16 ? __float_as_uint(a.b[l][l == 2 ? raw_row(n) : n])
+                         : (unsigned)(-scales[tid % 16] - (l == 0 ? 0 : kHiddenScale));
+        out[(a.layout.b[l] + (size_t)tile * kTileScaleBytes) / 4 + tid] = v;
+    }
+    // Zeros up to the next section.
+    auto pad = [&](size_t from, size_t to) {
+        for (size_t i = from / 4 + tid; i < to / 4; i += kPackThreads) out[i] = 0;
+    };
+    if (tile == a.nt[l] - 1) {
+        pad(a.layout.b[l] + (size_t)a.nt[l] * kTileScaleBytes,
+            l < 2 ? a.layout.w[l + 1] : a.layout.w0);
+        if (l == 0)
+            pad(a.layout.w0 + (size_t)a.hidden * kFeatures * sizeof(float), a.layout.total);
     }
 }
 
@@ -749,8 +781,8 @@ extern "C" int tb_hip_sac_actor_pack_device(const float *w0, const float *b0, co
     }
     a.out = static_cast<unsigned *>(packed);
     (void)hipGetLastError();
-    const size_t blocks = (a.layout.total / 4 + 255) / 256;
-    sac_pack_kernel<<<(unsigned)blocks, 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(a);
+    const unsigned blocks = (unsigned)(nt[0] + nt[1] + nt[2]);
+    sac_pack_kernel<<<blocks, kPackThreads, 0, reinterpret_cast<hipStream_t>(stream)>>>(a);
     return hipGetLastError() == hipSuccess;
 }
 
