@@ -304,21 +304,32 @@ __device__ __forceinline__ float tanh_hidden_scaled(float x) {
     return __builtin_fmaf(-32768.0f, __builtin_amdgcn_rcpf(e + 1.0f), 16384.0f);
 }
 
-// A workgroup's NW waves share NW / 2 groups of 16 environments: in the
-// 142 -> hidden and hidden -> hidden layers wave w computes output tiles
-// w, w + NW, ... for all groups; in the hidden -> 30 layer (two tiles per
-// group) wave w computes tile w % 2 of group w / 2.  The finished tiles go
-// through LDS to all the waves as the next layer's input fragments.  Above
-// 4 hidden tiles NW = 8: a 16,384-row batch is 256 workgroups, one per CU,
-// every SIMD holds two waves with the same matrix-core work, and a CU reads
-// each weight once (NW = 4, two workgroups per CU, reads each weight twice
-// per CU: 9.4 against 9.1 us at hidden 128; four groups on four waves, one
-// wave per SIMD: 11.7 us).  Up to 4 hidden tiles NW = 4, so that waves do
-// not compute empty tiles (hidden 16: 6.4 against 7.3 us).
+// A workgroup's NW waves share G groups of 16 environments: in the 142 ->
+// hidden and hidden -> hidden layers wave w computes output tiles w, w + NW,
+// ... for all groups; in the hidden -> 30 layer (two tiles per group) wave w
+// computes tile w % 2 of its groups.  The finished tiles go through LDS to
+// all the waves as the next layer's input fragments.
+//
+// Full batches: G = NW / 2.  Above 4 hidden tiles NW = 8: a 16,384-row batch
+// is 256 workgroups, one per CU, every SIMD holds two waves with the same
+// matrix-core work, and a CU reads each weight once (NW = 4, two workgroups
+// per CU, reads each weight twice per CU: 9.4 against 9.1 us at hidden 128;
+// four groups on four waves, one wave per SIMD: 11.7 us).  Up to 4 hidden
+// tiles NW = 4, so that waves do not compute empty tiles (hidden 16: 6.4
+// against 7.3 us).
 template <int HT>
 struct Shape {
     static constexpr int waves = HT <= 4 ? 4 : 8;
     static constexpr int groups = waves / 2;  // groups of 16 environments per workgroup pass
+};
+// Small batches leave CUs idle, and their time is one workgroup's latency:
+// the round trips for the weights of three layers and the matrix-core steps
+// of its groups.  So fewer environments per workgroup (1 or 2 groups), a
+// wave for every hidden tile (up to 16), and each layer's weights requested
+// as early as its registers allow, the second layer's with the first's.
+template <int HT>
+struct SmallShape {
+    static constexpr int waves = HT <= 4 ? 4 : HT <= 8 ? 8 : 16;
 };
 
 // LDS rows of the workgroup: one per environment, KC chunks of 128 bytes
@@ -332,7 +343,7 @@ __host__ __device__ constexpr int row_bytes(int kc) { return kc * kPieces * kChu
 // chunk s, pieces of positions 8g .. +7 of environment l % 16 of each group,
 // as two 16-byte LDS reads.  Every weight fragment a wave loads feeds
 // 3 G matrix-core steps, so L2 delivers 2 KiB of weights per 3 G MFMAs.
-// Weight chunks stream through a ring of ring_depth register slots: the
+// Weight chunks stream through a ring of D register slots: the
 // chunk of step s + D - 1 is requested while step s runs.  The loop has no
 // branches: a slot j past the layer's tiles (when NT is not a multiple of
 // NW) reads its weights and bias at an offset past the buffer end, which the
@@ -349,9 +360,9 @@ constexpr int ring_depth() { return TPW <= 2 ? 4 : 2; }
 // The first weight chunks and the bias of this wave's tiles of one layer,
 // requested ahead of the layer (layer_prefetch) so that their round trip
 // overlaps the previous phase of the pass.
-template <int TPW>
+template <int TPW, int D>
 struct LayerWeights {
-    u32x4 ring[ring_depth<TPW>()][TPW][kPieces];
+    u32x4 ring[D][TPW][kPieces];
     f32x4 bias[TPW];
     i32x4 unscale[TPW];
 };
@@ -383,11 +394,10 @@ __device__ __forceinline__ void load_chunk(__amdgpu_buffer_rsrc_t rsrc, unsigned
                 rsrc, wl[j], w_off + kBlockBytes * (nt[j] * KC + s) + 1024u * p, 0);
 }
 
-template <int KC, int NT, int TPW, int NW>
+template <int KC, int NT, int TPW, int NW, int D>
 __device__ __forceinline__ void layer_prefetch(__amdgpu_buffer_rsrc_t rsrc, unsigned w_off,
                                                unsigned b_off, int w, int lane,
-                                               LayerWeights<TPW> &lw) {
-    constexpr int D = ring_depth<TPW>();
+                                               LayerWeights<TPW, D> &lw) {
     unsigned wl[TPW], bl[TPW];
     int nt[TPW];
     tile_slots<NT, TPW, NW>(w, lane, wl, bl, nt);
@@ -419,12 +429,11 @@ constexpr int kTermX[kTerms] = {0, 1, 0};
 // sums times 2^(row exponent - shift[q]), plus the bias.  `rows` are the
 // layer's input rows in LDS, RS bytes apart; shift[q] is the scale exponent
 // of group q's inputs beyond the one the packed exponents already undo.
-template <int KC, int NT, int TPW, int G, int RS, int NW>
+template <int KC, int NT, int TPW, int G, int RS, int NW, int D>
 __device__ __forceinline__ void layer_tiles(__amdgpu_buffer_rsrc_t rsrc, unsigned w_off,
-                                            const u32x4 *rows, LayerWeights<TPW> &lw,
+                                            const u32x4 *rows, LayerWeights<TPW, D> &lw,
                                             const int (&shift)[G], f32x4 (&out)[TPW][G], int w,
                                             int lane) {
-    constexpr int D = ring_depth<TPW>();
     constexpr int RS16 = RS / 16;
     const int g = lane >> 4;
     const u32x4 *in = rows + (lane & 15) * RS16 + g;  // group q, chunk s, piece p:
@@ -520,13 +529,22 @@ __device__ __forceinline__ void store_tiles(unsigned char *rows, f32x4 (&h)[TPW]
     }
 }
 
-template <int HT, int G, int NW>
+// EARLY: the second layer's first weight chunks are requested with the first
+// layer's (small batches), else when the first layer's are used up.
+template <int HT, int G, int NW, bool EARLY>
 __global__ __launch_bounds__(NW * 64) void sac_actor_kernel(ActArgs a) {
     constexpr int TPW = (HT + NW - 1) / NW;  // hidden tiles per wave
     constexpr int HC = (HT + 1) / 2;                 // hidden chunks of 32 inputs
-    // The hidden -> 30 layer's 2 G (tile, group) pairs, G2 groups per wave.
-    static_assert(2 * G % NW == 0, "whole groups per wave in the hidden -> 30 layer");
-    constexpr int G2 = 2 * G / NW;
+    // Ring slots per layer.  EARLY holds a whole layer where 128 registers
+    // allow it (16 waves): 5 slots for the first layer, 6 or 5 of up to 8 chunks
+    // for the second, all for the last.
+    constexpr int D0 = EARLY ? kFeatureChunks : ring_depth<TPW>();
+    constexpr int D1 = EARLY ? (HC < 7 - G ? HC : 7 - G) : ring_depth<TPW>();
+    constexpr int D2 = EARLY ? HC : ring_depth<1>();
+    // The hidden -> 30 layer's 2 G (tile, group) pairs: G2 groups per wave,
+    // or one for the first 2 G waves.
+    static_assert(2 * G % NW == 0 || 2 * G < NW, "whole groups per wave in the hidden -> 30 layer");
+    constexpr int G2 = 2 * G < NW ? 1 : 2 * G / NW;
     constexpr int E = 16 * G;                        // environments per workgroup pass
     // Buffer 1 holds the features during layer 0 and the second hidden layer
     // afterwards; buffer 0 the first hidden layer.
@@ -543,210 +561,246 @@ __global__ __launch_bounds__(NW * 64) void sac_actor_kernel(ActArgs a) {
     const int g = lane >> 4, j = lane & 15;
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(a.packed, a.packed_bytes);
 
-    // The loop bound is uniform over the block, so every wave meets the
-    // barriers; rows past the batch end compute on zeros and store nothing.
-    // Groups go to workgroups in XCD-contiguous order, the order in which the
-    // feature kernel writes its rows, so that behind it a workgroup reads
-    // rows its own XCD wrote.
-    for (size_t base = xcd_contiguous(blockIdx.x, gridDim.x) * E; base < a.batch;
-         base += (size_t)gridDim.x * E) {
-        // Stage the feature rows in buffer 1 (rows are 568 bytes, 8-byte
-        // aligned): kRowThreads consecutive threads share an environment,
-        // each loading kRowPairs consecutive float pairs, every load of the
-        // pass issued before any LDS store so that the rows arrive in one
-        // round trip.  Rows past the batch end read as zero; inputs 142 to
-        // 159 are zero padding.
-        constexpr int kRowThreads = NW * 64 / E;                 // 8
-        constexpr int kRowPairs = 16 * kFeatureChunks / kRowThreads;  // 10
-        static_assert(kRowThreads * kRowPairs == 16 * kFeatureChunks, "row split");
-        const int se = tid / kRowThreads, sr = tid % kRowThreads;
-        f32x2 pairs[kRowPairs];
-        {
-            const size_t rows = a.batch - base < (size_t)E ? a.batch - base : (size_t)E;
-            const __amdgpu_buffer_rsrc_t frs =
-                make_rsrc(a.features + base * kFeatures, (unsigned)(rows * kFeatures * 4));
+    // One pass per workgroup, without a grid-stride loop (in one the compiler
+    // keeps addresses and literals in registers across it).  Rows past the
+    // batch end compute on zeros and store nothing.  Groups go to workgroups
+    // in XCD-contiguous order, the order in which the feature kernel writes
+    // its rows, so that behind it a workgroup reads rows its own XCD wrote.
+    const size_t base =
+        ((size_t)blockIdx.y * gridDim.x + xcd_contiguous(blockIdx.x, gridDim.x)) * E;
+    if (base >= a.batch) return;
+    // Stage the feature rows in buffer 1 (rows are 568 bytes, 8-byte
+    // aligned): kRowThreads consecutive threads share an environment,
+    // each loading kRowPairs consecutive float pairs, every load of the
+    // pass issued before any LDS store so that the rows arrive in one
+    // round trip.  Rows past the batch end read as zero; inputs 142 to
+    // 159 are zero padding.
+    constexpr int kRowThreads = NW * 64 / E < 16 ? NW * 64 / E : 16;  // 8 or 16
+    constexpr int kRowPairs = 16 * kFeatureChunks / kRowThreads;      // 10 or 5
+    static_assert(kRowThreads * kRowPairs == 16 * kFeatureChunks, "row split");
+    const int se = tid / kRowThreads, sr = tid % kRowThreads;
+    const bool stages = E * kRowThreads == NW * 64 || tid < E * kRowThreads;  // whole waves
+    const size_t rows = a.batch - base < (size_t)E ? a.batch - base : (size_t)E;
+    f32x2 pairs[kRowPairs];
+    if (stages) {
+        // Without a branch: a pair past the row's 142 reads past the end.
+        const __amdgpu_buffer_rsrc_t frs =
+            make_rsrc(a.features + base * kFeatures, (unsigned)(rows * kFeatures * 4));
 #pragma unroll
-            for (int it = 0; it < kRowPairs; ++it) {
-                const int k = 2 * (kRowPairs * sr + it);
-                pairs[it] = (f32x2){0.0f, 0.0f};
-                if (k < kFeatures)
-                    pairs[it] = __builtin_bit_cast(
-                        f32x2, __builtin_amdgcn_raw_buffer_load_b64(
-                                   frs, (unsigned)(se * kFeatures + k) * 4, 0, 0));
-            }
+        for (int it = 0; it < kRowPairs; ++it) {
+            const int k = 2 * (kRowPairs * sr + it);
+            const unsigned at = k < kFeatures ? (unsigned)(se * kFeatures + k) * 4 : kPastEnd;
+            pairs[it] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(frs, at, 0, 0));
         }
-        // Layer 0's first weight chunks and bias, requested with the
-        // features so that both round trips overlap.
-        LayerWeights<TPW> lw0;
-        layer_prefetch<kFeatureChunks, HT, TPW, NW>(wrs, a.w_off[0], a.b_off[0], w, lane, lw0);
-        // The hidden -> 30 layer gives wave w tile w % 2 of the G2 groups
-        // from group2 = G2 (w / 2) on: lane (g, j) then holds the (mean,
-        // log-std) pairs of actions 8 (w % 2) + 2 g and + 1 of environment j
-        // of each.  Their normal draws are loaded now and used after the
-        // three layers.
-        const int tile2 = w & 1, group2 = G2 * (w >> 1);
-        float drawn[G2][2];
+    }
+    // Layer 0's first weight chunks and bias, requested with the
+    // features so that both round trips overlap.
+    LayerWeights<TPW, D0> lw0;
+    layer_prefetch<kFeatureChunks, HT, TPW, NW>(wrs, a.w_off[0], a.b_off[0], w, lane, lw0);
+    LayerWeights<TPW, D1> lw1;
+    if constexpr (EARLY)
+        layer_prefetch<HC, HT, TPW, NW>(wrs, a.w_off[1], a.b_off[1], w, lane, lw1);
+    // The hidden -> 30 layer gives wave w tile w % 2 of the G2 groups
+    // from group2 = G2 (w / 2) on: lane (g, j) then holds the (mean,
+    // log-std) pairs of actions 8 (w % 2) + 2 g and + 1 of environment j
+    // of each.  Their normal draws are loaded now and used after the
+    // three layers.
+    const bool last = 2 * G >= NW || w < 2 * G;  // this wave has a pair
+    const int tile2 = w & 1, group2 = last ? G2 * (w >> 1) : 0;
+    float drawn[G2][2];
+    {
+        const __amdgpu_buffer_rsrc_t nrs =
+            make_rsrc(a.normals ? a.normals + base * kActions : nullptr,
+                      a.normals ? (unsigned)(rows * kActions * 4) : 0);
 #pragma unroll
-        for (int i = 0; i < G2; ++i) {
-            const size_t env2 = base + 16 * (group2 + i) + j;
+        for (int i = 0; i < G2; ++i)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int act = 8 * tile2 + 2 * g + h;
-                drawn[i][h] = 0.0f;
-                if (a.normals && act < kActions && env2 < a.batch)
-                    drawn[i][h] = a.normals[env2 * kActions + act];
+                const unsigned at =
+                    act < kActions ? (unsigned)((16 * (group2 + i) + j) * kActions + act) * 4 : kPastEnd;
+                drawn[i][h] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_raw_buffer_load_b32(nrs, at, 0, 0));
             }
-        }
-        // Infinite features go to the exact path (zero in the split operand);
-        // the row's largest other magnitude sets its scale.  The row's
-        // threads are kRowThreads consecutive lanes: both reduce by xor
-        // shuffles, and the first thread records them for layer 0.
-        {
-            unsigned m = 0;
-            int inf = 0;
+    }
+    // Infinite features go to the exact path (zero in the split operand);
+    // the row's largest other magnitude sets its scale.  The row's
+    // threads are kRowThreads consecutive lanes: both reduce by xor
+    // shuffles, and the first thread records them for layer 0.
+    if (stages) {
+        unsigned m = 0;
+        int inf = 0;
 #pragma unroll
-            for (int it = 0; it < kRowPairs; ++it) {
+        for (int it = 0; it < kRowPairs; ++it) {
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    if (infinite(pairs[it][h])) {
-                        pairs[it][h] = 0.0f;
-                        inf = 1;
-                    }
-                    const unsigned b = __float_as_uint(pairs[it][h]) & 0x7fffffffu;
-                    m = b > m ? b : m;
+            for (int h = 0; h < 2; ++h) {
+                if (infinite(pairs[it][h])) {
+                    pairs[it][h] = 0.0f;
+                    inf = 1;
                 }
-            }
-#pragma unroll
-            for (int d = 1; d < kRowThreads; d <<= 1) {
-                const unsigned o = (unsigned)__shfl_xor((int)m, d);
-                m = o > m ? o : m;
-                inf |= __shfl_xor(inf, d);
-            }
-            if (sr == 0) {
-                row_max[se] = m;
-                special[se] = inf;
-            }
-            const int t = row_exponent(m);
-            unsigned char *xs = reinterpret_cast<unsigned char *>(buf[1]);
-#pragma unroll
-            for (int it = 0; it < kRowPairs; ++it) {
-                const int k = 2 * (kRowPairs * sr + it);
-                const f32x2 x = {__builtin_amdgcn_ldexpf(pairs[it][0], t),
-                                 __builtin_amdgcn_ldexpf(pairs[it][1], t)};
-                unsigned pc[kPieces];
-                split_pair(x, pc[0], pc[1]);
-                unsigned char *at = xs + se * RS + (k >> 5) * kPieces * kChunkBytes + 2 * (k & 31);
-#pragma unroll
-                for (int p = 0; p < kPieces; ++p)
-                    *reinterpret_cast<unsigned *>(at + kChunkBytes * p) = pc[p];
+                const unsigned b = __float_as_uint(pairs[it][h]) & 0x7fffffffu;
+                m = b > m ? b : m;
             }
         }
-        __syncthreads();
-
-        // Each layer's first weight chunks are requested before the
-        // barrier that ends the previous layer.
-        LayerWeights<TPW> lw1;
-        {
-            f32x4 h[TPW][G];
-            int shift[G];
 #pragma unroll
-            for (int q = 0; q < G; ++q) shift[q] = row_exponent(row_max[16 * q + j]);
-            layer_tiles<kFeatureChunks, HT, TPW, G, RS, NW>(wrs, a.w_off[0], buf[1], lw0, shift, h,
-                                                            w, lane);
-            // The exact products of the infinite features, added by the
-            // lanes of their environment (rare).
-            bool mine[G];
-            bool any = false;
+        for (int d = 1; d < kRowThreads; d <<= 1) {
+            const unsigned o = (unsigned)__shfl_xor((int)m, d);
+            m = o > m ? o : m;
+            inf |= __shfl_xor(inf, d);
+        }
+        if (sr == 0) {
+            row_max[se] = m;
+            special[se] = inf;
+        }
+        const int t = row_exponent(m);
+        unsigned char *xs = reinterpret_cast<unsigned char *>(buf[1]);
+#pragma unroll
+        for (int it = 0; it < kRowPairs; ++it) {
+            const int k = 2 * (kRowPairs * sr + it);
+            const f32x2 x = {__builtin_amdgcn_ldexpf(pairs[it][0], t),
+                             __builtin_amdgcn_ldexpf(pairs[it][1], t)};
+            unsigned pc[kPieces];
+            split_pair(x, pc[0], pc[1]);
+            unsigned char *at = xs + se * RS + (k >> 5) * kPieces * kChunkBytes + 2 * (k & 31);
+#pragma unroll
+            for (int p = 0; p < kPieces; ++p)
+                *reinterpret_cast<unsigned *>(at + kChunkBytes * p) = pc[p];
+        }
+    }
+    __syncthreads();
+
+    // Each layer's first weight chunks are requested before the
+    // barrier that ends the previous layer.
+    {
+        f32x4 h[TPW][G];
+        int shift[G];
+#pragma unroll
+        for (int q = 0; q < G; ++q) shift[q] = row_exponent(row_max[16 * q + j]);
+        layer_tiles<kFeatureChunks, HT, TPW, G, RS, NW>(wrs, a.w_off[0], buf[1], lw0, shift, h,
+                                                        w, lane);
+        // The exact products of the infinite features, added by the
+        // lanes of their environment (rare).
+        bool mine[G];
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            mine[q] = special[16 * q + j] != 0;
+            any |= mine[q];
+        }
+        if (__builtin_amdgcn_ballot_w64(any)) {
+            const float *w0 = reinterpret_cast<const float *>(
+                static_cast<const unsigned char *>(a.packed) + a.w0_off);
 #pragma unroll
             for (int q = 0; q < G; ++q) {
-                mine[q] = special[16 * q + j] != 0;
-                any |= mine[q];
-            }
-            if (__builtin_amdgcn_ballot_w64(any)) {
-                const float *w0 = reinterpret_cast<const float *>(
-                    static_cast<const unsigned char *>(a.packed) + a.w0_off);
+                if (!mine[q]) continue;
+                const float *row = a.features + (base + 16 * q + j) * kFeatures;
+                for (int k = 0; k < kFeatures; ++k) {
+                    const float x = row[k];
+                    if (!infinite(x)) continue;
 #pragma unroll
-                for (int q = 0; q < G; ++q) {
-                    if (!mine[q]) continue;
-                    const float *row = a.features + (base + 16 * q + j) * kFeatures;
-                    for (int k = 0; k < kFeatures; ++k) {
-                        const float x = row[k];
-                        if (!infinite(x)) continue;
+                    for (int jj = 0; jj < TPW; ++jj)
 #pragma unroll
-                        for (int jj = 0; jj < TPW; ++jj)
-#pragma unroll
-                            for (int v = 0; v < 4; ++v) {
-                                const int n = 16 * (w + NW * jj) + 4 * g + v;
-                                if (n < a.hidden) h[jj][q][v] += x * w0[(size_t)n * kFeatures + k];
-                            }
-                    }
+                        for (int v = 0; v < 4; ++v) {
+                            const int n = 16 * (w + NW * jj) + 4 * g + v;
+                            if (n < a.hidden) h[jj][q][v] += x * w0[(size_t)n * kFeatures + k];
+                        }
                 }
             }
+        }
+        if constexpr (!EARLY)
             layer_prefetch<HC, HT, TPW, NW>(wrs, a.w_off[1], a.b_off[1], w, lane, lw1);
-            store_tiles<TPW, G, 2 * HC, RS, NW>(reinterpret_cast<unsigned char *>(buf[0]), h, w,
-                                                lane);
-        }
-        __syncthreads();
-        LayerWeights<1> lw2;
-        {
-            f32x4 h[TPW][G];
-            int shift[G] = {};
-            layer_tiles<HC, HT, TPW, G, RS, NW>(wrs, a.w_off[1], buf[0], lw1, shift, h, w, lane);
-            layer_prefetch<HC, 2, 1, NW>(wrs, a.w_off[2], a.b_off[2], tile2, lane, lw2);
-            store_tiles<TPW, G, 2 * HC, RS, NW>(reinterpret_cast<unsigned char *>(buf[1]), h, w,
-                                                lane);
-        }
-        __syncthreads();
-        {
-            f32x4 r[1][G2];
-            const int shift[G2] = {};
-            layer_tiles<HC, 2, 1, G2, RS, NW>(wrs, a.w_off[2], buf[1] + group2 * 16 * (RS / 16), lw2,
-                                          shift, r, tile2, lane);
-            // training.c:310-327 on this lane's two actions of each group
-            // (the last lane group of tile 1 holds one action and the
-            // padding).
+        store_tiles<TPW, G, 2 * HC, RS, NW>(reinterpret_cast<unsigned char *>(buf[0]), h, w,
+                                            lane);
+    }
+    __syncthreads();
+    LayerWeights<1, D2> lw2;
+    {
+        f32x4 h[TPW][G];
+        int shift[G] = {};
+        layer_tiles<HC, HT, TPW, G, RS, NW>(wrs, a.w_off[1], buf[0], lw1, shift, h, w, lane);
+        if (last) layer_prefetch<HC, 2, 1, NW>(wrs, a.w_off[2], a.b_off[2], tile2, lane, lw2);
+        store_tiles<TPW, G, 2 * HC, RS, NW>(reinterpret_cast<unsigned char *>(buf[1]), h, w,
+                                            lane);
+    }
+    __syncthreads();
+    if (last) {
+        f32x4 r[1][G2];
+        const int shift[G2] = {};
+        layer_tiles<HC, 2, 1, G2, RS, NW>(wrs, a.w_off[2], buf[1] + group2 * 16 * (RS / 16), lw2,
+                                      shift, r, tile2, lane);
+        // training.c:310-327 on this lane's two actions of each group
+        // (the last lane group of tile 1 holds one action and the
+        // padding).
 #pragma unroll
-            for (int i = 0; i < G2; ++i) {
-                const size_t env2 = base + 16 * (group2 + i) + j;
-                const bool live = env2 < a.batch;
+        for (int i = 0; i < G2; ++i) {
+            const size_t env2 = base + 16 * (group2 + i) + j;
+            const bool live = env2 < a.batch;
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int act_i = 8 * tile2 + 2 * g + h;
-                    if (act_i >= kActions) continue;
-                    const float mean_raw = r[0][i][2 * h], ls_raw = r[0][i][2 * h + 1];
-                    if (a.raw && live) {
-                        a.raw[env2 * kRaw + act_i] = mean_raw;
-                        a.raw[env2 * kRaw + kActions + act_i] = ls_raw;
-                    }
-                    const float log_std = clampf(finite_or_zero(ls_raw), -3.5f, -1.6f);
-                    const float sd = expf(log_std);
-                    const float eps =
-                        a.normals ? drawn[i][h] * (act_i == 14 ? 0.15f : 1.0f) : 0.0f;
-                    const float z = clampf(finite_or_zero(mean_raw) + sd * eps, -8.0f, 8.0f);
-                    const float act = tanhf(z);
-                    if (live) a.actions[env2 * kActions + act_i] = act;
-                    const float gaussian = -0.5f * eps * eps - log_std - 0.5f * logf(2.0f * kPi);
-                    term_s[16 * (group2 + i) + j][act_i] =
-                        gaussian - logf(1.0f - act * act + 1.0e-6f);
+            for (int h = 0; h < 2; ++h) {
+                const int act_i = 8 * tile2 + 2 * g + h;
+                if (act_i >= kActions) continue;
+                const float mean_raw = r[0][i][2 * h], ls_raw = r[0][i][2 * h + 1];
+                if (a.raw && live) {
+                    a.raw[env2 * kRaw + act_i] = mean_raw;
+                    a.raw[env2 * kRaw + kActions + act_i] = ls_raw;
                 }
+                const float log_std = clampf(finite_or_zero(ls_raw), -3.5f, -1.6f);
+                const float sd = expf(log_std);
+                const float eps =
+                    a.normals ? drawn[i][h] * (act_i == 14 ? 0.15f : 1.0f) : 0.0f;
+                const float z = clampf(finite_or_zero(mean_raw) + sd * eps, -8.0f, 8.0f);
+                const float act = tanhf(z);
+                if (live) a.actions[env2 * kActions + act_i] = act;
+                const float gaussian = -0.5f * eps * eps - log_std - 0.5f * logf(2.0f * kPi);
+                term_s[16 * (group2 + i) + j][act_i] =
+                    gaussian - logf(1.0f - act * act + 1.0e-6f);
             }
         }
-        __syncthreads();
-        if (a.log_prob && tid < E && base + tid < a.batch) {
-            float lp = 0.0f;  // summed in action order, as the reference does
-            if (a.normals)
-                for (int i = 0; i < kActions; ++i) lp += term_s[tid][i];
-            a.log_prob[base + tid] = lp;
-        }
+    }
+    __syncthreads();
+    if (a.log_prob && tid < E && base + tid < a.batch) {
+        float lp = 0.0f;  // summed in action order, as the reference does
+        if (a.normals)
+            for (int i = 0; i < kActions; ++i) lp += term_s[tid][i];
+        a.log_prob[base + tid] = lp;
     }
 }
 
+constexpr size_t kGridX = 65536;  // workgroups per row of the grid
+
+template <int HT, int G, int NW, bool EARLY>
+void launch_shape(const ActArgs &a, hipStream_t s) {
+    const size_t want = (a.batch + 16 * G - 1) / (16 * G);
+    const dim3 blocks((unsigned)(want < kGridX ? want : kGridX),
+                      (unsigned)((want + kGridX - 1) / kGridX));
+    sac_actor_kernel<HT, G, NW, EARLY><<<blocks, NW * 64, 0, s>>>(a);
+}
+
+// Shape by batch.  One group of 16 rows per workgroup while that is at most
+// one workgroup per CU (4,096 rows), two up to 8,192, above that full
+// workgroups, whose weight reads (every workgroup reads all weights) and
+// matrix-core steps are shared by the most rows.  Up to 4 hidden tiles the
+// full workgroup is two groups itself.  With 5 to 8 hidden tiles two groups
+// also serve batches over 16,384 rows, where full workgroups, one per CU,
+// need a second round and three of these fit a CU.  Measured on one box (us;
+// one group / two groups / full; all were 8.0-14.2 up to 8,192 rows in the
+// full shape with its loop over passes):
+//   hidden 64:  256 rows 4.4 / 5.1 / 5.0, 4,096 4.6 / 5.2 / 5.1, 8,192 5.4 / 5.3 / 5.2
+//   hidden 128: 256 rows 4.8 / 6.3 / 8.1, 4,096 5.2 / 6.4 / 8.4, 8,192 7.1 / 6.5 / 8.4,
+//               16,384 12.0 / 9.3 / 9.0, 16,500 14.4 / 12.8 / 15.7, 65,536 41.4 / 30.1 / 32.2
+//   hidden 256: 256 rows 7.7 / 9.4 / 12.3, 4,096 8.4 / 9.5 / 12.6, 8,192 14.8 / 9.7 / 12.7,
+//               16,384 28.9 / 19.1 / 14.3, 40,000 68.2 / 44.5 / 38.6
+constexpr size_t kOneGroupMax = 4096, kTwoGroupMax = 8192, kFullMax = 16384;
+
 template <int HT>
 void launch_act(const ActArgs &a, hipStream_t s) {
-    constexpr int NW = Shape<HT>::waves, G = Shape<HT>::groups;
-    const size_t want = (a.batch + 16 * G - 1) / (16 * G);
-    const unsigned blocks = want > 65536 ? 65536u : (unsigned)want;
-    sac_actor_kernel<HT, G, NW><<<blocks, NW * 64, 0, s>>>(a);
+    constexpr int small = SmallShape<HT>::waves;
+    if (a.batch <= kOneGroupMax) return launch_shape<HT, 1, small, true>(a, s);
+    if constexpr (HT > 4) {
+        if (a.batch <= kTwoGroupMax || (HT <= 8 && a.batch > kFullMax))
+            return launch_shape<HT, 2, small, true>(a, s);
+    }
+    launch_shape<HT, Shape<HT>::groups, Shape<HT>::waves, false>(a, s);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
