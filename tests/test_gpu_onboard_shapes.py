@@ -1,0 +1,102 @@
+"""The onboard and actor-input entries' workgroup shapes (csrc/onboard.hip): a
+row's outputs do not depend on the batch it comes in.  Every batch size around
+a shape's bounds (a group of 16, one, two and four groups, equal shares, the
+two-stream form) against the rows of a batch in another shape, bit for bit,
+and each shape on the generator's non-finite and signed-zero rows."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from tests.test_gpu_onboard import compare, in_window, run_onboard
+from turbinator_c_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+SIZES = (1, 15, 16, 17, 31, 33, 1000, 8191, 8192, 8193, 16383, 16384, 16385, 20011, 32767, 32768)
+
+
+@pytest.fixture(scope="module")
+def tiled(torch_cuda):
+    """4,096 distinct environments (ordinary and special), tiled on the device."""
+    torch = torch_cuda
+    parts = [synth.make_batch(2048, seed=71, threads=16),
+             synth.make_batch(1024, seed=72, variant=synth.SPECIAL, threads=16),
+             synth.make_batch(1024, seed=73, variant=synth.EDGE_QUARTERS, threads=16)]
+    obs = in_window(np.concatenate([p.obs for p in parts]))
+    mission = np.concatenate([p.mission for p in parts])
+    order = np.random.default_rng(7).permutation(4096)
+    rows = torch.arange(32800, device="cuda") % 4096
+    return (torch.from_numpy(obs[order]).cuda()[rows].contiguous(),
+            torch.from_numpy(mission[order]).cuda()[rows].contiguous())
+
+
+@pytest.mark.parametrize("diag", [False, True])
+def test_onboard_rows_do_not_depend_on_the_batch(torch_cuda, hip, tiled, diag):
+    torch = torch_cuda
+    obs, mission = tiled
+    s = torch.cuda.current_stream()
+
+    def run(n):
+        out = [torch.full((n + 1, w), 7.0, device="cuda") for w in (24, 15, 5)]
+        assert hip.onboard_tactical_prior_device(obs, mission, out[0], out[1],
+                                                 out[2] if diag else None, n, s) == 1
+        torch.cuda.synchronize()
+        return out
+
+    want = run(4096)
+    for n in SIZES:
+        print(f"[gpu-case] onboard {n} diag {diag}", flush=True)
+        for got, full, k in zip(run(n), want, (0, 1, 2)):
+            if k == 2 and not diag:
+                continue
+            assert bool((got[n] == 7.0).all()), n  # nothing past the batch
+            rows = torch.arange(n, device="cuda") % 4096
+            same = got[:n].view(torch.int32) == full[rows].view(torch.int32)
+            assert bool(same.all()), (n, k, torch.nonzero(~same)[:5].tolist())
+
+
+@pytest.mark.parametrize("n", [1, 47, 1024, 10000, 17000])
+def test_special_rows_in_every_shape(torch_cuda, hip, n):
+    b = synth.make_batch(n, seed=500 + n, variant=synth.SPECIAL, threads=16)
+    # 3e38 overflows inside the reference's formulas, where the last bit of an
+    # angle decides an infinity's sign
+    obs, mission = in_window(b.obs), b.mission.copy()
+    obs[np.abs(obs) == np.float32(3e38)] = np.float32(7.5)
+    mission[np.abs(mission) == np.float32(3e38)] = np.float32(0.25)
+    print(f"[gpu-case] onboard special {n}", flush=True)
+    compare(run_onboard(torch_cuda, hip, obs, mission), oracle.onboard(obs, mission),
+            f"special {n}")
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 3071, 3072, 3073])
+def test_actor_rows_do_not_depend_on_the_batch(torch_cuda, hip, tiled, n):
+    torch = torch_cuda
+    obs, mission = tiled
+    print(f"[gpu-case] actor inputs {n}", flush=True)
+    g = torch.Generator("cuda").manual_seed(5)
+    cameras = torch.randint(0, 256, (4096, 16384), dtype=torch.uint8, device="cuda", generator=g)
+    s = torch.cuda.current_stream()
+    widths = {"proprio": 91, "mission_vec": 49, "tactical": 24, "prior": 15, "lidar": 12288,
+              "luma": 16384}
+
+    def run(k, lidar=True, luma=True):
+        out = {w: torch.full((k + 1, v), 7.0, device="cuda") for w, v in widths.items()}
+        assert hip.actor_inputs_device(
+            obs, mission, cameras, out["proprio"], out["mission_vec"], out["tactical"],
+            out["prior"], out["lidar"] if lidar else None, out["luma"] if luma else None, k,
+            s) == 1
+        torch.cuda.synchronize()
+        return out
+
+    want = run(4000)
+    for planes in ((True, True), (True, False), (False, True), (False, False)):
+        got = run(n, *planes)
+        for w in widths:
+            if (w == "lidar" and not planes[0]) or (w == "luma" and not planes[1]):
+                assert bool((got[w] == 7.0).all())
+                continue
+            assert bool((got[w][n] == 7.0).all()), (w, planes)
+            same = got[w][:n].view(torch.int32) == want[w][:n].view(torch.int32)
+            assert bool(same.all()), (w, planes, torch.nonzero(~same)[:5].tolist())

@@ -27,21 +27,21 @@
 //     (onboard_features.cuh:208-244), so unless the caller asks for the
 //     scan's diagnostics each environment gets only the part its mission
 //     uses, and the next environment's ranges are requested only as far as
-//     it needs them.  In the onboard entry the environments whose mission
-//     uses the scan are shared out over the 16 waves of a CU from a pool in
-//     LDS, so the waves that would have drawn several slalom missions do
-//     not set the kernel's time; the actor entry's scan, which also writes
-//     the LiDAR channels of every environment, keeps a static share;
+//     it needs them.  The environments whose mission uses the scan are shared
+//     out over a workgroup's waves from a pool in LDS, so the waves that
+//     would have drawn several slalom missions do not set the kernel's time;
+//     the actor entry's scan for large batches, which also writes the LiDAR
+//     channels of every environment, keeps a static share;
 //   * the tactical features and the controller (mission decode, targets,
-//     landing / standard / inversion / BWB laws, cannon) run in a second
-//     kernel from the parked scan results, both on one quad of lanes per
-//     environment (lane a evaluates arm a and a quarter of the independent
-//     transcendental calls), except where the workgroups of 64 environments
-//     fill the chip (the onboard entry from 8,192 environments): there one
-//     kernel does both, each workgroup scanning its own environments into
-//     LDS before their controller runs, which saves the second launch and
-//     the parked results' round trip.  The angles
-//     that reach its angle wraps use a correctly rounded atan2: exact angles
+//     landing / standard / inversion / BWB laws, cannon) run on one quad of
+//     lanes per environment (lane a evaluates arm a and a quarter of the
+//     independent transcendental calls), in the same workgroup as their
+//     scan: a launch of their own cost its start, a second staging of the
+//     inputs and the scan results' round trip.  Small batches give the
+//     flight controller, the rest of the controller and the scan their own
+//     waves, so that the chain that sets the time, the flight controller's,
+//     runs beside the scan up to the point that needs it.  The angles that
+//     reach its angle wraps use a correctly rounded atan2: exact angles
 //     (from equal or zero components) reach a wrap's discontinuity, where
 //     one ulp flips the wrapped error's sign.
 //
@@ -58,7 +58,6 @@
 
 #include <atomic>
 #include <mutex>
-#include <type_traits>
 
 #include "turbinator/training/hip_features.h"
 #include "onboard_math.h"
@@ -682,9 +681,9 @@ __device__ __forceinline__ ChainInputs chain_inputs(const float *obs, const floa
     return in;
 }
 
-// Whether every value the active lanes read is finite and below
-// onboard_math::kTameMax: the sum of their squares is below its square.
-__device__ __forceinline__ bool tame_inputs(const ChainInputs &in) {
+// Whether a value that the lane reads is infinite, NaN or not below
+// onboard_math::kTameMax: unless the sum of their squares is below its square.
+__device__ __forceinline__ bool wild_inputs(const ChainInputs &in) {
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < 13; ++i) s = __builtin_fmaf(in.head[i], in.head[i], s);
@@ -694,8 +693,25 @@ __device__ __forceinline__ bool tame_inputs(const ChainInputs &in) {
     for (int k = 0; k < 6; ++k) s = __builtin_fmaf(in.tail[k], in.tail[k], s);
 #pragma unroll
     for (int i = 0; i < 10; ++i) s = __builtin_fmaf(in.m[i], in.m[i], s);
-    return __builtin_amdgcn_ballot_w64(
-               !(s < onboard_math::kTameMax * onboard_math::kTameMax)) == 0;
+    return !(s < onboard_math::kTameMax * onboard_math::kTameMax);
+}
+
+// Sine and cosine of atan2(y, x) from the components; a wild lane's are those
+// of the rounded angle, as the reference forms them: what they multiply may
+// be infinite or near the largest float, and then it matters that the sine of
+// a float near pi is about 1e-7 and not the exact value.
+template <bool TAME>
+__device__ __forceinline__ onboard_math::Direction ob_direction(float y, float x, bool wild) {
+    onboard_math::Direction d = onboard_math::direction(y, x);
+    if constexpr (!TAME) {
+        if (__builtin_amdgcn_ballot_w64(wild)) {
+            float s, c;
+            sincosf(ob_atan2<false>(y, x), &s, &c);
+            d.s = wild ? s : d.s;
+            d.c = wild ? c : d.c;
+        }
+    }
+    return d;
 }
 
 // The inputs as the controller reads them (onboard_features.cuh:12-22, 95-99).
@@ -720,7 +736,8 @@ __device__ __forceinline__ void controller_inputs(ChainInputs &in) {
 // its order from the broadcasts.  Lane a returns features 6a .. 6a + 5 in t,
 // mapped as the reference maps them (NaN -> 0, +-inf -> +-1).
 template <bool TAME>
-__device__ __forceinline__ void tactical_quad(const ChainInputs &in, int a, float (&t)[6]) {
+__device__ __forceinline__ void tactical_quad(const ChainInputs &in, bool wild, int a,
+                                              float (&t)[6]) {
     const float pi = kPi;
     const float *o = in.head, *m = in.m;
     const float o44 = in.tail[2], o45 = in.tail[3], o46 = in.tail[4], o47 = in.tail[5];
@@ -758,23 +775,7 @@ __device__ __forceinline__ void tactical_quad(const ChainInputs &in, int a, floa
     // bearing atan2(ry, rx) on the others, from their components; the angles
     // themselves are used nowhere else.
     const float ty_a = a == 0 ? bx_y : ry, tx_a = a == 0 ? bx_x : rx;
-    onboard_math::Direction at_a = onboard_math::direction(ty_a, tx_a);
-    if constexpr (!TAME) {
-        // Where a value that they multiply or come from is not finite, they
-        // are those of the rounded angle, as the reference forms them: an
-        // infinity times the sine of a float near pi is an infinity, times
-        // an exact zero it would be NaN.  (The sum of magnitudes may
-        // overflow; such a row takes that form too.)
-        const float reach = (fabsf(ty_a) + fabsf(tx_a)) + (fabsf(o[3]) + fabsf(o[4])) +
-                            (fabsf(bz_x) + fabsf(bz_y));
-        const bool odd = !(reach < __builtin_huge_valf());
-        if (__builtin_amdgcn_ballot_w64(odd)) {
-            float s, c;
-            sincosf(atan2f(ty_a, tx_a), &s, &c);
-            at_a.s = odd ? s : at_a.s;
-            at_a.c = odd ? c : at_a.c;
-        }
-    }
+    const onboard_math::Direction at_a = ob_direction<TAME>(ty_a, tx_a, wild);
     const float cy = quad_lane<0>(at_a.c), sy = quad_lane<0>(at_a.s);
     const float cb = quad_lane<1>(at_a.c), sb = quad_lane<1>(at_a.s);
     v[8] = cy * bz_y - sy * bz_x;
@@ -886,9 +887,11 @@ struct ArmOutputs {
 // value is the one the per-environment code forms.  The cannon and the BWB
 // law share nothing with this chain but its inputs: gunnery_quad forms them
 // on the waves of the tactical features, which are done far earlier.
-template <bool TAME>
-__device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, const MissionFlags &f,
-                                                  const ScanResult &scan, int a) {
+// `fetch` returns the scan result; everything that does not depend on it is
+// formed before it is called.
+template <bool TAME, class Fetch>
+__device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, bool wild,
+                                                  const MissionFlags &f, int a, Fetch fetch) {
     using onboard_math::quotient;
     const float pi = kPi;
     const float max_installed = 294.2f * 0.85f;
@@ -911,7 +914,7 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, const M
     const float spool = ob_clamp<TAME>(in.arm[0], 0.0f, 1.0f);
     const float thrust = max_installed * (idle_frac + (1.0f - idle_frac) * spool);
     const float outer = ob_atan2<TAME>(in.arm[1], in.arm[2]);
-    const onboard_math::Direction o_sc = onboard_math::direction(in.arm[1], in.arm[2]);
+    const onboard_math::Direction o_sc = ob_direction<TAME>(in.arm[1], in.arm[2], wild);
     const float c_inner = onboard_math::cos_float<TAME>(in.arm[3]);
     const Quad4 fz = quad_all(thrust * o_sc.c * c_inner), ft = quad_all(thrust * o_sc.s * c_inner);
     float total_fz = 0.0f, jammed_yaw_ft = 0.0f;
@@ -975,14 +978,49 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, const M
     const float errx = ex - px, erry = ey - py;
     const float horiz_dist = ob_hypot<TAME>(errx, erry);
 
-    // Sine and cosine of yaw and of the closest return's bearing from their
-    // components (a rotation's rows; a range inside the window), and the sine
-    // of the slalom hill phase.
-    const onboard_math::Direction sc = onboard_math::direction(a == 0 ? r10 : scan.min_r_dy,
-                                                               a == 0 ? r00 : scan.min_r_dx);
-    const float cyaw = quad_lane<0>(sc.c), syaw = quad_lane<0>(sc.s);
+    const float tilt = acosf(ct);
+    const bool need_headroom = (int)f.inversion | (int)f.arena | (int)(ct < 0.88f);
+    const bool urgent_climb = (int)f.arena & ((int)(pz < 8.5f) | (int)(vz < -1.2f)) &
+                              (int)(ct > 0.58f);
+    const float room = ob_clamp<TAME>(3.95f - 0.90f * omega_norm - 1.30f * tilt, 2.55f, 3.95f);
+    const float calm_coll = need_headroom ? room : 3.95f;
+    const float max_coll = urgent_climb ? 3.95f : calm_coll;
+    const float tilt_scale_h =
+        ob_clamp<TAME>(1.0f - 1.5f * fmaxf(tilt - 0.15f, 0.0f), 0.0f, 1.0f);
+    const float calm_scale = need_headroom ? tilt_scale_h : 1.0f;
+    const float horiz_scale = urgent_climb ? 0.0f : calm_scale;
+    const float cw_x = body_z_y, cw_y = -body_z_x;
+    const float tt_x = 2.0f * (-uz * cw_y), tt_y = 2.0f * (uz * cw_x);
+    const float tt_z = 2.0f * (ux * cw_y - uy * cw_x);
+    const float te_x = cw_x + qw * tt_x + (uy * tt_z - uz * tt_y);
+    const float te_y = cw_y + qw * tt_y + (uz * tt_x - ux * tt_z);
+    const float te_z = qw * tt_z + (ux * tt_y - uy * tt_x);
+    const float te_norm = ob_norm3<TAME>(te_x, te_y, te_z);
+    const float per_te = quotient<TAME>(tilt, fmaxf(te_norm, 1.0e-5f));
+    const float tilt_scale = te_norm > 1.0e-5f ? per_te : 0.0f;
+    const float e_rx = te_x * tilt_scale, e_ry = te_y * tilt_scale;
+
+    const bool inv_hold_yaw = ((int)f.inversion | (int)f.arena) &
+                              ((int)(pz < 6.0f) | (int)(vz < -0.5f) | (int)(ct < 0.88f));
+    const bool opp_bearing_valid = (int)f.arena & (int)(fabsf(m[1]) + fabsf(m[2]) > 0.1f);
+    const float target_bearing = opp_bearing_valid ? opp_bearing : raw_bearing;
+    const bool face = (int)f.arena & (int)(horiz_dist > 1.0f) & (int)!inv_hold_yaw;
+    const float held_yaw = inv_hold_yaw ? yaw : 0.0f;
+    const float facing_yaw = target_bearing - cannon_az_ctr;
+    const float desired_yaw = face ? facing_yaw : held_yaw;
+    const float yaw_err = ob_wrap<TAME>(desired_yaw, yaw);
+
+    const float horiz_speed = ob_hypot<TAME>(vx, vy);
     const float hill = ob_clamp<TAME>(div_const(px - 6.0f, 30.0f), 0.0f, 1.0f);
     const float hill_sin = onboard_math::sin_half_turn(hill);
+
+    const ScanResult scan = fetch();
+
+    // Sine and cosine of yaw and of the closest return's bearing from their
+    // components (a rotation's rows; a range inside the window).
+    const onboard_math::Direction sc = ob_direction<TAME>(
+        a == 0 ? r10 : scan.min_r_dy, a == 0 ? r00 : scan.min_r_dx, wild);
+    const float cyaw = quad_lane<0>(sc.c), syaw = quad_lane<0>(sc.s);
 
     const bool avoid = (int)f.dodge & (int)(scan.min_r < 7.5f);
     const float away_x = -quad_lane<1>(sc.s) * 2.2f, away_y = quad_lane<1>(sc.c) * 2.2f;
@@ -1011,7 +1049,6 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, const M
         (int)f.slalom & (int)(nearest_dx < 10.2f) & (int)(horiz_dist > 3.0f);
 
     const float pad_z = fmaxf(ez, 0.60f), above_pad = pz - pad_z;
-    const float horiz_speed = ob_hypot<TAME>(vx, vy);
     const float transit_cap = heavy_cargo ? 2.65f : 3.4f;
     const float near_cap = heavy_cargo ? 1.25f : 1.6f;
     const float low_cap = above_pad < 1.2f ? 0.55f : near_cap;
@@ -1078,19 +1115,8 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, const M
     const float des_ay = landing_like ? des_ay_land : des_ay_std;
     const float des_az = landing_like ? des_az_land : des_az_std;
 
-    const float tilt = acosf(ct);
-    const bool need_headroom = (int)f.inversion | (int)f.arena | (int)(ct < 0.88f);
-    const bool urgent_climb = (int)f.arena & ((int)(pz < 8.5f) | (int)(vz < -1.2f)) &
-                              (int)(ct > 0.58f);
-    const float room = ob_clamp<TAME>(3.95f - 0.90f * omega_norm - 1.30f * tilt, 2.55f, 3.95f);
-    const float calm_coll = need_headroom ? room : 3.95f;
-    const float max_coll = urgent_climb ? 3.95f : calm_coll;
     const float fz_des = ob_clamp<TAME>(quotient<TAME>(weight + mass * des_az, fmaxf(ct, 0.45f)),
                                         0.10f * weight, max_coll * max_installed);
-    const float tilt_scale_h =
-        ob_clamp<TAME>(1.0f - 1.5f * fmaxf(tilt - 0.15f, 0.0f), 0.0f, 1.0f);
-    const float calm_scale = need_headroom ? tilt_scale_h : 1.0f;
-    const float horiz_scale = urgent_climb ? 0.0f : calm_scale;
     const float tilt_comp = f.turbine_out ? 0.65f : 0.0f;
     const float damp_v = active_slalom ? 0.8f : 0.4f;
     const float fx_world =
@@ -1102,27 +1128,6 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, const M
     const float max_fh = active_slalom ? 105.0f : lat_fh;
     const float fx_body = ob_clamp<TAME>(cyaw * fx_world + syaw * fy_world, -max_fh, max_fh);
     const float fy_body = ob_clamp<TAME>(-syaw * fx_world + cyaw * fy_world, -max_fh, max_fh);
-
-    const float cw_x = body_z_y, cw_y = -body_z_x;
-    const float tt_x = 2.0f * (-uz * cw_y), tt_y = 2.0f * (uz * cw_x);
-    const float tt_z = 2.0f * (ux * cw_y - uy * cw_x);
-    const float te_x = cw_x + qw * tt_x + (uy * tt_z - uz * tt_y);
-    const float te_y = cw_y + qw * tt_y + (uz * tt_x - ux * tt_z);
-    const float te_z = qw * tt_z + (ux * tt_y - uy * tt_x);
-    const float te_norm = ob_norm3<TAME>(te_x, te_y, te_z);
-    const float per_te = quotient<TAME>(tilt, fmaxf(te_norm, 1.0e-5f));
-    const float tilt_scale = te_norm > 1.0e-5f ? per_te : 0.0f;
-    const float e_rx = te_x * tilt_scale, e_ry = te_y * tilt_scale;
-
-    const bool inv_hold_yaw = ((int)f.inversion | (int)f.arena) &
-                              ((int)(pz < 6.0f) | (int)(vz < -0.5f) | (int)(ct < 0.88f));
-    const bool opp_bearing_valid = (int)f.arena & (int)(fabsf(m[1]) + fabsf(m[2]) > 0.1f);
-    const float target_bearing = opp_bearing_valid ? opp_bearing : raw_bearing;
-    const bool face = (int)f.arena & (int)(horiz_dist > 1.0f) & (int)!inv_hold_yaw;
-    const float held_yaw = inv_hold_yaw ? yaw : 0.0f;
-    const float facing_yaw = target_bearing - cannon_az_ctr;
-    const float desired_yaw = face ? facing_yaw : held_yaw;
-    const float yaw_err = ob_wrap<TAME>(desired_yaw, yaw);
 
     const float parasite_scale = f.turbine_out ? 0.35f : 1.0f;
     const float tau_x_par = -0.1625f * fy_body * parasite_scale;
@@ -1207,8 +1212,8 @@ struct GunOutputs {
 };
 
 template <bool TAME>
-__device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, const MissionFlags &f,
-                                                   int a) {
+__device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool wild,
+                                                   const MissionFlags &f, int a) {
     using onboard_math::quotient;
     const float pi = kPi;
     const float gravity = 9.80665f;
@@ -1331,7 +1336,7 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, const 
     const float throttle = (a & 1) ? u1 : u0;
     const float pitch_up = asinf(ob_clamp<TAME>(r20, -1.0f, 1.0f));
     const float climb_err = climb_des - vz;
-    const onboard_math::Direction bank = onboard_math::direction(r21, r22);
+    const onboard_math::Direction bank = ob_direction<TAME>(r21, r22, wild);
     const float cos_bank = bank.c, sin_bank = bank.s;
     float desired_pitch = ob_clamp<TAME>(0.062831853f + 0.75f * gamma_des + 0.035f * climb_err +
                                              0.09f * (1.0f - fmaxf(cos_bank, 0.5f)),
@@ -1440,21 +1445,19 @@ __device__ __forceinline__ void park_scan(float *park, const ScanResult &s) {
     park[6] = __int_as_float(s.cluster_count);
 }
 
-// Phase 1 of the actor entry, and of the onboard entry below 2,560
-// environments.  Each wave scans one environment at a time;
+// Phase 1 of the actor entry's two-stream form.  Each wave scans one
+// environment at a time;
 // workgroups are persistent (the ray table is loaded into LDS once per
 // workgroup, the only barrier).  Wave g of the grid takes environments g,
 // g + W, g + 2W, ... (W waves in the grid).  Their scan frames (attitude
 // rows, py) and scan needs (scan_need) are formed up front, lane j for the
 // wave's j-th environment, and each environment's frame and need are then
 // read from its lane into scalar registers.  Each environment's ranges are
-// requested while the previous one finishes, as far as its need goes (the
-// PLANES form reads every range: it writes the LiDAR channels of each
-// environment's scan rays).  The 32-byte result is parked in the
+// requested while the previous one finishes; every range is read, for the
+// LiDAR channels of the scan rays.  The 32-byte result is parked in the
 // environment's own prior row (60 bytes), which phase 2 reads before it
 // writes the 15 prior values there: no scratch memory is needed.
-template <bool PLANES>
-__global__ __launch_bounds__(kBlockThreads) void onboard_scan_kernel(OnboardRows rows) {
+__global__ __launch_bounds__(kBlockThreads) void actor_scan_kernel(OnboardRows rows) {
     __shared__ RayPlanes rays;
     __shared__ u32x2 lists[kWavesPerBlock][kListCap + 64];  // + a spare entry per lane
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1472,16 +1475,13 @@ __global__ __launch_bounds__(kBlockThreads) void onboard_scan_kernel(OnboardRows
     };
     // Lane j forms the frame of the wave's j-th environment from here (a
     // lane past the batch repeats the current one, whose row exists), and
-    // what its mission uses of the scan (all of it when the caller asks for
-    // the scan's diagnostics).
+    // what its mission uses of the scan.
     auto frame_obs = [&](size_t first) {
         const size_t e0 = first + (size_t)lane * waves, e = e0 < rows.batch ? e0 : first;
         return load_frame_obs(obs_of(e), reinterpret_cast<const float *>(
                                              rows.mission + e * rows.mission_stride));
     };
-    auto frame_need = [&](const FrameObs &v) {
-        return rows.diag ? kNeedAll : scan_need(v.m4, v.m5);
-    };
+    auto frame_need = [&](const FrameObs &v) { return scan_need(v.m4, v.m5); };
     FrameObs first_obs = frame_obs(env);
     float rg[kScanRays];
     load_ranges(obs_rsrc(obs_of(env), true), obs_rsrc(obs_of(env), true), lane, rg);
@@ -1497,24 +1497,15 @@ __global__ __launch_bounds__(kBlockThreads) void onboard_scan_kernel(OnboardRows
                                   __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine.py), k));
         const size_t next_env = env + waves;
         const bool has_next = next_env < rows.batch;
-        // The next environment's ranges are requested only when it uses
-        // them (or when the actor's planes need them); the first
-        // environment of the next 64 has no need formed yet and is loaded.
         const int need = __builtin_amdgcn_readlane(need_mine, k);
-        const int need_next = k + 1 < 64 ? __builtin_amdgcn_readlane(need_mine, (k + 1) & 63)
-                                         : kNeedAll;
-        const float *next_obs = has_next ? obs_of(next_env) : nullptr;
         const __amdgpu_buffer_rsrc_t next =
-            obs_rsrc(next_obs, has_next && (PLANES || need_next != kNeedNone));
-        const __amdgpu_buffer_rsrc_t next_upper =
-            obs_rsrc(next_obs, has_next && (PLANES || (need_next & kNeedCorridor)));
-        if (PLANES)
-            write_channel_planes(
-                rg, __builtin_amdgcn_make_buffer_rsrc(rows.lidar + env * 12288, (short)0,
-                                                      12288 * 4, kBufferWord3),
-                lane);
+            obs_rsrc(has_next ? obs_of(next_env) : nullptr, has_next);
+        write_channel_planes(
+            rg, __builtin_amdgcn_make_buffer_rsrc(rows.lidar + env * 12288, (short)0,
+                                                  12288 * 4, kBufferWord3),
+            lane);
         ScanResult s;
-        scan_env(rg, rays, f, next, next_upper, lane, lists[__builtin_amdgcn_readfirstlane(tid >> 6)],
+        scan_env(rg, rays, f, next, next, lane, lists[__builtin_amdgcn_readfirstlane(tid >> 6)],
                  s, need);
         if (lane == 0) park_scan(rows.prior + env * 15, s);
         if (!has_next) break;
@@ -1528,334 +1519,48 @@ __global__ __launch_bounds__(kBlockThreads) void onboard_scan_kernel(OnboardRows
     }
 }
 
-// Phase 1 of the H2 entry: the scan of the environments whose mission uses
-// it, shared out over a CU.  One workgroup of 16 waves per CU takes
-// environments g, g + G, g + 2G, ... (G workgroups in the grid), up to 1,024
-// per round.  Each wave forms the frames and needs of 64 of them (lane j the
-// j-th); an environment whose mission uses no scan result parks the empty
-// result from its lane, and the others are entered (frame, need) in the
-// workgroup's pool in LDS.  The waves then take pool entries one at a time
-// from a counter in LDS, the next one taken while the current one is
-// scanned so that its ranges are requested as far as its need goes.  Which
-// wave scans which environment varies from call to call; each result
-// depends only on its environment.  A static share of the environments
-// would leave the waves that drew several slalom missions working long after
-// the others: at 16,384 environments (four per wave) that wave sets the
-// kernel's time.  The onboard entry uses this kernel from 2,560
-// environments, except for the batches that the one-kernel form takes.
-constexpr int kPoolThreads = 1024;
-constexpr int kPoolWaves = kPoolThreads / 64;
-constexpr int kPoolRound = kPoolThreads;  // environments per round, one per thread
-constexpr unsigned kPoolBlocks = 256;     // one workgroup per CU
-// The onboard entry's batch from which the pool pays.  Measured on one box
-// (static share -> pool, us): 2,048 envs 17.4 -> 17.9, 3,072 18.5 -> 18.1,
-// 4,096 19.6 -> 18.2, 16,384 28.4 -> 25.3; below 2,048 the pool is 0.9-1.5
-// us slower (the needs are formed before any range is requested, and a
-// workgroup holds at most a few environments whose mission uses the scan).
-constexpr size_t kPoolMinBatch = 2560;
-// The onboard entry's batches that take the one-kernel form (each
-// workgroup scans its own 64 environments, then runs their controller).
-// Two of its workgroups fit a CU, so one's scan overlaps the other's
-// controller; below kFusedMinBatch the workgroups are fewer than the CUs and
-// the two-kernel form spreads the scan over all of them.  Measured on one
-// box (two kernels -> one, us): 4,000 envs 15.2 -> 16.3, 8,000 17.4 -> 17.0,
-// 20,000 28.2 -> 24.7, 39,999 46.5 -> 42.8, 65,000 60.1 -> 50.3.
-constexpr size_t kFusedMinBatch = 8192;
-struct PoolEntry {
-    unsigned env;  // kMaxBatch < 2^31
-    int need;
-    float r[9], py;
-};
+// The onboard entry's workgroups: one group of 16 environments up to
+// kOneGroupMax (two workgroups on every CU), two up to kTwoGroupMax, four
+// above, in equal shares while that is one round of kRoundBlocks.  Fewer
+// groups are shorter chains, more share the ray table, the launch and the
+// scanning waves.  Measured on one box, us, scenes as the generator makes
+// them / cluttered (two launches before, the scan and the control kernel;
+// one group; two; four):
+//    1,000  16.1 / 18.2   9.4 / 11.2  12.5 / 15.3       --
+//    8,192  20.5 / 23.3  11.5 / 14.2  12.9 / 16.3  15.8 / 18.6
+//   12,288  21.2 / 24.5  18.9 / 22.6  15.6 / 19.0  18.6 / 21.1
+//   16,384  22.3 / 25.3  21.5 / 25.6  15.9 / 19.3  20.5 / 22.9
+//   17,000  34.6 / 38.3       --      22.5 / 26.9  21.2 / 23.6
+//   32,768  42.8 / 46.2       --      31.0 / 37.6  27.1 / 29.7
+//   39,999  55.8 / 59.3  46.8 / 55.4  37.8 / 46.0  37.5 / 41.8
+//   65,536  78.5 / 82.0  73.6 / 87.1  57.3 / 67.8  49.0 / 54.2
+// (Equal shares over two rounds lose: 39,999 at 40 each 40.2 / 45.2, since a
+// CU's last workgroup alone runs faster than two.)
+constexpr size_t kOneGroupMax = 8192, kTwoGroupMax = 16384;
+constexpr size_t kRoundBlocks = 512;  // workgroups resident at once: two per CU
+constexpr int kPoolWaves = kControlThreads / 64;
 
-__global__ __launch_bounds__(kPoolThreads) void onboard_scan_pool_kernel(OnboardRows rows) {
-    __shared__ RayPlanes rays;
-    __shared__ u32x2 lists[kPoolWaves][kListCap + 64];  // + a spare entry per lane
-    __shared__ PoolEntry pool[kPoolRound];
-    __shared__ int pool_count, pool_next;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const size_t groups = gridDim.x;
-    // The launch gives every workgroup at least one environment.
-    const size_t mine = (rows.batch - blockIdx.x + groups - 1) / groups;
-    const size_t rounds = (mine + kPoolRound - 1) / kPoolRound;
-    auto obs_of = [&](size_t e) {
-        return reinterpret_cast<const float *>(rows.obs + e * rows.obs_stride);
-    };
-    for (int i = tid; i < 1536; i += kPoolThreads) {
-        rays.d[0][i] = kRayDir[i * 3 + 0];
-        rays.d[1][i] = kRayDir[i * 3 + 1];
-        rays.d[2][i] = kRayDir[i * 3 + 2];
-    }
-    if (tid == 0) {
-        pool_count = 0;
-        pool_next = 0;
-    }
-    __syncthreads();
-    // One lane takes the next entry for its wave.
-    auto take = [&]() {
-        int t = 0;
-        if (lane == 0)
-            t = __hip_atomic_fetch_add(&pool_next, 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-        return __builtin_amdgcn_readfirstlane(t);
-    };
-    auto entry_env = [&](int t, size_t &env, int &need) {
-        env = (unsigned)__builtin_amdgcn_readfirstlane((int)pool[t].env);
-        need = __builtin_amdgcn_readfirstlane(pool[t].need);
-    };
-    auto entry_frame = [&](int t) {
-        ScanFrame f;
-#pragma unroll
-        for (int i = 0; i < 9; ++i)
-            f.r[i] = __builtin_bit_cast(
-                float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, pool[t].r[i])));
-        f.py = __builtin_bit_cast(
-            float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, pool[t].py)));
-        return f;
-    };
-    u32x2 *list = lists[wave];
-    float rg[kScanRays];
-    for (size_t round = 0; round < rounds; ++round) {
-        // Thread x forms environment i = x of the round.
-        const size_t i = round * kPoolRound + (size_t)tid;
-        const size_t e = blockIdx.x + i * groups;
-        const bool valid = i < mine;
-        if (__builtin_amdgcn_readfirstlane((int)valid)) {  // lane 0 is valid whenever any lane is
-            const size_t row = valid ? e : blockIdx.x;
-            FrameObs v = load_frame_obs(
-                obs_of(row), reinterpret_cast<const float *>(rows.mission + row * rows.mission_stride));
-            const ScanFrame f = scan_frame(v);
-            const int need = rows.diag ? kNeedAll : scan_need(v.m4, v.m5);
-            const bool entered = valid && need != kNeedNone;
-            if (valid && !entered)
-                park_scan(rows.prior + e * 15, ScanResult{30.0f, 0.0f, 0.0f, 30.0f, 0.0f, -1, 0, 0});
-            const uint64_t m = __builtin_amdgcn_ballot_w64(entered);
-            int base = 0;
-            if (lane == 0 && m)
-                base = __hip_atomic_fetch_add(&pool_count, (int)__builtin_popcountll(m),
-                                              __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            base = __builtin_amdgcn_readfirstlane(base);
-            if (entered) {
-                PoolEntry &p = pool[base + (int)__builtin_amdgcn_mbcnt_hi(
-                                               (unsigned)(m >> 32),
-                                               __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u))];
-                p.env = (unsigned)e;
-                p.need = need;
-#pragma unroll
-                for (int k = 0; k < 9; ++k) p.r[k] = f.r[k];
-                p.py = f.py;
-            }
-        }
-        __syncthreads();
-        const int count = __builtin_amdgcn_readfirstlane(pool_count);
-        int t = take();
-        if (t < count) {
-            size_t env;
-            int need;
-            entry_env(t, env, need);
-            load_ranges(obs_rsrc(obs_of(env), true),
-                        obs_rsrc(obs_of(env), (need & kNeedCorridor) != 0), lane, rg);
-            for (;;) {
-                const ScanFrame f = entry_frame(t);
-                // The next entry is taken before this one is scanned: the
-                // scan requests its ranges once these are consumed.
-                const int t_next = take();
-                const bool has_next = t_next < count;
-                size_t next_env = env;
-                int next_need = kNeedNone;
-                if (has_next) entry_env(t_next, next_env, next_need);
-                const float *next_obs = obs_of(next_env);
-                ScanResult s;
-                scan_env(rg, rays, f, obs_rsrc(next_obs, has_next),
-                         obs_rsrc(next_obs, has_next && (next_need & kNeedCorridor)), lane, list,
-                         s, need);
-                if (lane == 0) park_scan(rows.prior + env * 15, s);
-                if (!has_next) break;
-                t = t_next;
-                env = next_env;
-                need = next_need;
-            }
-        }
-        // Every wave has taken past the end of this round's pool.
-        __syncthreads();
-        if (tid == 0) {
-            pool_count = 0;
-            pool_next = 0;
-        }
-        __syncthreads();
-    }
-}
-
-// Phase 2's inputs for the 64 environments of a workgroup: obs[0..47],
-// mission[0..9] and the parked scan result.  Odd row pitches put the rows a
+// The inputs of N environments in LDS: obs[0..47], mission[0..9], the scan
+// result, and for the actor obs[4144..4147].  Odd row pitches put the rows a
 // wave reads (64 lanes, or 16 quads) on different LDS banks.
 constexpr int kStageObs = 48, kStageObsPitch = 49, kStageMissionPitch = 11, kStageScanPitch = 9;
-struct ControlStage {
-    float obs[64][kStageObsPitch];
-    float mission[64][kStageMissionPitch];
-    float scan[64][kStageScanPitch];
-    float tail[64][5];  // obs[4144..4147], for the actor's scalar wave
+template <int N>
+struct Stage {
+    float obs[N][kStageObsPitch];
+    float mission[N][kStageMissionPitch];
+    float scan[N][kStageScanPitch];
+    float tail[N][5];
 };
 
-// Phase 2: the tactical features and the controller, from the parked scan
-// result (FUSED: from the workgroup's own scan, phase 1 and 2 in one
-// kernel).  A workgroup covers 64 environments: waves 0..3 run the flight
-// controller, waves 4..7 the tactical features, the cannon and the BWB law,
-// each on one quad of lanes per environment (16 per wave), so every SIMD
-// holds one wave of each.  The time of the chains is their instruction
-// count (onboard_math.h), so they are written without branches (conditions
-// are formed first and values selected; as nested conditionals they became
-// 130 branches, with the computation inside and five instructions of mask
-// handling each), take short forms of the functions, and have a form for
-// tame inputs without the reference's checks for infinities and NaN.
-// Cycles of a workgroup's chains at 1,000 environments, before these and
-// after: 16,800 in the flight wave that held BWB missions (13,700 in the
-// others) and 4,800 in the tactical waves -> 7,000 and 11,600.
-//   * One pass per workgroup, without a grid-stride loop: in a loop the
-//     compiler kept 64-bit coefficients and literals in registers across it,
-//     256 of them; without it the chains fit in 128, and two workgroups in a
-//     CU.
-// For the actor's inputs (SCALARS) each tactical wave then writes the symlog
-// scalars and mission values of its 16 environments, one row per store (on
-// the scan waves they cost the scan kernel 6 µs and the plane kernel of the
-// next call 6 µs more).
-//   * The workgroup first stages every input its chains read (all loads
-//     issued at once, coalesced over the rows' first 192 bytes), so the
-//     chains read LDS: read from global memory at their points of use, the
-//     values came in a dozen dependent round trips.
-//   * Values are formed in registers and then stored to each destination
-//     (the tactical / prior rows and, for the actor, their copies in
-//     proprio and mission_vec).
-// FUSED: the workgroup also scans its own environments (the onboard
-// entry's one-kernel form), from a pool in LDS over its eight waves, and the
-// results go straight into the stage.
-struct FusedScanLds {
-    RayPlanes rays;
-    u32x2 lists[2 * kControlWaves][kListCap + 64];  // + a spare entry per lane
-    PoolEntry pool[64];
-    int count, next;
-};
-
-// The scan of the workgroup's 64 staged environments (base + e), called by
-// every wave after the stage is written: wave 0 forms each environment's
-// frame and need from the stage (lane e), writes the empty result of those
-// whose mission uses no scan result and enters the others in the pool; then
-// every wave takes entries one at a time, the next one taken before the
-// current one is scanned so that its ranges are requested as far as its
-// need goes, and lane 0 writes each result into the stage.  Ends with the
-// workgroup's barrier, so the results are visible to the control phase.
-__device__ __forceinline__ void fused_scan(const OnboardRows &rows, size_t base,
-                                           ControlStage &stage, FusedScanLds &fused, int w,
-                                           int lane) {
-    auto obs_of = [&](size_t e) {
-        return reinterpret_cast<const float *>(rows.obs + e * rows.obs_stride);
-    };
-    auto stage_result = [&](int e, const ScanResult &r) {
-        float *sc = stage.scan[e];
-        sc[0] = r.min_r;
-        sc[1] = r.min_r_dx;
-        sc[2] = r.min_r_dy;
-        sc[3] = r.min_dx_c;
-        sc[4] = r.cluster_y_sum;
-        sc[5] = __int_as_float(r.min_ray);
-        sc[6] = __int_as_float(r.cluster_count);
-    };
-    if (w == 0) {
-        const int e = lane;
-        const bool valid = base + (size_t)e < rows.batch;
-        FrameObs v{stage.obs[e][1], stage.obs[e][6], stage.obs[e][7], stage.obs[e][8],
-                   stage.obs[e][9], stage.mission[e][4], stage.mission[e][5]};
-        const ScanFrame f = scan_frame(v);
-        const int need = rows.diag ? kNeedAll : scan_need(v.m4, v.m5);
-        const bool entered = valid && need != kNeedNone;
-        if (valid && !entered) stage_result(e, ScanResult{30.0f, 0.0f, 0.0f, 30.0f, 0.0f, -1, 0, 0});
-        // Corridor scans (the longest) first.
-        const bool front = (need & kNeedCorridor) != 0;
-        const uint64_t mf = __builtin_amdgcn_ballot_w64(entered && front);
-        const uint64_t mb = __builtin_amdgcn_ballot_w64(entered && !front);
-        const uint64_t m = mf | mb;
-        if (entered) {
-            const uint64_t mine = front ? mf : mb;
-            const unsigned rank = __builtin_amdgcn_mbcnt_hi(
-                (unsigned)(mine >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0u));
-            PoolEntry &p = fused.pool[(front ? 0u : (unsigned)__builtin_popcountll(mf)) + rank];
-            p.env = (unsigned)e;
-            p.need = need;
-#pragma unroll
-            for (int k = 0; k < 9; ++k) p.r[k] = f.r[k];
-            p.py = f.py;
-        }
-        if (lane == 0) {
-            fused.count = (int)__builtin_popcountll(m);
-            fused.next = 0;
-        }
-    }
-    __syncthreads();
-    const int count = __builtin_amdgcn_readfirstlane(fused.count);
-    auto take = [&]() {
-        int t = 0;
-        if (lane == 0)
-            t = __hip_atomic_fetch_add(&fused.next, 1, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_WORKGROUP);
-        return __builtin_amdgcn_readfirstlane(t);
-    };
-    auto entry = [&](int t, int &slot, int &need) {
-        slot = __builtin_amdgcn_readfirstlane((int)fused.pool[t].env);
-        need = __builtin_amdgcn_readfirstlane(fused.pool[t].need);
-    };
-    int t = take();
-    if (t < count) {
-        int slot, need;
-        entry(t, slot, need);
-        float rg[kScanRays];
-        const float *o = obs_of(base + (size_t)slot);
-        load_ranges(obs_rsrc(o, true), obs_rsrc(o, (need & kNeedCorridor) != 0), lane, rg);
-        for (;;) {
-            ScanFrame f;
-#pragma unroll
-            for (int i = 0; i < 9; ++i)
-                f.r[i] = __builtin_bit_cast(
-                    float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, fused.pool[t].r[i])));
-            f.py = __builtin_bit_cast(
-                float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, fused.pool[t].py)));
-            const int t_next = take();
-            const bool has_next = t_next < count;
-            int next_slot = slot, next_need = kNeedNone;
-            if (has_next) entry(t_next, next_slot, next_need);
-            const float *next_obs = obs_of(base + (size_t)next_slot);
-            ScanResult r;
-            scan_env(rg, fused.rays, f, obs_rsrc(next_obs, has_next),
-                     obs_rsrc(next_obs, has_next && (next_need & kNeedCorridor)), lane,
-                     fused.lists[w], r, need);
-            if (lane == 0) stage_result(slot, r);
-            if (!has_next) break;
-            t = t_next;
-            slot = next_slot;
-            need = next_need;
-        }
-    }
-    __syncthreads();
-}
-
-template <bool SCALARS, bool FUSED>
-__global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
-void onboard_control_kernel(OnboardRows rows) {
-    constexpr int CW = kControlWaves, N = 64, kThreads = kControlThreads;
-    __shared__ ControlStage stage;
-    __shared__ std::conditional_t<FUSED, FusedScanLds, char> fused;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int a = lane & 3;
-    if constexpr (FUSED) {
-        for (int i = tid; i < 1536; i += kThreads) {
-            fused.rays.d[0][i] = kRayDir[i * 3 + 0];
-            fused.rays.d[1][i] = kRayDir[i * 3 + 1];
-            fused.rays.d[2][i] = kRayDir[i * 3 + 2];
-        }
-    }
-    const size_t base = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * N;
-    if (base >= rows.batch) return;
-    // Rows past the batch end re-read the last row; nothing uses them.
+// Stages environments base .. base + N - 1, every load issued at once and
+// coalesced over the rows' first 192 bytes, so that the chains read LDS: read
+// from global memory at their points of use, the values came in a dozen
+// dependent round trips.  PARKED: also the scan results parked in the prior
+// rows.  Rows past the batch end re-read the last row; nothing uses them.
+template <int N, bool TAIL, bool PARKED>
+__device__ __forceinline__ void stage_inputs(const OnboardRows &rows, size_t base, Stage<N> &stage,
+                                             int tid) {
+    constexpr int kThreads = kControlThreads;
     auto row_of = [&](int e) {
         const size_t env = base + (size_t)e;
         return env < rows.batch ? env : rows.batch - 1;
@@ -1863,8 +1568,8 @@ void onboard_control_kernel(OnboardRows rows) {
     constexpr int kObsLoads = (N * kStageObs + kThreads - 1) / kThreads;
     constexpr int kMissionLoads = (N * 10 + kThreads - 1) / kThreads;
     constexpr int kScanLoads = (N * 7 + kThreads - 1) / kThreads;
-    // Every thread issues all its loads unconditionally (an index past
-    // the stage re-reads the stage's last value), so they leave at once.
+    // Every thread issues all its loads unconditionally (an index past the
+    // stage re-reads the stage's last value), so they leave at once.
     float vo[kObsLoads], vm[kMissionLoads], vs[kScanLoads], vt = 0.0f;
 #pragma unroll
     for (int k = 0; k < kObsLoads; ++k) {
@@ -1878,17 +1583,19 @@ void onboard_control_kernel(OnboardRows rows) {
         const int e = idx / 10, i = idx - 10 * e;
         vm[k] = reinterpret_cast<const float *>(rows.mission + row_of(e) * rows.mission_stride)[i];
     }
+    if (PARKED) {
 #pragma unroll
-    for (int k = 0; k < kScanLoads; ++k) {
-        const int idx = min(tid + kThreads * k, N * 7 - 1);
-        const int e = idx / 7, i = idx - 7 * e;
-        vs[k] = FUSED ? 0.0f : rows.prior[row_of(e) * 15 + i];
+        for (int k = 0; k < kScanLoads; ++k) {
+            const int idx = min(tid + kThreads * k, N * 7 - 1);
+            const int e = idx / 7, i = idx - 7 * e;
+            vs[k] = rows.prior[row_of(e) * 15 + i];
+        }
     }
-    if (SCALARS) {
+    if (TAIL) {
         const int idx = min(tid, N * 4 - 1);
         const int e = idx / 4;
-        vt = reinterpret_cast<const float *>(
-            rows.obs + row_of(e) * rows.obs_stride)[4144 + idx - 4 * e];
+        vt = reinterpret_cast<const float *>(rows.obs +
+                                             row_of(e) * rows.obs_stride)[4144 + idx - 4 * e];
     }
 #pragma unroll
     for (int k = 0; k < kObsLoads; ++k) {
@@ -1902,152 +1609,381 @@ void onboard_control_kernel(OnboardRows rows) {
         const int e = idx / 10;
         if (idx < N * 10) stage.mission[e][idx - 10 * e] = vm[k];
     }
+    if (PARKED) {
 #pragma unroll
-    for (int k = 0; k < kScanLoads; ++k) {
-        const int idx = tid + kThreads * k;
-        const int e = idx / 7;
-        if (!FUSED && idx < N * 7) stage.scan[e][idx - 7 * e] = vs[k];
+        for (int k = 0; k < kScanLoads; ++k) {
+            const int idx = tid + kThreads * k;
+            const int e = idx / 7;
+            if (idx < N * 7) stage.scan[e][idx - 7 * e] = vs[k];
+        }
     }
-    if (SCALARS && tid < N * 4) stage.tail[tid / 4][tid % 4] = vt;
-    __syncthreads();
-    if constexpr (FUSED) fused_scan(rows, base, stage, fused, w, lane);
+    if (TAIL && tid < N * 4) stage.tail[tid / 4][tid % 4] = vt;
+}
 
-    const int slot = 16 * (w & (CW - 1)) + (lane >> 2);
-    const size_t env = base + (size_t)slot;
-    if (env < rows.batch) {
-        ChainInputs in = chain_inputs(stage.obs[slot], stage.mission[slot], a);
-        const bool tame = tame_inputs(in);
-        float *const prior = rows.prior + env * 15;
-        float *const p = rows.proprio ? rows.proprio + env * 91 + 52 : nullptr;
-        float *const mv = rows.proprio ? rows.mission_vec + env * 49 + 10 : nullptr;
-        auto store_arm = [&](const ArmOutputs &n) {
-            prior[a] = n.throttle;
-            prior[4 + a] = n.outer;
-            prior[8 + a] = n.inner;
-            if (p) {
-                p[24 + a] = n.throttle;
-                p[28 + a] = n.outer;
-                p[32 + a] = n.inner;
-                mv[24 + a] = n.throttle;
-                mv[28 + a] = n.outer;
-                mv[32 + a] = n.inner;
-            }
-        };
-        if (w >= CW) {
-            // Lane a of the quad writes features 6a .. 6a + 5.
-            float t[6];
-            if (tame) tactical_quad<true>(in, a, t);
-            else tactical_quad<false>(in, a, t);
-            float *tac = rows.tactical + env * 24 + 6 * a;
-#pragma unroll
-            for (int i = 0; i < 6; ++i) tac[i] = t[i];
-            if (p) {
-#pragma unroll
-                for (int i = 0; i < 6; ++i) {
-                    p[6 * a + i] = t[i];
-                    mv[6 * a + i] = t[i];
-                }
-            }
-            if (!tame) controller_inputs(in);
-            const MissionFlags f = mission_flags(in.m);
-            const GunOutputs g = tame ? gunnery_quad<true>(in, f, a) : gunnery_quad<false>(in, f, a);
-            if (f.bwb) store_arm(g.arm);
-            if (a == 0) {
-                prior[12] = g.az;
-                prior[13] = g.el;
-                prior[14] = g.fire;
-                if (p) {
-                    p[36] = g.az;
-                    p[37] = g.el;
-                    p[38] = g.fire;
-                    mv[36] = g.az;
-                    mv[37] = g.el;
-                    mv[38] = g.fire;
-                }
-            }
-        } else {
-            const float *sc = stage.scan[slot];
-            ScanResult s;
-            s.min_r = sc[0];
-            s.min_r_dx = sc[1];
-            s.min_r_dy = sc[2];
-            s.min_dx_c = sc[3];
-            s.cluster_y_sum = sc[4];
-            s.min_ray = __float_as_int(sc[5]);
-            s.cluster_count = __float_as_int(sc[6]);
-            // Read from LDS before the chain, like the other inputs.
-            asm volatile("" : "+v"(s.min_r), "+v"(s.min_r_dx), "+v"(s.min_r_dy), "+v"(s.min_dx_c),
-                         "+v"(s.cluster_y_sum), "+v"(s.min_ray), "+v"(s.cluster_count));
-            if (!tame) controller_inputs(in);
-            const MissionFlags f = mission_flags(in.m);
-            const ArmOutputs n =
-                tame ? flight_quad<true>(in, f, s, a) : flight_quad<false>(in, f, s, a);
-            if (!f.bwb) store_arm(n);  // a BWB mission's are the other waves'
-            if (rows.diag && a == 0) {
-                float *d = rows.diag + env * 5;
-                d[0] = s.min_r;
-                d[1] = (float)s.min_ray;
-                d[2] = s.min_dx_c;
-                d[3] = (float)s.cluster_count;
-                d[4] = s.cluster_y_sum;
-            }
+template <int N>
+__device__ __forceinline__ void stage_result(Stage<N> &stage, int e, const ScanResult &r) {
+    float *sc = stage.scan[e];
+    sc[0] = r.min_r;
+    sc[1] = r.min_r_dx;
+    sc[2] = r.min_r_dy;
+    sc[3] = r.min_dx_c;
+    sc[4] = r.cluster_y_sum;
+    sc[5] = __int_as_float(r.min_ray);
+    sc[6] = __int_as_float(r.cluster_count);
+}
+
+// Where an environment's tactical and prior values go: their rows, and for
+// the actor their copies in proprio and mission_vec.
+struct OutputRows {
+    float *tactical, *prior, *proprio, *mission_vec;
+    __device__ __forceinline__ OutputRows(const OnboardRows &rows, size_t env)
+        : tactical(rows.tactical + env * 24), prior(rows.prior + env * 15),
+          proprio(rows.proprio ? rows.proprio + env * 91 + 52 : nullptr),
+          mission_vec(rows.proprio ? rows.mission_vec + env * 49 + 10 : nullptr) {}
+    __device__ __forceinline__ void arm(int a, const ArmOutputs &n) const {
+        prior[a] = n.throttle;
+        prior[4 + a] = n.outer;
+        prior[8 + a] = n.inner;
+        if (proprio) {
+            proprio[24 + a] = n.throttle;
+            proprio[28 + a] = n.outer;
+            proprio[32 + a] = n.inner;
+            mission_vec[24 + a] = n.throttle;
+            mission_vec[28 + a] = n.outer;
+            mission_vec[32 + a] = n.inner;
         }
     }
-    if (SCALARS && w >= CW) {
-        // Lane l's input: obs[l] (l < 48), obs[4144 + l - 48] (l < 52),
-        // mission[l - 52] (l < 62).
-        const int lo = min(lane, kStageObs - 1), lt = min(max(lane - 48, 0), 3),
-                  lm = min(max(lane - 52, 0), 9);
-        // All 16 inputs are read first, so the 16 chains are
-        // independent; rows past the batch end (staged as copies of the
-        // last row) store nothing.
-        float raw[16];
+};
+
+// One wave: the tactical features, the cannon and the BWB law of the 16
+// environments from `first` of the stage on, a quad of lanes each.
+template <int N>
+__device__ __forceinline__ void support_wave(const OnboardRows &rows, size_t base,
+                                             const Stage<N> &stage, int first, int lane) {
+    const int a = lane & 3, slot = first + (lane >> 2);
+    const size_t env = base + (size_t)slot;
+    if (env >= rows.batch) return;
+    ChainInputs in = chain_inputs(stage.obs[slot], stage.mission[slot], a);
+    const bool wild = wild_inputs(in), tame = __builtin_amdgcn_ballot_w64(wild) == 0;
+    const OutputRows out(rows, env);
+    // Lane a of the quad writes features 6a .. 6a + 5.
+    float t[6];
+    if (tame) tactical_quad<true>(in, wild, a, t);
+    else tactical_quad<false>(in, wild, a, t);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int e = 16 * (w - CW) + j;
-            raw[j] = lane < 48 ? stage.obs[e][lo]
-                               : (lane < 52 ? stage.tail[e][lt] : stage.mission[e][lm]);
+    for (int i = 0; i < 6; ++i) out.tactical[6 * a + i] = t[i];
+    if (out.proprio) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) {
+            out.proprio[6 * a + i] = t[i];
+            out.mission_vec[6 * a + i] = t[i];
         }
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const size_t env = base + (size_t)(16 * (w - CW) + j);
-            const bool valid = env < rows.batch;
-            const size_t row = valid ? env : base;
-            actor_scalars(raw[j], lane, rows.proprio + row * 91, rows.mission_vec + row * 49,
-                          valid);
+    }
+    if (!tame) controller_inputs(in);
+    const MissionFlags f = mission_flags(in.m);
+    const GunOutputs g =
+        tame ? gunnery_quad<true>(in, wild, f, a) : gunnery_quad<false>(in, wild, f, a);
+    if (f.bwb) out.arm(a, g.arm);
+    if (a == 0) {
+        out.prior[12] = g.az;
+        out.prior[13] = g.el;
+        out.prior[14] = g.fire;
+        if (out.proprio) {
+            out.proprio[36] = g.az;
+            out.proprio[37] = g.el;
+            out.proprio[38] = g.fire;
+            out.mission_vec[36] = g.az;
+            out.mission_vec[37] = g.el;
+            out.mission_vec[38] = g.fire;
         }
     }
 }
 
-// One workgroup per 64 environments.
-dim3 control_grid(size_t batch) {
-    const size_t want = (batch + 63) / 64;
+// One wave: the flight controller of the 16 environments from `first` on.
+// `wait` returns when their scan results are in the stage.
+template <int N, class Wait>
+__device__ __forceinline__ void flight_wave(const OnboardRows &rows, size_t base,
+                                            const Stage<N> &stage, int first, int lane, Wait wait) {
+    const int a = lane & 3, slot = first + (lane >> 2);
+    const size_t env = base + (size_t)slot;
+    if (env >= rows.batch) return;
+    ChainInputs in = chain_inputs(stage.obs[slot], stage.mission[slot], a);
+    const bool wild = wild_inputs(in), tame = __builtin_amdgcn_ballot_w64(wild) == 0;
+    if (!tame) controller_inputs(in);
+    const MissionFlags f = mission_flags(in.m);
+    ScanResult s;
+    auto fetch = [&]() {
+        wait();
+        const float *sc = stage.scan[slot];
+        s.min_r = sc[0];
+        s.min_r_dx = sc[1];
+        s.min_r_dy = sc[2];
+        s.min_dx_c = sc[3];
+        s.cluster_y_sum = sc[4];
+        s.min_ray = __float_as_int(sc[5]);
+        s.cluster_count = __float_as_int(sc[6]);
+        // Read from LDS at once, like the other inputs.
+        asm volatile("" : "+v"(s.min_r), "+v"(s.min_r_dx), "+v"(s.min_r_dy), "+v"(s.min_dx_c),
+                     "+v"(s.cluster_y_sum), "+v"(s.min_ray), "+v"(s.cluster_count));
+        return s;
+    };
+    const ArmOutputs n =
+        tame ? flight_quad<true>(in, wild, f, a, fetch) : flight_quad<false>(in, wild, f, a, fetch);
+    if (!f.bwb) OutputRows(rows, env).arm(a, n);  // a BWB mission's are the support wave's
+    if (rows.diag && a == 0) {
+        float *d = rows.diag + env * 5;
+        d[0] = s.min_r;
+        d[1] = (float)s.min_ray;
+        d[2] = s.min_dx_c;
+        d[3] = (float)s.cluster_count;
+        d[4] = s.cluster_y_sum;
+    }
+}
+
+// One wave: the actor's symlog scalars and mission values of `Count`
+// environments first, first + step, ... of the stage.  Lane l's input:
+// obs[l] (l < 48), obs[4144 + l - 48] (l < 52), mission[l - 52] (l < 62).
+template <int Count, int N>
+__device__ __forceinline__ void scalars_wave(const OnboardRows &rows, size_t base,
+                                             const Stage<N> &stage, int first, int step,
+                                             int lane) {
+    const int lo = min(lane, kStageObs - 1), lt = min(max(lane - 48, 0), 3),
+              lm = min(max(lane - 52, 0), 9);
+    // All inputs are read first, so the chains are independent; rows past
+    // the stage or the batch end (staged as copies of the last row) store
+    // nothing.
+    float raw[Count];
+#pragma unroll
+    for (int j = 0; j < Count; ++j) {
+        const int e = min(first + step * j, N - 1);
+        raw[j] = lane < 48 ? stage.obs[e][lo]
+                           : (lane < 52 ? stage.tail[e][lt] : stage.mission[e][lm]);
+    }
+#pragma unroll
+    for (int j = 0; j < Count; ++j) {
+        const int e = first + step * j;
+        const size_t env = base + (size_t)e;
+        const bool valid = e < N && env < rows.batch;
+        const size_t row = valid ? env : base;
+        actor_scalars(raw[j], lane, rows.proprio + row * 91, rows.mission_vec + row * 49, valid);
+    }
+}
+
+// Phase 2 of the actor entry's two-stream form: the tactical features, the
+// controller and the actor's scalars from the parked scan results.  A
+// workgroup covers 64 environments: waves 0..3 run the flight controller,
+// waves 4..7 the tactical features, the cannon and the BWB law, each on one
+// quad of lanes per environment (16 per wave), so every SIMD holds one wave
+// of each; the latter then write the symlog scalars and mission values, one
+// row per store (on the scan waves they cost the scan kernel 6 µs and the
+// plane kernel of the next call 6 µs more).
+//
+// The time of the chains is their instruction count (onboard_math.h), so they
+// are written without branches (conditions are formed first and values
+// selected; as nested conditionals they became 130 branches, with the
+// computation inside and five instructions of mask handling each), take short
+// forms of the functions, and have a form for tame inputs without the
+// reference's checks for infinities and NaN.  Cycles of a workgroup's chains
+// at 1,000 environments, before these and after: 16,800 in the flight wave
+// that held BWB missions (13,700 in the others) and 4,800 in the tactical
+// waves -> 7,000 and 11,600.
+//   * One pass per workgroup, without a grid-stride loop: in a loop the
+//     compiler kept 64-bit coefficients and literals in registers across it,
+//     256 of them; without it the chains fit in 128.
+__global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void actor_control_kernel(OnboardRows rows) {
+    __shared__ Stage<64> stage;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const size_t base = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 64;
+    if (base >= rows.batch) return;
+    stage_inputs<64, true, true>(rows, base, stage, tid);
+    __syncthreads();
+    if (w < kControlWaves) {
+        flight_wave(rows, base, stage, 16 * w, lane, [] {});
+    } else {
+        support_wave(rows, base, stage, 16 * (w - kControlWaves), lane);
+        scalars_wave<16>(rows, base, stage, 16 * (w - kControlWaves), 1, lane);
+    }
+}
+
+// The onboard entry, and the actor entry's small batches: the scan, the
+// tactical features and the controller of G groups of 16 environments in one
+// workgroup of eight waves.
+//   * G = 1, 2: waves 0 .. G-1 run the flight controllers, waves G .. 2G-1
+//     the tactical features, cannon and BWB law, which need no scan; the
+//     others scan, and the support waves join them when they are done.
+//   * G = 4: all waves scan, then four of each role run the controllers.
+//     Two workgroups fit a CU, so one's scan overlaps the other's chains.
+//   * Wave 7 forms each environment's frame and need (lane e), stages the
+//     empty result of those whose mission uses no scan result and enters the
+//     others in a pool in LDS, corridor scans (the longest) first.  The
+//     scanning waves take entries one at a time, the next one taken before
+//     the current one is scanned so that its ranges are requested as far as
+//     its need goes.  Which wave scans which environment varies from call to
+//     call; each result depends only on its environment.
+//   * The flight waves form what does not depend on the scan and then wait
+//     until their group's results are staged: wave 7 publishes each group's
+//     count, every scanner takes its result off it.  The waves of a workgroup
+//     are resident together and no scanner waits for a flight wave, so the
+//     wait ends.
+struct PoolEntry {
+    unsigned env;
+    int need;
+    float r[9], py;
+};
+
+template <int G>
+struct OnboardLds {
+    RayPlanes rays;
+    u32x2 lists[kPoolWaves][kListCap + 64];  // + a spare entry per lane
+    PoolEntry pool[16 * G];
+    Stage<16 * G> stage;
+    int count, next, ready;
+    int left[G];  // results the group still lacks, once ready
+};
+
+template <int G, bool SCALARS>
+__device__ __forceinline__ void onboard_block(const OnboardRows &rows, size_t base,
+                                              OnboardLds<G> &s) {
+    constexpr int N = 16 * G, kThreads = kControlThreads;
+    constexpr bool kRoles = 2 * G < kPoolWaves;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    stage_inputs<N, SCALARS, false>(rows, base, s.stage, tid);
+    for (int i = tid; i < 1536; i += kThreads) {
+        s.rays.d[0][i] = kRayDir[i * 3 + 0];
+        s.rays.d[1][i] = kRayDir[i * 3 + 1];
+        s.rays.d[2][i] = kRayDir[i * 3 + 2];
+    }
+    if (tid == 0) {
+        s.next = 0;
+        s.ready = 0;
+    }
+    __syncthreads();
+    auto spin = [](int *word, int until) {
+        while (__hip_atomic_load(word, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != until)
+            __builtin_amdgcn_s_sleep(1);
+    };
+    if (kRoles && w < G) {
+        flight_wave(rows, base, s.stage, 16 * w, lane, [&] {
+            spin(&s.ready, 1);
+            spin(&s.left[w], 0);
+        });
+        return;
+    }
+    auto obs_of = [&](int e) {
+        return reinterpret_cast<const float *>(rows.obs + (base + (size_t)e) * rows.obs_stride);
+    };
+    if (w == kPoolWaves - 1) {
+        const int e = lane & (N - 1);
+        const bool valid = (N == 64 || lane < N) && base + (size_t)e < rows.batch;
+        FrameObs v{s.stage.obs[e][1], s.stage.obs[e][6], s.stage.obs[e][7], s.stage.obs[e][8],
+                   s.stage.obs[e][9], s.stage.mission[e][4], s.stage.mission[e][5]};
+        const ScanFrame f = scan_frame(v);
+        const int need = rows.diag ? kNeedAll : scan_need(v.m4, v.m5);
+        const bool entered = valid && need != kNeedNone;
+        if (valid && !entered)
+            stage_result(s.stage, e, ScanResult{30.0f, 0.0f, 0.0f, 30.0f, 0.0f, -1, 0, 0});
+        const bool front = (need & kNeedCorridor) != 0;
+        const uint64_t mf = __builtin_amdgcn_ballot_w64(entered && front);
+        const uint64_t mb = __builtin_amdgcn_ballot_w64(entered && !front);
+        if (entered) {
+            const uint64_t mine = front ? mf : mb;
+            const unsigned rank = __builtin_amdgcn_mbcnt_hi(
+                (unsigned)(mine >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mine, 0u));
+            PoolEntry &p = s.pool[(front ? 0u : (unsigned)__builtin_popcountll(mf)) + rank];
+            p.env = (unsigned)e;
+            p.need = need;
+#pragma unroll
+            for (int k = 0; k < 9; ++k) p.r[k] = f.r[k];
+            p.py = f.py;
+        }
+        if (lane == 0) {
+            s.count = (int)__builtin_popcountll(mf | mb);
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                s.left[g] = __builtin_popcount((unsigned)((mf | mb) >> (16 * g)) & 0xffffu);
+        }
+        // The wave's LDS writes are in order; the release waits for them.
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0)
+            __hip_atomic_store(&s.ready, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    if (kRoles && w < 2 * G) support_wave(rows, base, s.stage, 16 * (w - G), lane);
+    spin(&s.ready, 1);
+    const int count = __builtin_amdgcn_readfirstlane(s.count);
+    auto take = [&]() {
+        int t = 0;
+        if (lane == 0)
+            t = __hip_atomic_fetch_add(&s.next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return __builtin_amdgcn_readfirstlane(t);
+    };
+    auto entry = [&](int t, int &slot, int &need) {
+        slot = __builtin_amdgcn_readfirstlane((int)s.pool[t].env);
+        need = __builtin_amdgcn_readfirstlane(s.pool[t].need);
+    };
+    int t = take();
+    if (t < count) {
+        int slot, need;
+        entry(t, slot, need);
+        float rg[kScanRays];
+        load_ranges(obs_rsrc(obs_of(slot), true), obs_rsrc(obs_of(slot), (need & kNeedCorridor) != 0),
+                    lane, rg);
+        for (;;) {
+            ScanFrame f;
+#pragma unroll
+            for (int i = 0; i < 9; ++i)
+                f.r[i] = __builtin_bit_cast(
+                    float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s.pool[t].r[i])));
+            f.py = __builtin_bit_cast(
+                float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s.pool[t].py)));
+            const int t_next = take();
+            const bool has_next = t_next < count;
+            int next_slot = slot, next_need = kNeedNone;
+            if (has_next) entry(t_next, next_slot, next_need);
+            const float *next_obs = obs_of(next_slot);
+            ScanResult r;
+            scan_env(rg, s.rays, f, obs_rsrc(next_obs, has_next),
+                     obs_rsrc(next_obs, has_next && (next_need & kNeedCorridor)), lane, s.lists[w],
+                     r, need);
+            if (lane == 0) {
+                stage_result(s.stage, slot, r);
+                __hip_atomic_fetch_sub(&s.left[slot / 16], 1, __ATOMIC_RELEASE,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            if (!has_next) break;
+            t = t_next;
+            slot = next_slot;
+            need = next_need;
+        }
+    }
+    if constexpr (!kRoles) {
+        __syncthreads();
+        if (w < G) flight_wave(rows, base, s.stage, 16 * w, lane, [] {});
+        else support_wave(rows, base, s.stage, 16 * (w - G), lane);
+    }
+    if (SCALARS) {
+        constexpr int kWaves = kPoolWaves - G, kEach = (N + kWaves - 1) / kWaves;
+        scalars_wave<kEach>(rows, base, s.stage, w - G, kWaves, lane);
+    }
+}
+
+// `share` environments per workgroup, at most 16 G.
+template <int G>
+__global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void onboard_kernel(OnboardRows rows, unsigned share) {
+    __shared__ OnboardLds<G> lds;
+    const size_t base = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * share;
+    if (base >= rows.batch) return;
+    if (rows.batch - base > share) rows.batch = base + share;  // this workgroup's end
+    onboard_block<G, false>(rows, base, lds);
+}
+
+// A grid of `want` workgroups.
+dim3 wide_grid(size_t want) {
     return dim3((unsigned)(want < kControlGridX ? want : kControlGridX),
                 (unsigned)((want + kControlGridX - 1) / kControlGridX));
-}
-
-// `pooled` selects the pooled scan, which holds a whole CU per workgroup:
-// for calls whose scan runs alone, not beside the actor's plane kernel.
-int launch_onboard(const OnboardRows &rows, hipStream_t s, bool pooled) {
-    const size_t scan_want = (rows.batch + kWavesPerBlock - 1) / kWavesPerBlock;
-    const unsigned scan_blocks = scan_want > kScanBlocks ? kScanBlocks : (unsigned)scan_want;
-    if (rows.lidar) {
-        onboard_scan_kernel<true><<<scan_blocks, kBlockThreads, 0, s>>>(rows);
-    } else if (pooled) {
-        // At least 16 environments per workgroup (one per wave) while that
-        // fills the chip.
-        const size_t want = (rows.batch + kPoolWaves - 1) / kPoolWaves;
-        onboard_scan_pool_kernel<<<want > kPoolBlocks ? kPoolBlocks : (unsigned)want,
-                                   kPoolThreads, 0, s>>>(rows);
-    } else {
-        onboard_scan_kernel<false><<<scan_blocks, kBlockThreads, 0, s>>>(rows);
-    }
-    const dim3 ctrl = control_grid(rows.batch);
-    if (rows.proprio)
-        onboard_control_kernel<true, false><<<ctrl, kControlThreads, 0, s>>>(rows);
-    else
-        onboard_control_kernel<false, false><<<ctrl, kControlThreads, 0, s>>>(rows);
-    return hipGetLastError() == hipSuccess;
 }
 
 }  // namespace
@@ -2069,15 +2005,19 @@ extern "C" int tb_hip_onboard_tactical_prior_device(const float *obs, const floa
     rows.mission_vec = nullptr;
     rows.lidar = nullptr;
     rows.batch = batch_size;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     (void)hipGetLastError();
-    if (batch_size >= kFusedMinBatch) {
-        onboard_control_kernel<false, true>
-            <<<control_grid(batch_size), kControlThreads, 0,
-               reinterpret_cast<hipStream_t>(stream)>>>(rows);
-        return hipGetLastError() == hipSuccess;
+    if (batch_size <= kOneGroupMax) {
+        onboard_kernel<1><<<wide_grid((batch_size + 15) / 16), kControlThreads, 0, s>>>(rows, 16);
+    } else if (batch_size <= kTwoGroupMax) {
+        onboard_kernel<2><<<wide_grid((batch_size + 31) / 32), kControlThreads, 0, s>>>(rows, 32);
+    } else {
+        const size_t share = batch_size < 64 * kRoundBlocks
+                                 ? (batch_size + kRoundBlocks - 1) / kRoundBlocks : 64;
+        onboard_kernel<4><<<wide_grid((batch_size + share - 1) / share), kControlThreads, 0, s>>>(
+            rows, (unsigned)share);
     }
-    return launch_onboard(rows, reinterpret_cast<hipStream_t>(stream),
-                          batch_size >= kPoolMinBatch);
+    return hipGetLastError() == hipSuccess;
 }
 
 // ---------------------------------------------------------------------------
@@ -2087,13 +2027,13 @@ extern "C" int tb_hip_onboard_tactical_prior_device(const float *obs, const floa
 // per environment streams the LiDAR block once into the six channel planes
 // and the cameras once into luma: LiDAR in 16-byte loads, camera bytes in
 // 4-byte loads so that each lane's 4 luma values are one float4 and every
-// store instruction writes 1 KiB of consecutive output.  From the split
-// threshold on, the scan kernel writes the channels of the rays it reads
-// (elevation rows 0..5) and this kernel only those of rows 6..15, so each
-// LiDAR range is read from HBM once.
-// The control kernel's controller waves add each environment's 52 symlog
-// scalars and mission values after their chains, and store tactical / prior
-// and their copies.  Fusing the scan into the streaming launch was measured
+// store instruction writes 1 KiB of consecutive output.  In the two-stream
+// form the scan kernel writes the channels of the rays it reads (elevation
+// rows 0..5) and the plane kernel only those of rows 6..15, so each LiDAR
+// range is read from HBM once.  The onboard workgroups also write each
+// environment's 52 symlog scalars and mission values, and the copies of
+// tactical / prior.  In large batches, fusing the scan into the streaming
+// workgroups was measured
 // slower: next to saturated HBM traffic the scan's dependent loads stall.  Luma is
 // the reference's `(float)b * (1.0f / 255.0f) - 0.5f` as its CUDA build
 // evaluates it: nvcc contracts the product and difference into one fused
@@ -2115,13 +2055,21 @@ struct ActorRows {
     const unsigned char *cameras;
     float *lidar, *luma;
     size_t batch;
-    bool scan_rows;  // also the channels of the scan rows (else the scan kernel writes them)
 };
 
 __device__ __forceinline__ f32x4 lidar_channel4(f32x4 r, int kind) {
     f32x4 o;
 #pragma unroll
     for (int e = 0; e < 4; ++e) o[e] = lidar_channel(r[e], kind);
+    return o;
+}
+
+// Four camera bytes as luma.
+__device__ __forceinline__ f32x4 luma4(unsigned w) {
+    f32x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        o[e] = __builtin_fmaf((float)((w >> (8 * e)) & 0xffu), 1.0f / 255.0f, -0.5f);
     return o;
 }
 
@@ -2150,10 +2098,10 @@ __global__ __launch_bounds__(kStreamThreads) void actor_stream_kernel(ActorRows 
     for (size_t env = xcd_contiguous(blockIdx.x, gridDim.x); env < rows.batch;
          env += gridDim.x) {
         // float4 t is bins 4(t%512).. of head t/512, elevation row
-        // (t%512)/32.  Unless `scan_rows`, the scan kernel writes rows 0..5
+        // (t%512)/32.  The scan kernel writes rows 0..5
         // (threads with t%512 < 192, whole waves) and this kernel the other
         // ten.
-        const bool lidar = rows.lidar && (rows.scan_rows || (t & 511) >= kScanRowThreads);
+        const bool lidar = rows.lidar && (t & 511) >= kScanRowThreads;
         f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
         if (lidar)
             v = __builtin_nontemporal_load(
@@ -2176,50 +2124,92 @@ __global__ __launch_bounds__(kStreamThreads) void actor_stream_kernel(ActorRows 
             float *dst = rows.luma + env * 16384;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const unsigned w = px[k];
-                f32x4 o;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    o[e] = __builtin_fmaf((float)((w >> (8 * e)) & 0xffu), 1.0f / 255.0f,
-                                          -0.5f);
-                store_plane(dst, 16384 * 4, t + 1024 * k, o);
+                store_plane(dst, 16384 * 4, t + 1024 * k, luma4(px[k]));
             }
         }
     }
 }
 
-// The scan and control kernels run beside the plane kernel on a second
-// stream of the device, forked from and joined back to the caller's stream.
-// The plane kernel is write-bound and keeps one workgroup per CU; the scan
-// and control workgroups fit beside it, and their latency-bound chains
-// overlap its streams.  It is the controller that gains most: the scan alone
-// on the second stream, with the controller after the join, measured 437.9
-// against 433.0 us at 16,384 environments (before the split below).
+// The same planes by half a workgroup: 512 threads, each both heads' float4 t
+// and camera words t + 512 k.
+__device__ __forceinline__ void actor_planes_block(const ActorRows &rows, size_t env) {
+    const int t = threadIdx.x;
+    f32x4 v[2];
+    if (rows.lidar) {
+        const f32x4 *src = reinterpret_cast<const f32x4 *>(rows.obs + env * 4148 + 48);
+#pragma unroll
+        for (int head = 0; head < 2; ++head) v[head] = __builtin_nontemporal_load(src + 512 * head + t);
+    }
+    unsigned px[8];
+    if (rows.luma) {
+        const unsigned *cam = reinterpret_cast<const unsigned *>(rows.cameras + env * 16384);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) px[k] = __builtin_nontemporal_load(cam + t + 512 * k);
+    }
+    if (rows.lidar) {
+        float *dst = rows.lidar + env * 12288;
+#pragma unroll
+        for (int kind = 0; kind < 3; ++kind)
+#pragma unroll
+            for (int head = 0; head < 2; ++head)
+                store_plane(dst, 12288 * 4, (head + 2 * kind) * 512 + t,
+                            lidar_channel4(v[head], kind));
+    }
+    if (rows.luma) {
+        float *dst = rows.luma + env * 16384;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) store_plane(dst, 16384 * 4, t + 512 * k, luma4(px[k]));
+    }
+}
+
+// The whole preparation of a small batch in one launch: the first
+// `onboard_blocks` workgroups take 16 environments' onboard features and
+// scalars each (the longest chains start first), the others one
+// environment's planes each.
+__global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void actor_one_kernel(OnboardRows rows, ActorRows planes, unsigned onboard_blocks) {
+    __shared__ OnboardLds<1> lds;
+    if (blockIdx.x < onboard_blocks)
+        onboard_block<1, true>(rows, (size_t)blockIdx.x * 16, lds);
+    else
+        actor_planes_block(planes, blockIdx.x - onboard_blocks);
+}
+
+// The onboard features and scalars alone, for any batch.
+__global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void actor_onboard_kernel(OnboardRows rows) {
+    __shared__ OnboardLds<1> lds;
+    const size_t base = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 16;
+    if (base >= rows.batch) return;
+    onboard_block<1, true>(rows, base, lds);
+}
+
+// From kOverlapMinBatch environments the scan and control kernels run beside
+// the plane kernel on a second stream of the device, forked from and joined
+// back to the caller's stream.  The plane kernel is write-bound and keeps one
+// workgroup per CU; the scan and control workgroups fit beside it, and their
+// latency-bound chains overlap its streams.  It is the controller that gains
+// most: the scan alone on the second stream, with the controller after the
+// join, measured 437.9 against 433.0 us at 16,384 environments (before the
+// split below).
 //
-// Split of the LiDAR channel planes: from kSplitMinBatch environments the
-// scan kernel writes the channels of the 1,536 rays it reads (elevation rows
-// 0..5 of each head) and the plane kernel only the other rows, so the entry
-// reads every LiDAR range from HBM once instead of reading the scan rows
-// twice.  Measured on the entry (one box, outputs bit-equal in every mode;
-// one stream without / with the split, two streams without / with it):
-//    batch    one stream     two streams
-//      256    25.1 / 26.3    41.7 / 44.1
-//      512    32.0 / 31.0    45.6 / 45.7
-//    1,536    59.7 / 55.8    58.5 / 63.0
-//    1,792    65.4 / 62.9    62.7 / 66.5
-//    2,048    76.3 / 70.8    67.8 / 70.4
-//    2,432    88.8 / 86.8    73.7 / 75.4
-//    2,560    88.8 / 86.6    81.2 / 80.2
-//    4,096   128.9 / 123.6  124.1 / 111.7
-//    8,192   230.4 / 222.9  225.3 / 214.5
-//   16,384       --          428.5 / 412.5
-// So batches below kOverlapMinBatch keep one stream (the fork and join cost
-// several microseconds), with the split from kSplitMinBatch; from
-// kOverlapMinBatch two streams, with the split from kSplitOverlapMinBatch
-// (below it the longer scan holds up the second stream).
-constexpr size_t kSplitMinBatch = 512;
-constexpr size_t kSplitOverlapMinBatch = 2560;
-constexpr size_t kOverlapMinBatch = 1792;
+// Split of the LiDAR channel planes: the scan kernel writes the channels of
+// the 1,536 rays it reads (elevation rows 0..5 of each head) and the plane
+// kernel only the other rows, so the entry reads every LiDAR range from HBM
+// once instead of reading the scan rows twice (428.5 -> 412.5 us at 16,384).
+// Without LiDAR channels the second stream runs the onboard kernel instead.
+//
+// Smaller batches take one launch (actor_one_kernel): the fork and join cost
+// several microseconds, and the onboard workgroups are spread over CUs that
+// also run plane workgroups.  Measured on one box, us (before: one stream and
+// three launches up to 1,792 environments, two streams above; one launch; two
+// streams with the split):
+//       64   19.9    8.6    --       2,048   67.6   54.9   70.1
+//      256   22.9   12.7    --       2,560   75.6   70.3   77.2
+//    1,000   42.6   28.0   52.9      3,072   87.4   85.6   87.3
+//    1,500   56.5   41.1   63.2      3,500   97.1   97.6   97.3
+//                                    4,096  112.8  116.4  112.5
+constexpr size_t kOverlapMinBatch = 3072;
 constexpr int kMaxDevices = 64;
 
 struct SideStream {
@@ -2284,33 +2274,6 @@ extern "C" int tb_hip_actor_inputs_device(const float *obs, const float *mission
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     (void)hipGetLastError();
     const bool planes = lidar_channels || camera_luma;
-    SideStream *side = planes && batch_size >= kOverlapMinBatch ? side_stream(s) : nullptr;
-    const bool split = lidar_channels && batch_size >= kSplitMinBatch &&
-                       (!side || batch_size >= kSplitOverlapMinBatch);
-    std::unique_lock<std::mutex> order;
-    if (side) {
-        order = std::unique_lock<std::mutex>(side->order);
-        if (hipEventRecord(side->fork, s) != hipSuccess ||
-            hipStreamWaitEvent(side->stream, side->fork, 0) != hipSuccess)
-            return 0;
-    }
-    if (planes) {
-        ActorRows ar;
-        ar.obs = obs;
-        ar.cameras = cameras;
-        ar.lidar = lidar_channels;
-        ar.luma = camera_luma;
-        ar.batch = batch_size;
-        ar.scan_rows = !split;
-        // One workgroup per CU: the launch asks for more than half of the
-        // CU's 160 KB of LDS, which the kernel does not use (by registers a
-        // CU holds two; one measured 462.7 -> 445.0 us for the entry,
-        // identical outputs: fewer requests in flight keep the write-bound
-        // streams more efficient).
-        constexpr unsigned kOneWorkgroupLds = (160 * 1024 / 2 + 1 + 1023) / 1024 * 1024;
-        actor_stream_kernel<<<batch_size > kMaxBlocks ? kMaxBlocks : (unsigned)batch_size,
-                              kStreamThreads, kOneWorkgroupLds, s>>>(ar);
-    }
     OnboardRows rows;
     rows.obs = reinterpret_cast<const unsigned char *>(obs);
     rows.obs_stride = 4148 * sizeof(float);
@@ -2321,12 +2284,55 @@ extern "C" int tb_hip_actor_inputs_device(const float *obs, const float *mission
     rows.diag = nullptr;
     rows.proprio = proprio;
     rows.mission_vec = mission_vec;
-    rows.lidar = split ? lidar_channels : nullptr;
+    rows.lidar = nullptr;
     rows.batch = batch_size;
-    if (!side) return launch_onboard(rows, s, false);
-    const int ok = launch_onboard(rows, side->stream, false);
-    if (hipEventRecord(side->join, side->stream) != hipSuccess ||
-        hipStreamWaitEvent(s, side->join, 0) != hipSuccess)
+    ActorRows ar;
+    ar.obs = obs;
+    ar.cameras = cameras;
+    ar.lidar = lidar_channels;
+    ar.luma = camera_luma;
+    ar.batch = batch_size;
+    const dim3 onboard_grid = wide_grid((batch_size + 15) / 16);
+    if (!planes) {
+        actor_onboard_kernel<<<onboard_grid, kControlThreads, 0, s>>>(rows);
+        return hipGetLastError() == hipSuccess;
+    }
+    if (batch_size < kOverlapMinBatch) {
+        const unsigned onboard_blocks = (unsigned)((batch_size + 15) / 16);
+        actor_one_kernel<<<onboard_blocks + (unsigned)batch_size, kControlThreads, 0, s>>>(
+            rows, ar, onboard_blocks);
+        return hipGetLastError() == hipSuccess;
+    }
+    SideStream *side = side_stream(s);
+    std::unique_lock<std::mutex> order;
+    if (side) {
+        order = std::unique_lock<std::mutex>(side->order);
+        if (hipEventRecord(side->fork, s) != hipSuccess ||
+            hipStreamWaitEvent(side->stream, side->fork, 0) != hipSuccess)
+            return 0;
+    }
+    // One workgroup per CU: the launch asks for more than half of the
+    // CU's 160 KB of LDS, which the kernel does not use (by registers a
+    // CU holds two; one measured 462.7 -> 445.0 us for the entry,
+    // identical outputs: fewer requests in flight keep the write-bound
+    // streams more efficient).
+    constexpr unsigned kOneWorkgroupLds = (160 * 1024 / 2 + 1 + 1023) / 1024 * 1024;
+    actor_stream_kernel<<<batch_size > kMaxBlocks ? kMaxBlocks : (unsigned)batch_size,
+                          kStreamThreads, kOneWorkgroupLds, s>>>(ar);
+    const hipStream_t beside = side ? side->stream : s;
+    if (lidar_channels) {
+        rows.lidar = lidar_channels;
+        const size_t scan_want = (batch_size + kWavesPerBlock - 1) / kWavesPerBlock;
+        actor_scan_kernel<<<scan_want > kScanBlocks ? kScanBlocks : (unsigned)scan_want,
+                            kBlockThreads, 0, beside>>>(rows);
+        actor_control_kernel<<<wide_grid((batch_size + 63) / 64), kControlThreads, 0, beside>>>(
+            rows);
+    } else {
+        actor_onboard_kernel<<<onboard_grid, kControlThreads, 0, beside>>>(rows);
+    }
+    const int ok = hipGetLastError() == hipSuccess;
+    if (side && (hipEventRecord(side->join, side->stream) != hipSuccess ||
+                 hipStreamWaitEvent(s, side->join, 0) != hipSuccess))
         return 0;
     return ok;
 }
