@@ -651,21 +651,62 @@ __device__ __forceinline__ float quad_pick(int a, float v0, float v1, float v2, 
     return high ? hi : lo;
 }
 
-// The staged inputs that a lane of the control kernel's two chains reads,
+// How the chains are spread over lanes.  QUAD: an environment's four lanes
+// hold one arm each and repeat the shared part, except that independent calls
+// of one function are spread over them and broadcast: the shortest chain, for
+// batches that leave the chip waiting for it.  Otherwise one lane holds the
+// environment and its four arms: 4,100 instead of 10,800 instructions for 64
+// environments, for batches that fill the chip.  Both form every value by the
+// same operations.
+template <bool QUAD>
+constexpr int kArms = QUAD ? 1 : 4;  // arms per lane
+
+// Every arm's value from the lane's own.
+template <bool QUAD>
+__device__ __forceinline__ Quad4 every_arm(const float (&v)[kArms<QUAD>]) {
+    if constexpr (QUAD) return quad_all(v[0]);
+    else return Quad4{{v[0], v[1], v[2], v[3]}};
+}
+// Of four values the one of the lane's arm k.
+template <bool QUAD>
+__device__ __forceinline__ float arm_pick(int a, int k, float v0, float v1, float v2, float v3) {
+    if constexpr (QUAD) return quad_pick(a, v0, v1, v2, v3);
+    else return k == 0 ? v0 : (k == 1 ? v1 : (k == 2 ? v2 : v3));  // k is a constant
+}
+// f of four arguments, or pairs.
+template <bool QUAD, class F>
+__device__ __forceinline__ Quad4 spread(int a, F f, float x0, float x1, float x2, float x3) {
+    if constexpr (QUAD) return quad_all(f(quad_pick(a, x0, x1, x2, x3)));
+    else return Quad4{{f(x0), f(x1), f(x2), f(x3)}};
+}
+template <bool QUAD, class F>
+__device__ __forceinline__ Quad4 spread2(int a, F f, float y0, float y1, float y2, float y3,
+                                         float x0, float x1, float x2, float x3) {
+    if constexpr (QUAD) return quad_all(f(quad_pick(a, y0, y1, y2, y3), quad_pick(a, x0, x1, x2, x3)));
+    else return Quad4{{f(y0, x0), f(y1, x1), f(y2, x2), f(y3, x3)}};
+}
+
+// The staged inputs that a lane of the control kernel's chains reads,
 // taken from LDS all at once: an empty asm on each value keeps the compiler
 // from sinking its read to the first use, where every read would cost the
-// chain its own LDS round trip.  `head` is obs[0..12], `arm` the lane's arm's
-// four values obs[16 + 4 k + a], `tail` obs[40], obs[41], obs[44..47].
+// chain its own LDS round trip.  `head` is obs[0..12], `arm` the four values
+// obs[16 + 4 k + arm] of the lane's arms, `tail` obs[40], obs[41], obs[44..47].
+template <bool QUAD>
 struct ChainInputs {
-    float head[13], arm[4], tail[6], m[10];
+    float head[13], arm[4][kArms<QUAD>], tail[6], m[10];
 };
 
-__device__ __forceinline__ ChainInputs chain_inputs(const float *obs, const float *mission, int a) {
-    ChainInputs in;
+template <bool QUAD>
+__device__ __forceinline__ ChainInputs<QUAD> chain_inputs(const float *obs, const float *mission,
+                                                          int a) {
+    constexpr int K = kArms<QUAD>;
+    ChainInputs<QUAD> in;
 #pragma unroll
     for (int i = 0; i < 13; ++i) in.head[i] = obs[i];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) in.arm[k] = obs[16 + 4 * k + a];
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < K; ++i) in.arm[k][i] = obs[16 + 4 * k + (QUAD ? a : i)];
 #pragma unroll
     for (int k = 0; k < 6; ++k) in.tail[k] = obs[k < 2 ? 40 + k : 42 + k];
 #pragma unroll
@@ -673,7 +714,9 @@ __device__ __forceinline__ ChainInputs chain_inputs(const float *obs, const floa
 #pragma unroll
     for (int i = 0; i < 13; ++i) asm volatile("" : "+v"(in.head[i]));
 #pragma unroll
-    for (int k = 0; k < 4; ++k) asm volatile("" : "+v"(in.arm[k]));
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < K; ++i) asm volatile("" : "+v"(in.arm[k][i]));
 #pragma unroll
     for (int k = 0; k < 6; ++k) asm volatile("" : "+v"(in.tail[k]));
 #pragma unroll
@@ -683,12 +726,15 @@ __device__ __forceinline__ ChainInputs chain_inputs(const float *obs, const floa
 
 // Whether a value that the lane reads is infinite, NaN or not below
 // onboard_math::kTameMax: unless the sum of their squares is below its square.
-__device__ __forceinline__ bool wild_inputs(const ChainInputs &in) {
+template <bool QUAD>
+__device__ __forceinline__ bool wild_inputs(const ChainInputs<QUAD> &in) {
     float s = 0.0f;
 #pragma unroll
     for (int i = 0; i < 13; ++i) s = __builtin_fmaf(in.head[i], in.head[i], s);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) s = __builtin_fmaf(in.arm[k], in.arm[k], s);
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < kArms<QUAD>; ++i) s = __builtin_fmaf(in.arm[k][i], in.arm[k][i], s);
 #pragma unroll
     for (int k = 0; k < 6; ++k) s = __builtin_fmaf(in.tail[k], in.tail[k], s);
 #pragma unroll
@@ -715,38 +761,60 @@ __device__ __forceinline__ onboard_math::Direction ob_direction(float y, float x
 }
 
 // The inputs as the controller reads them (onboard_features.cuh:12-22, 95-99).
-__device__ __forceinline__ void controller_inputs(ChainInputs &in) {
+template <bool QUAD>
+__device__ __forceinline__ void controller_inputs(ChainInputs<QUAD> &in) {
 #pragma unroll
     for (int i = 0; i < 13; ++i) in.head[i] = ob_obs(in.head[i]);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) in.arm[k] = ob_obs(in.arm[k]);
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < kArms<QUAD>; ++i) in.arm[k][i] = ob_obs(in.arm[k][i]);
 #pragma unroll
     for (int k = 0; k < 6; ++k) in.tail[k] = ob_obs(in.tail[k]);
 #pragma unroll
     for (int i = 0; i < 10; ++i) in.m[i] = ob_mission(in.m[i]);
 }
 
-// onboard_features.cuh:25-86 on the four lanes of a quad: lane a evaluates
-// arm a's thrust terms, and the independent calls of one function are spread
-// over the quad and broadcast (the three atanh of the mission offsets; the
-// directions of yaw and of the target bearing; the two hypotenuses and the
-// two atan2f of the aim; eight tanhf in two calls), so a lane makes 8 calls
-// instead of the 25 of the per-environment chain.  Every call takes the
-// arguments the reference's code gives it, and the arm sums are formed in
-// its order from the broadcasts.  Lane a returns features 6a .. 6a + 5 in t,
-// mapped as the reference maps them (NaN -> 0, +-inf -> +-1).
-template <bool TAME>
-__device__ __forceinline__ void tactical_quad(const ChainInputs &in, bool wild, int a,
-                                              float (&t)[6]) {
+// Two of them.
+struct Direction2 {
+    float s0, c0, s1, c1;
+};
+template <bool TAME, bool QUAD>
+__device__ __forceinline__ Direction2 directions(int a, float y0, float x0, float y1, float x1,
+                                                 bool wild) {
+    if constexpr (QUAD) {
+        const onboard_math::Direction d =
+            ob_direction<TAME>(a == 0 ? y0 : y1, a == 0 ? x0 : x1, wild);
+        return Direction2{quad_lane<0>(d.s), quad_lane<0>(d.c), quad_lane<1>(d.s),
+                          quad_lane<1>(d.c)};
+    } else {
+        const onboard_math::Direction d = ob_direction<TAME>(y0, x0, wild),
+                                      e = ob_direction<TAME>(y1, x1, wild);
+        return Direction2{d.s, d.c, e.s, e.c};
+    }
+}
+
+// onboard_features.cuh:25-86.  Every call takes the arguments the reference's
+// code gives it, and the arm sums are formed in its order.  v[0..23] are the
+// features before the reference's last mapping.
+template <bool TAME, bool QUAD>
+__device__ __forceinline__ void tactical_values(const ChainInputs<QUAD> &in, bool wild, int a,
+                                                float (&v)[24]) {
+    constexpr int K = kArms<QUAD>;
     const float pi = kPi;
     const float *o = in.head, *m = in.m;
     const float o44 = in.tail[2], o45 = in.tail[3], o46 = in.tail[4], o47 = in.tail[5];
-    const float spool_a = ob_clamp<TAME>(in.arm[0], 0.0f, 1.0f);
-    const float thrust_a = 0.036f + 0.964f * spool_a;
-    const float ci_a = onboard_math::cos_float<TAME>(in.arm[3]);
-    const Quad4 spool = quad_all(spool_a);
-    const Quad4 fz = quad_all(thrust_a * in.arm[2] * ci_a);
-    const Quad4 tz = quad_all(thrust_a * in.arm[1] * ci_a);
+    float spool_a[K], fz_a[K], tz_a[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        spool_a[i] = ob_clamp<TAME>(in.arm[0][i], 0.0f, 1.0f);
+        const float thrust_a = 0.036f + 0.964f * spool_a[i];
+        const float ci_a = onboard_math::cos_float<TAME>(in.arm[3][i]);
+        fz_a[i] = thrust_a * in.arm[2][i] * ci_a;
+        tz_a[i] = thrust_a * in.arm[1][i] * ci_a;
+    }
+    const Quad4 spool = every_arm<QUAD>(spool_a), fz = every_arm<QUAD>(fz_a),
+                tz = every_arm<QUAD>(tz_a);
     float tau_z = 0.0f, spool_mean = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -754,7 +822,6 @@ __device__ __forceinline__ void tactical_quad(const ChainInputs &in, bool wild, 
         spool_mean += spool.v[i];
     }
     spool_mean *= 0.25f;
-    float v[24];
     v[0] = fz.v[1] - fz.v[3];
     v[1] = fz.v[2] - fz.v[0];
     v[2] = 0.5f * tau_z;
@@ -767,17 +834,15 @@ __device__ __forceinline__ void tactical_quad(const ChainInputs &in, bool wild, 
     const float ct = ob_clamp<TAME>(1.0f - 2.0f * (qx * qx + qy * qy), -1.0f, 1.0f);
     const float bx_x = 1.0f - 2.0f * (qy * qy + qz * qz);
     const float bx_y = 2.0f * (qx * qy + qw * qz);
-    // rx, ry, rz on lanes 0, 1, 2 (lane 3 repeats rz).
-    const float r_a = onboard_math::atanh_float(ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]),
-                                                               -0.995f, 0.995f)) * 20.0f;
-    const float rx = quad_lane<0>(r_a), ry = quad_lane<1>(r_a), rz = quad_lane<2>(r_a);
-    // Sine and cosine of yaw = atan2(bx_y, bx_x) on lane 0 and of the target
-    // bearing atan2(ry, rx) on the others, from their components; the angles
-    // themselves are used nowhere else.
-    const float ty_a = a == 0 ? bx_y : ry, tx_a = a == 0 ? bx_x : rx;
-    const onboard_math::Direction at_a = ob_direction<TAME>(ty_a, tx_a, wild);
-    const float cy = quad_lane<0>(at_a.c), sy = quad_lane<0>(at_a.s);
-    const float cb = quad_lane<1>(at_a.c), sb = quad_lane<1>(at_a.s);
+    const Quad4 offsets = spread<QUAD>(
+        a, [](float x) { return onboard_math::atanh_float(ob_clamp<TAME>(x, -0.995f, 0.995f)); },
+        m[7], m[8], m[9], m[9]);
+    const float rx = offsets.v[0] * 20.0f, ry = offsets.v[1] * 20.0f, rz = offsets.v[2] * 20.0f;
+    // Sine and cosine of yaw = atan2(bx_y, bx_x) and of the target bearing
+    // atan2(ry, rx), from their components; the angles themselves are used
+    // nowhere else.
+    const Direction2 dir = directions<TAME, QUAD>(a, bx_y, bx_x, ry, rx, wild);
+    const float cy = dir.c0, sy = dir.s0, cb = dir.c1, sb = dir.s1;
     v[8] = cy * bz_y - sy * bz_x;
     v[9] = -sy * bz_y - cy * bz_x;
     v[10] = ct;
@@ -794,25 +859,23 @@ __device__ __forceinline__ void tactical_quad(const ChainInputs &in, bool wild, 
     const float bx = wx + 2.0f * (uy * cz - uz * cyq);
     const float by = wy + 2.0f * (uz * cx - ux * cz);
     const float bz = wz + 2.0f * (ux * cyq - uy * cx);
-    // The hypotenuse of (rx, ry) on lane 0, of (bx, by) on the others; then
-    // the aim's azimuth on lane 0 and elevation on the others.
-    const float hy_a = ob_hypot<TAME>(a == 0 ? rx : bx, a == 0 ? ry : by);
-    const float h_rxy = quad_lane<0>(hy_a), h_bxy = quad_lane<1>(hy_a);
-    const float aim_a = atan2f(a == 0 ? by : bz, a == 0 ? bx : fmaxf(h_bxy, 0.2f));
-    const float az = ob_clamp<TAME>(quad_lane<0>(aim_a), pi / 12.0f, pi * 5.0f / 12.0f);
-    const float el = ob_clamp<TAME>(quad_lane<1>(aim_a), -pi / 6.0f, pi / 6.0f);
+    const Quad4 hyp = spread2<QUAD>(a, [](float x, float y) { return ob_hypot<TAME>(x, y); }, rx, bx,
+                                    bx, bx, ry, by, by, by);
+    const float h_rxy = hyp.v[0], h_bxy = fmaxf(hyp.v[1], 0.2f);
+    const Quad4 aim = spread2<QUAD>(a, [](float y, float x) { return atan2f(y, x); }, by, bz, bz, bz,
+                                    bx, h_bxy, h_bxy, h_bxy);
+    const float az = ob_clamp<TAME>(aim.v[0], pi / 12.0f, pi * 5.0f / 12.0f);
+    const float el = ob_clamp<TAME>(aim.v[1], -pi / 6.0f, pi / 6.0f);
     const float err = ob_hypot<TAME>(az - o44, el - o45);
-    const float th1 = tanhf(quad_pick(a, (cy * rx + sy * ry) * 0.08f, (-sy * rx + cy * ry) * 0.08f,
-                                      rz * 0.12f, h_rxy * 0.05f));
-    const float th2 = tanhf(quad_pick(a, (cy * o[3] + sy * o[4]) * 0.15f,
-                                      (-sy * o[3] + cy * o[4]) * 0.15f, err * 2.0f, 0.0f));
-    v[12] = quad_lane<0>(th1);
-    v[13] = quad_lane<1>(th1);
-    v[14] = quad_lane<2>(th1);
-    v[15] = quad_lane<3>(th1);
-    v[16] = quad_lane<0>(th2);
-    v[17] = quad_lane<1>(th2);
-    v[21] = quad_lane<2>(th2);
+    const Quad4 th1 = spread<QUAD>(a, [](float x) { return tanhf(x); }, (cy * rx + sy * ry) * 0.08f,
+                                   (-sy * rx + cy * ry) * 0.08f, rz * 0.12f, h_rxy * 0.05f);
+    const Quad4 th2 = spread<QUAD>(a, [](float x) { return tanhf(x); }, (cy * o[3] + sy * o[4]) * 0.15f,
+                                   (-sy * o[3] + cy * o[4]) * 0.15f, err * 2.0f, 0.0f);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[12 + i] = th1.v[i];
+    v[16] = th2.v[0];
+    v[17] = th2.v[1];
+    v[21] = th2.v[2];
     v[18] = expf(-fmaxf(o[2] - 0.62f, 0.0f));
     v[19] = div_const(az - pi * 0.25f, pi / 6.0f);
     v[20] = div_const(el, pi / 6.0f);
@@ -821,11 +884,12 @@ __device__ __forceinline__ void tactical_quad(const ChainInputs &in, bool wild, 
     v[22] = ready ? 1.0f : -1.0f;
     // sin(bearing - pi/4 - yaw) by the addition theorem.
     v[23] = ((sb * cy - cb * sy) - (cb * cy + sb * sy)) * 0x1.6a09e6p-1f;  // 1 / sqrt 2
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        const float x = quad_pick(a, v[k], v[6 + k], v[12 + k], v[18 + k]);
-        t[k] = TAME ? x : finite_as(x, 1.0f);
-    }
+}
+
+// The reference's last mapping (NaN -> 0, +-inf -> +-1).
+template <bool TAME>
+__device__ __forceinline__ float tactical_out(float x) {
+    return TAME ? x : finite_as(x, 1.0f);
 }
 
 // The mission's flags (onboard_features.cuh:107-109, 126-136, 433-437).
@@ -871,27 +935,26 @@ __device__ __forceinline__ Goal goal_of(const MissionFlags &f, float px, float p
     return g;
 }
 
-// One lane's share of the flight controls: its arm's throttle, outer and
+// One lane's share of the flight controls: its arms' throttle, outer and
 // inner commands.
+template <bool QUAD>
 struct ArmOutputs {
-    float throttle, outer, inner;
+    float throttle[kArms<QUAD>], outer[kArms<QUAD>], inner[kArms<QUAD>];
 };
 
 // The flight controller: onboard_features.cuh:88-432 without the cannon, with
-// the LiDAR passes replaced by `scan`, on the four lanes of a quad: lane a
-// evaluates arm a's terms (the two per-arm loops, :114-125 and :376-391) and
-// the four lanes repeat the shared chain, except that independent calls of
-// one function are spread over the quad (three atan2, three atanh, two
-// directions) and their results broadcast.  The arm sums and the running
-// maximum are formed in the reference's order from quad broadcasts, so every
-// value is the one the per-environment code forms.  The cannon and the BWB
-// law share nothing with this chain but its inputs: gunnery_quad forms them
-// on the waves of the tactical features, which are done far earlier.
+// the LiDAR passes replaced by the scan's result (the two per-arm loops are
+// :114-125 and :376-391).  The arm sums and the running maximum are formed in
+// the reference's order, so every value is the one its code forms.  The
+// cannon and the BWB law share nothing with this chain but its inputs: other
+// waves form them (gunnery_values).
 // `fetch` returns the scan result; everything that does not depend on it is
 // formed before it is called.
-template <bool TAME, class Fetch>
-__device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, bool wild,
-                                                  const MissionFlags &f, int a, Fetch fetch) {
+template <bool TAME, bool QUAD, class Fetch>
+__device__ __forceinline__ ArmOutputs<QUAD> flight_values(const ChainInputs<QUAD> &in, bool wild,
+                                                          const MissionFlags &f, int a,
+                                                          Fetch fetch) {
+    constexpr int K = kArms<QUAD>;
     using onboard_math::quotient;
     const float pi = kPi;
     const float max_installed = 294.2f * 0.85f;
@@ -910,13 +973,19 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, bool wi
     const float ox = o[10], oy = o[11], oz = o[12];
     const float omega_norm = ob_norm3<TAME>(ox, oy, oz);
 
-    // Arm a of the four (this lane's); the quad exchanges the arm forces.
-    const float spool = ob_clamp<TAME>(in.arm[0], 0.0f, 1.0f);
-    const float thrust = max_installed * (idle_frac + (1.0f - idle_frac) * spool);
-    const float outer = ob_atan2<TAME>(in.arm[1], in.arm[2]);
-    const onboard_math::Direction o_sc = ob_direction<TAME>(in.arm[1], in.arm[2], wild);
-    const float c_inner = onboard_math::cos_float<TAME>(in.arm[3]);
-    const Quad4 fz = quad_all(thrust * o_sc.c * c_inner), ft = quad_all(thrust * o_sc.s * c_inner);
+    // This lane's arms; then every arm's forces.
+    float spool[K], thrust[K], outer[K], fz_a[K], ft_a[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        spool[i] = ob_clamp<TAME>(in.arm[0][i], 0.0f, 1.0f);
+        thrust[i] = max_installed * (idle_frac + (1.0f - idle_frac) * spool[i]);
+        outer[i] = ob_atan2<TAME>(in.arm[1][i], in.arm[2][i]);
+        const onboard_math::Direction o_sc = ob_direction<TAME>(in.arm[1][i], in.arm[2][i], wild);
+        const float c_inner = onboard_math::cos_float<TAME>(in.arm[3][i]);
+        fz_a[i] = thrust[i] * o_sc.c * c_inner;
+        ft_a[i] = thrust[i] * o_sc.s * c_inner;
+    }
+    const Quad4 fz = every_arm<QUAD>(fz_a), ft = every_arm<QUAD>(ft_a);
     float total_fz = 0.0f, jammed_yaw_ft = 0.0f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -937,18 +1006,17 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, bool wi
     const bool heavy_cargo = (int)f.cargo & (int)payload;
     const bool landing_like = (int)f.landing | (int)heavy_cargo;
 
-    // The mission offsets, one per lane; then yaw, the opponent bearing and
-    // the goal bearing.
-    const Quad4 offsets = quad_all(onboard_math::atanh_float(
-        ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]), -0.9995f, 0.9995f)));
+    const Quad4 offsets = spread<QUAD>(
+        a, [](float x) { return onboard_math::atanh_float(ob_clamp<TAME>(x, -0.9995f, 0.9995f)); },
+        m[7], m[8], m[9], m[9]);
     const float relx = offsets.v[0] * 20.0f;
     const float rely = offsets.v[1] * 20.0f;
     const float relz = offsets.v[2] * 20.0f;
     const Goal goal = goal_of(f, px, py, pz, relx, rely, relz);
     const float tx = goal.x, ty = goal.y, tz = goal.z;
     const float dx_opp = tx - px, dy_opp = ty - py;
-    const Quad4 angles = quad_all(ob_atan2<TAME>(quad_pick(a, r10, m[1], dy_opp, dy_opp),
-                                                 quad_pick(a, r00, m[2], dx_opp, dx_opp)));
+    const Quad4 angles = spread2<QUAD>(a, [](float y, float x) { return ob_atan2<TAME>(y, x); },
+                                       r10, m[1], dy_opp, dy_opp, r00, m[2], dx_opp, dx_opp);
     const float yaw = angles.v[0], opp_bearing = angles.v[1], raw_bearing = angles.v[2];
 
     float ex = tx, ey = ty, ez = tz;
@@ -1018,12 +1086,12 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, bool wi
 
     // Sine and cosine of yaw and of the closest return's bearing from their
     // components (a rotation's rows; a range inside the window).
-    const onboard_math::Direction sc = ob_direction<TAME>(
-        a == 0 ? r10 : scan.min_r_dy, a == 0 ? r00 : scan.min_r_dx, wild);
-    const float cyaw = quad_lane<0>(sc.c), syaw = quad_lane<0>(sc.s);
+    const Direction2 dir =
+        directions<TAME, QUAD>(a, r10, r00, scan.min_r_dy, scan.min_r_dx, wild);
+    const float cyaw = dir.c0, syaw = dir.s0;
 
     const bool avoid = (int)f.dodge & (int)(scan.min_r < 7.5f);
-    const float away_x = -quad_lane<1>(sc.s) * 2.2f, away_y = quad_lane<1>(sc.c) * 2.2f;
+    const float away_x = -dir.s1 * 2.2f, away_y = dir.c1 * 2.2f;
     const float avoid_x = avoid ? away_x : 0.0f, avoid_y = avoid ? away_y : 0.0f;
     const float min_dx_c = scan.min_dx_c;
     const int cluster_count = scan.cluster_count;
@@ -1140,10 +1208,7 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, bool wi
     const float tau_y_cmd = ob_clamp<TAME>(
         95.0f * e_ry - 64.0f * oy - 0.90f * tau_y_net - tau_y_par, -max_txy, max_txy);
     const float tau_z_cmd = ob_clamp<TAME>(22.0f * yaw_err - 18.0f * oz, -70.0f, 70.0f);
-    // {q - ty, q + tx, q + ty, q - tx}[a]; q - t and q + (-t) are the same
-    // IEEE operation.
     const float half_tx = tau_x_cmd * 0.5f, half_ty = tau_y_cmd * 0.5f;
-    const float fz_cmd = 0.25f * fz_des + quad_pick(a, -half_ty, half_tx, half_ty, -half_tx);
     const float yaw_ft = (tau_z_cmd - 0.40f * jammed_yaw_ft) * 0.25f;
     const float fx_outer = ft.v[3] - ft.v[1];
     const float fy_outer = ft.v[0] - ft.v[2];
@@ -1155,65 +1220,79 @@ __device__ __forceinline__ ArmOutputs flight_quad(const ChainInputs &in, bool wi
     const float spool_gain = f.turbine_out ? 10.5f : std_gain;
     const bool land_idle = (int)f.landing & (int)(pz <= 0.638f) & (int)(up_horiz < 0.85f) &
                            (int)(fabsf(vz) < 0.20f);
-    const float sin_alpha =
-        ob_clamp<TAME>(quotient<TAME>(yaw_ft, fmaxf(thrust, 30.0f)), -0.35f, 0.35f);
-    const float yaw_alpha = asinf(sin_alpha);
-    float outer_cmd =
-        ob_clamp<TAME>(6.5f * ob_wrap<TAME>(yaw_alpha, outer), -outer_limit, outer_limit);
-    const float urx = quad_pick(a, 1.0f, 0.0f, -1.0f, 0.0f);
-    const float ury = quad_pick(a, 0.0f, 1.0f, 0.0f, -1.0f);
-    const float fr_req = 0.5f * (fx_rem * urx + fy_rem * ury);
-    const float sin_in = ob_clamp<TAME>(quotient<TAME>(fr_req, fmaxf(thrust, 40.0f)),
-                                        -max_sin_inner, max_sin_inner);
-    float inner_cmd = ob_clamp<TAME>(asinf(sin_in), -inner_limit * 0.90f, inner_limit * 0.90f);
-    // cos(yaw_alpha) cos(inner_cmd), both arcsines (|sin_in| <= 0.44, so the
-    // limit on inner_cmd is never met): one square root of the product of
-    // the two squared cosines, which is at least 0.70.
-    const float nominal_cos =
-        fmaxf(__builtin_amdgcn_sqrtf(__builtin_fmaf(-sin_alpha, sin_alpha, 1.0f) *
-                                     __builtin_fmaf(-sin_in, sin_in, 1.0f)), 0.70f);
-    const float lift_thrust = quotient<TAME>(fmaxf(fz_cmd, 0.0f), nominal_cos);
     const float idle_thrust = 0.15f * weight * 0.25f;
-    const float target_thrust = land_idle ? idle_thrust : lift_thrust;
-    const float u_des = ob_clamp<TAME>(
-        div_const(target_thrust - min_thrust, max_installed - min_thrust), 0.0f, 1.0f);
-    const float u_raw = u_des + spool_gain * (u_des - spool);
+    float outer_cmd[K], inner_cmd[K], u_raw[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        // {q - ty, q + tx, q + ty, q - tx}[arm]; q - t and q + (-t) are the
+        // same IEEE operation.
+        const float fz_cmd =
+            0.25f * fz_des + arm_pick<QUAD>(a, i, -half_ty, half_tx, half_ty, -half_tx);
+        const float sin_alpha =
+            ob_clamp<TAME>(quotient<TAME>(yaw_ft, fmaxf(thrust[i], 30.0f)), -0.35f, 0.35f);
+        const float yaw_alpha = asinf(sin_alpha);
+        outer_cmd[i] =
+            ob_clamp<TAME>(6.5f * ob_wrap<TAME>(yaw_alpha, outer[i]), -outer_limit, outer_limit);
+        const float urx = arm_pick<QUAD>(a, i, 1.0f, 0.0f, -1.0f, 0.0f);
+        const float ury = arm_pick<QUAD>(a, i, 0.0f, 1.0f, 0.0f, -1.0f);
+        const float fr_req = 0.5f * (fx_rem * urx + fy_rem * ury);
+        const float sin_in = ob_clamp<TAME>(quotient<TAME>(fr_req, fmaxf(thrust[i], 40.0f)),
+                                            -max_sin_inner, max_sin_inner);
+        inner_cmd[i] = ob_clamp<TAME>(asinf(sin_in), -inner_limit * 0.90f, inner_limit * 0.90f);
+        // cos(yaw_alpha) cos(inner_cmd), both arcsines (|sin_in| <= 0.44, so
+        // the limit on inner_cmd is never met): one square root of the
+        // product of the two squared cosines, which is at least 0.70.
+        const float nominal_cos =
+            fmaxf(__builtin_amdgcn_sqrtf(__builtin_fmaf(-sin_alpha, sin_alpha, 1.0f) *
+                                         __builtin_fmaf(-sin_in, sin_in, 1.0f)), 0.70f);
+        const float lift_thrust = quotient<TAME>(fmaxf(fz_cmd, 0.0f), nominal_cos);
+        const float target_thrust = land_idle ? idle_thrust : lift_thrust;
+        const float u_des = ob_clamp<TAME>(
+            div_const(target_thrust - min_thrust, max_installed - min_thrust), 0.0f, 1.0f);
+        u_raw[i] = u_des + spool_gain * (u_des - spool[i]);
+    }
     // The reference's running maximum over arms 0..3, from -inf.
-    const Quad4 u_all = quad_all(u_raw);
+    const Quad4 u_all = every_arm<QUAD>(u_raw);
     float max_raw = -__builtin_huge_valf();
 #pragma unroll
     for (int i = 0; i < 4; ++i) max_raw = fmaxf(max_raw, u_all.v[i]);
     const float excess = ob_clamp<TAME>(max_raw - 1.0f, 0.0f, urgent_climb ? 0.10f : 0.45f);
-    float throttle = ob_clamp<TAME>(u_raw - (need_headroom ? excess : 0.0f), 0.0f, 1.0f);
+    const float shed = need_headroom ? excess : 0.0f;
     const bool inv_mode = ct < 0.20f;
     const float inv_rx = te_norm > 1.0e-5f ? e_rx : tilt;
     const float tx_inv = 130.0f * inv_rx - 52.0f * ox;
     const float ty_inv = 130.0f * e_ry - 52.0f * oy;
-    const float arm_mom = quad_pick(a, -ty_inv, tx_inv, ty_inv, -tx_inv);
-    const float inv_throttle = arm_mom > 12.0f ? 0.58f : 0.0f;
-    const float inv_outer = ob_clamp<TAME>(-outer * 6.0f, -outer_limit, outer_limit);
-    throttle = inv_mode ? inv_throttle : throttle;
-    outer_cmd = inv_mode ? inv_outer : outer_cmd;
-    inner_cmd = inv_mode ? 0.0f : inner_cmd;
-    ArmOutputs out;
-    out.throttle = ob_clamp<TAME>(throttle * 2.0f - 1.0f, -1.0f, 1.0f);
-    out.outer = ob_clamp<TAME>(outer_cmd * (1.0f / outer_limit), -1.0f, 1.0f);
-    out.inner = ob_clamp<TAME>(div_const(inner_cmd, inner_limit), -1.0f, 1.0f);
+    ArmOutputs<QUAD> out;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        float throttle = ob_clamp<TAME>(u_raw[i] - shed, 0.0f, 1.0f);
+        const float arm_mom = arm_pick<QUAD>(a, i, -ty_inv, tx_inv, ty_inv, -tx_inv);
+        const float inv_throttle = arm_mom > 12.0f ? 0.58f : 0.0f;
+        const float inv_outer = ob_clamp<TAME>(-outer[i] * 6.0f, -outer_limit, outer_limit);
+        throttle = inv_mode ? inv_throttle : throttle;
+        const float outer_out = inv_mode ? inv_outer : outer_cmd[i];
+        const float inner_out = inv_mode ? 0.0f : inner_cmd[i];
+        out.throttle[i] = ob_clamp<TAME>(throttle * 2.0f - 1.0f, -1.0f, 1.0f);
+        out.outer[i] = ob_clamp<TAME>(outer_out * (1.0f / outer_limit), -1.0f, 1.0f);
+        out.inner[i] = ob_clamp<TAME>(div_const(inner_out, inner_limit), -1.0f, 1.0f);
+    }
     return out;
 }
 
 // The cannon (onboard_features.cuh:393-430) and, for BWB missions, the BWB
 // law, which replaces every prior value (:433-510): the cannon's azimuth,
-// elevation and fire (identical in the four lanes) and, for a BWB mission,
-// lane a's arm commands.
+// elevation and fire (identical in a quad's lanes) and, for a BWB mission,
+// the lane's arm commands.
+template <bool QUAD>
 struct GunOutputs {
     float az, el, fire;
-    ArmOutputs arm;  // BWB missions only
+    ArmOutputs<QUAD> arm;  // BWB missions only
 };
 
-template <bool TAME>
-__device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool wild,
-                                                   const MissionFlags &f, int a) {
+template <bool TAME, bool QUAD>
+__device__ __forceinline__ GunOutputs<QUAD> gunnery_values(const ChainInputs<QUAD> &in, bool wild,
+                                                           const MissionFlags &f, int a) {
+    constexpr int K = kArms<QUAD>;
     using onboard_math::quotient;
     const float pi = kPi;
     const float gravity = 9.80665f;
@@ -1233,8 +1312,9 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool w
     const float ct = ob_clamp<TAME>(r22, -1.0f, 1.0f);
     const bool inv_mode = ct < 0.20f;
 
-    const Quad4 offsets = quad_all(onboard_math::atanh_float(
-        ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]), -0.9995f, 0.9995f)));
+    const Quad4 offsets = spread<QUAD>(
+        a, [](float x) { return onboard_math::atanh_float(ob_clamp<TAME>(x, -0.9995f, 0.9995f)); },
+        m[7], m[8], m[9], m[9]);
     const Goal goal = goal_of(f, px, py, pz, offsets.v[0] * 20.0f, offsets.v[1] * 20.0f,
                               offsets.v[2] * 20.0f);
     // The aim point in the body frame.
@@ -1254,9 +1334,9 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool w
     // (the ground track above 2.5 m/s, else yaw).
     const float gs = ob_hypot<TAME>(vx, vy);
     const float course_y = gs > 2.5f ? vy : r10, course_x = gs > 2.5f ? vx : r00;
-    const Quad4 angles = quad_all(ob_atan2<TAME>(
-        quad_pick(a, aim_by, aim_bz, r21, course_y),
-        quad_pick(a, aim_bx, fmaxf(ob_hypot<TAME>(aim_bx, aim_by), 0.2f), r22, course_x)));
+    const auto atan2_of = [](float y, float x) { return ob_atan2<TAME>(y, x); };
+    const Quad4 angles = spread2<QUAD>(a, atan2_of, aim_by, aim_bz, r21, course_y, aim_bx,
+                                       fmaxf(ob_hypot<TAME>(aim_bx, aim_by), 0.2f), r22, course_x);
     const float des_cannon_az =
         ob_clamp<TAME>(angles.v[0], cannon_az_ctr - cannon_az_half, cannon_az_ctr + cannon_az_half);
     const float des_cannon_el = ob_clamp<TAME>(angles.v[1], -cannon_el_lim, cannon_el_lim);
@@ -1270,18 +1350,19 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool w
     const float aimed_az =
         ob_clamp<TAME>(div_const(des_cannon_az - cannon_az_ctr, cannon_az_half), -1.0f, 1.0f);
     const float aimed_el = ob_clamp<TAME>(div_const(des_cannon_el, cannon_el_lim), -1.0f, 1.0f);
-    GunOutputs out;
+    GunOutputs<QUAD> out;
     out.az = cannon ? aimed_az : 0.0f;
     out.az = inv_mode ? -1.0f : out.az;
     out.el = cannon ? aimed_el : 0.0f;
     out.fire = fire ? 0.8f : -0.8f;
-    out.arm = ArmOutputs{0.0f, 0.0f, 0.0f};
+    out.arm = ArmOutputs<QUAD>{};
     if (!f.bwb) return out;
 
     const float vb_x = r00 * vx + r10 * vy + r20 * vz;
     const float vb_y = r01 * vx + r11 * vy + r21 * vz;
-    const Quad4 b_offsets = quad_all(onboard_math::atanh_float(
-        ob_clamp<TAME>(quad_pick(a, m[7], m[8], m[9], m[9]), -0.9999f, 0.9999f)));
+    const Quad4 b_offsets = spread<QUAD>(
+        a, [](float x) { return onboard_math::atanh_float(ob_clamp<TAME>(x, -0.9999f, 0.9999f)); },
+        m[7], m[8], m[9], m[9]);
     const float brx = b_offsets.v[0] * 20.0f;
     const float bry = b_offsets.v[1] * 20.0f;
     const float brz = b_offsets.v[2] * 20.0f;
@@ -1313,10 +1394,8 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool w
     const float bbx = r00 * bax + r10 * bay + r20 * baz;
     const float bby = r01 * bax + r11 * bay + r21 * baz;
     const float bbz = r02 * bax + r12 * bay + r22 * baz;
-    const Quad4 b_angles = quad_all(ob_atan2<TAME>(
-        quad_pick(a, gy, climb_des, bby, bbz),
-        quad_pick(a, gx, fmaxf(gs, 14.0f), fmaxf(bbx, 0.2f),
-                  fmaxf(ob_hypot<TAME>(bbx, bby), 0.2f))));
+    const Quad4 b_angles = spread2<QUAD>(a, atan2_of, gy, climb_des, bby, bbz, gx, fmaxf(gs, 14.0f),
+                                         fmaxf(bbx, 0.2f), fmaxf(ob_hypot<TAME>(bbx, bby), 0.2f));
     const float desired_yaw_b = b_angles.v[0], gamma_des = b_angles.v[1];
     const float b_az = ob_clamp<TAME>(b_angles.v[2], -pi / 6.0f, pi / 6.0f);
     const float b_el = ob_clamp<TAME>(b_angles.v[3], -cannon_el_lim, cannon_el_lim);
@@ -1333,7 +1412,6 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool w
                                         -0.45f, 0.45f);
     const float u0 = ob_clamp<TAME>(u_coll + diff_u, 0.05f, 1.0f);
     const float u1 = ob_clamp<TAME>(u_coll - diff_u, 0.05f, 1.0f);
-    const float throttle = (a & 1) ? u1 : u0;
     const float pitch_up = asinf(ob_clamp<TAME>(r20, -1.0f, 1.0f));
     const float climb_err = climb_des - vz;
     const onboard_math::Direction bank = ob_direction<TAME>(r21, r22, wild);
@@ -1352,7 +1430,6 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool w
     const float gimbal = pi / 6.0f;
     const float inner0 = ob_clamp<TAME>(0.85f * (q_up + o[11]) + 0.03f, -gimbal, gimbal);
     const float inner1 = ob_clamp<TAME>(-0.65f * (r_left - o[12]) - 0.025f * vb_y, -gimbal, gimbal);
-    const float inner_cmd = quad_pick(a, inner0, inner1, 0.0f, 0.0f);
     const float b_err = ob_hypot<TAME>(ob_wrap<TAME>(b_az, o44), b_el - o45);
     const bool b_fire = (int)loaded & (int)(b_err < 0.045f) & (int)(bdist < 165.0f) &
                         (int)(bbx > 0.0f);
@@ -1361,9 +1438,14 @@ __device__ __forceinline__ GunOutputs gunnery_quad(const ChainInputs &in, bool w
     out.az = f.arena ? b_norm_az : 0.0f;
     out.el = f.arena ? b_norm_el : 0.0f;
     out.fire = b_fire ? 0.8f : -0.8f;
-    out.arm.throttle = ob_clamp<TAME>(throttle * 2.0f - 1.0f, -1.0f, 1.0f);
-    out.arm.outer = 0.0f;
-    out.arm.inner = ob_clamp<TAME>(div_const(inner_cmd, inner_limit), -1.0f, 1.0f);
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const float throttle = arm_pick<QUAD>(a, i, u0, u1, u0, u1);
+        const float inner_cmd = arm_pick<QUAD>(a, i, inner0, inner1, 0.0f, 0.0f);
+        out.arm.throttle[i] = ob_clamp<TAME>(throttle * 2.0f - 1.0f, -1.0f, 1.0f);
+        out.arm.outer[i] = 0.0f;
+        out.arm.inner[i] = ob_clamp<TAME>(div_const(inner_cmd, inner_limit), -1.0f, 1.0f);
+    }
     return out;
 }
 
@@ -1632,6 +1714,31 @@ __device__ __forceinline__ void stage_result(Stage<N> &stage, int e, const ScanR
     sc[6] = __int_as_float(r.cluster_count);
 }
 
+template <int N>
+__device__ __forceinline__ ScanResult staged_result(const Stage<N> &stage, int e) {
+    const float *sc = stage.scan[e];
+    ScanResult s;
+    s.min_r = sc[0];
+    s.min_r_dx = sc[1];
+    s.min_r_dy = sc[2];
+    s.min_dx_c = sc[3];
+    s.cluster_y_sum = sc[4];
+    s.min_ray = __float_as_int(sc[5]);
+    s.cluster_count = __float_as_int(sc[6]);
+    // Read from LDS at once, like the other inputs.
+    asm volatile("" : "+v"(s.min_r), "+v"(s.min_r_dx), "+v"(s.min_r_dy), "+v"(s.min_dx_c),
+                 "+v"(s.cluster_y_sum), "+v"(s.min_ray), "+v"(s.cluster_count));
+    return s;
+}
+
+__device__ __forceinline__ void store_scan_diag(float *d, const ScanResult &s) {
+    d[0] = s.min_r;
+    d[1] = (float)s.min_ray;
+    d[2] = s.min_dx_c;
+    d[3] = (float)s.cluster_count;
+    d[4] = s.cluster_y_sum;
+}
+
 // Where an environment's tactical and prior values go: their rows, and for
 // the actor their copies in proprio and mission_vec.
 struct OutputRows {
@@ -1640,17 +1747,17 @@ struct OutputRows {
         : tactical(rows.tactical + env * 24), prior(rows.prior + env * 15),
           proprio(rows.proprio ? rows.proprio + env * 91 + 52 : nullptr),
           mission_vec(rows.proprio ? rows.mission_vec + env * 49 + 10 : nullptr) {}
-    __device__ __forceinline__ void arm(int a, const ArmOutputs &n) const {
-        prior[a] = n.throttle;
-        prior[4 + a] = n.outer;
-        prior[8 + a] = n.inner;
+    __device__ __forceinline__ void arm(int a, const ArmOutputs<true> &n) const {
+        prior[a] = n.throttle[0];
+        prior[4 + a] = n.outer[0];
+        prior[8 + a] = n.inner[0];
         if (proprio) {
-            proprio[24 + a] = n.throttle;
-            proprio[28 + a] = n.outer;
-            proprio[32 + a] = n.inner;
-            mission_vec[24 + a] = n.throttle;
-            mission_vec[28 + a] = n.outer;
-            mission_vec[32 + a] = n.inner;
+            proprio[24 + a] = n.throttle[0];
+            proprio[28 + a] = n.outer[0];
+            proprio[32 + a] = n.inner[0];
+            mission_vec[24 + a] = n.throttle[0];
+            mission_vec[28 + a] = n.outer[0];
+            mission_vec[32 + a] = n.inner[0];
         }
     }
 };
@@ -1663,13 +1770,21 @@ __device__ __forceinline__ void support_wave(const OnboardRows &rows, size_t bas
     const int a = lane & 3, slot = first + (lane >> 2);
     const size_t env = base + (size_t)slot;
     if (env >= rows.batch) return;
-    ChainInputs in = chain_inputs(stage.obs[slot], stage.mission[slot], a);
+    ChainInputs<true> in = chain_inputs<true>(stage.obs[slot], stage.mission[slot], a);
     const bool wild = wild_inputs(in), tame = __builtin_amdgcn_ballot_w64(wild) == 0;
     const OutputRows out(rows, env);
     // Lane a of the quad writes features 6a .. 6a + 5.
     float t[6];
-    if (tame) tactical_quad<true>(in, wild, a, t);
-    else tactical_quad<false>(in, wild, a, t);
+    {
+        float v[24];
+        if (tame) tactical_values<true, true>(in, wild, a, v);
+        else tactical_values<false, true>(in, wild, a, v);
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const float x = quad_pick(a, v[k], v[6 + k], v[12 + k], v[18 + k]);
+            t[k] = tactical_out<false>(x);
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 6; ++i) out.tactical[6 * a + i] = t[i];
     if (out.proprio) {
@@ -1681,8 +1796,8 @@ __device__ __forceinline__ void support_wave(const OnboardRows &rows, size_t bas
     }
     if (!tame) controller_inputs(in);
     const MissionFlags f = mission_flags(in.m);
-    const GunOutputs g =
-        tame ? gunnery_quad<true>(in, wild, f, a) : gunnery_quad<false>(in, wild, f, a);
+    const GunOutputs<true> g = tame ? gunnery_values<true, true>(in, wild, f, a)
+                                    : gunnery_values<false, true>(in, wild, f, a);
     if (f.bwb) out.arm(a, g.arm);
     if (a == 0) {
         out.prior[12] = g.az;
@@ -1707,37 +1822,72 @@ __device__ __forceinline__ void flight_wave(const OnboardRows &rows, size_t base
     const int a = lane & 3, slot = first + (lane >> 2);
     const size_t env = base + (size_t)slot;
     if (env >= rows.batch) return;
-    ChainInputs in = chain_inputs(stage.obs[slot], stage.mission[slot], a);
+    ChainInputs<true> in = chain_inputs<true>(stage.obs[slot], stage.mission[slot], a);
     const bool wild = wild_inputs(in), tame = __builtin_amdgcn_ballot_w64(wild) == 0;
     if (!tame) controller_inputs(in);
     const MissionFlags f = mission_flags(in.m);
     ScanResult s;
     auto fetch = [&]() {
         wait();
-        const float *sc = stage.scan[slot];
-        s.min_r = sc[0];
-        s.min_r_dx = sc[1];
-        s.min_r_dy = sc[2];
-        s.min_dx_c = sc[3];
-        s.cluster_y_sum = sc[4];
-        s.min_ray = __float_as_int(sc[5]);
-        s.cluster_count = __float_as_int(sc[6]);
-        // Read from LDS at once, like the other inputs.
-        asm volatile("" : "+v"(s.min_r), "+v"(s.min_r_dx), "+v"(s.min_r_dy), "+v"(s.min_dx_c),
-                     "+v"(s.cluster_y_sum), "+v"(s.min_ray), "+v"(s.cluster_count));
+        s = staged_result(stage, slot);
         return s;
     };
-    const ArmOutputs n =
-        tame ? flight_quad<true>(in, wild, f, a, fetch) : flight_quad<false>(in, wild, f, a, fetch);
+    const ArmOutputs<true> n = tame ? flight_values<true, true>(in, wild, f, a, fetch)
+                                    : flight_values<false, true>(in, wild, f, a, fetch);
     if (!f.bwb) OutputRows(rows, env).arm(a, n);  // a BWB mission's are the support wave's
-    if (rows.diag && a == 0) {
-        float *d = rows.diag + env * 5;
-        d[0] = s.min_r;
-        d[1] = (float)s.min_ray;
-        d[2] = s.min_dx_c;
-        d[3] = (float)s.cluster_count;
-        d[4] = s.cluster_y_sum;
+    if (rows.diag && a == 0) store_scan_diag(rows.diag + env * 5, s);
+}
+
+// The same for 64 staged environments, one lane each: three waves of a
+// workgroup, one for each part, write the rows in LDS, from where the
+// workgroup stores them coalesced.
+struct LaneRows {
+    float tactical[64][25];
+    float prior[64][15];
+    __device__ __forceinline__ void arms(int lane, const ArmOutputs<false> &n) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            prior[lane][i] = n.throttle[i];
+            prior[lane][4 + i] = n.outer[i];
+            prior[lane][8 + i] = n.inner[i];
+        }
     }
+};
+
+__device__ __forceinline__ void tactical_lanes(const Stage<64> &stage, int lane, LaneRows &out) {
+    const ChainInputs<false> in = chain_inputs<false>(stage.obs[lane], stage.mission[lane], 0);
+    const bool wild = wild_inputs(in);
+    float v[24];
+    if (__builtin_amdgcn_ballot_w64(wild) == 0) tactical_values<true, false>(in, wild, 0, v);
+    else tactical_values<false, false>(in, wild, 0, v);
+#pragma unroll
+    for (int k = 0; k < 24; ++k) out.tactical[lane][k] = tactical_out<false>(v[k]);
+}
+
+__device__ __forceinline__ void gunnery_lanes(const Stage<64> &stage, int lane, LaneRows &out) {
+    ChainInputs<false> in = chain_inputs<false>(stage.obs[lane], stage.mission[lane], 0);
+    const bool wild = wild_inputs(in), tame = __builtin_amdgcn_ballot_w64(wild) == 0;
+    if (!tame) controller_inputs(in);
+    const MissionFlags f = mission_flags(in.m);
+    const GunOutputs<false> g = tame ? gunnery_values<true, false>(in, wild, f, 0)
+                                     : gunnery_values<false, false>(in, wild, f, 0);
+    out.prior[lane][12] = g.az;
+    out.prior[lane][13] = g.el;
+    out.prior[lane][14] = g.fire;
+    if (f.bwb) out.arms(lane, g.arm);
+}
+
+__device__ __forceinline__ void flight_lanes(const Stage<64> &stage, int lane, LaneRows &out,
+                                             float *diag) {
+    ChainInputs<false> in = chain_inputs<false>(stage.obs[lane], stage.mission[lane], 0);
+    const bool wild = wild_inputs(in), tame = __builtin_amdgcn_ballot_w64(wild) == 0;
+    if (!tame) controller_inputs(in);
+    const MissionFlags f = mission_flags(in.m);
+    auto fetch = [&] { return staged_result(stage, lane); };
+    const ArmOutputs<false> n = tame ? flight_values<true, false>(in, wild, f, 0, fetch)
+                                     : flight_values<false, false>(in, wild, f, 0, fetch);
+    if (!f.bwb) out.arms(lane, n);
+    if (diag) store_scan_diag(diag, staged_result(stage, lane));
 }
 
 // One wave: the actor's symlog scalars and mission values of `Count`
@@ -1813,8 +1963,13 @@ void actor_control_kernel(OnboardRows rows) {
 //   * G = 1, 2: waves 0 .. G-1 run the flight controllers, waves G .. 2G-1
 //     the tactical features, cannon and BWB law, which need no scan; the
 //     others scan, and the support waves join them when they are done.
-//   * G = 4: all waves scan, then four of each role run the controllers.
-//     Two workgroups fit a CU, so one's scan overlaps the other's chains.
+//   * G = 4: all waves scan, then three run the flight controllers, the
+//     tactical features and the cannon and BWB law, one lane per environment,
+//     and all store the rows.  Two workgroups fit a CU and fill its issue
+//     slots, so instructions count and not the chain's length: one lane per
+//     environment takes 4,100 for 64 environments where quads take 10,800
+//     (27.3 -> 25.9 us at 32,768 environments, 54.4 -> 52.1 at 65,536
+//     cluttered; below 16,384 the quads' shorter chains win).
 //   * Wave 7 forms each environment's frame and need (lane e), stages the
 //     empty result of those whose mission uses no scan result and enters the
 //     others in a pool in LDS, corridor scans (the longest) first.  The
@@ -1959,9 +2114,26 @@ __device__ __forceinline__ void onboard_block(const OnboardRows &rows, size_t ba
         }
     }
     if constexpr (!kRoles) {
+        // Rows past the batch end (copies of the last one, staged without a
+        // scan result) are computed and not stored.
+        static_assert(G == 4 && !SCALARS && sizeof(LaneRows) <= sizeof(s.lists));
+        LaneRows &out = *reinterpret_cast<LaneRows *>(&s.lists[0][0]);
         __syncthreads();
-        if (w < G) flight_wave(rows, base, s.stage, 16 * w, lane, [] {});
-        else support_wave(rows, base, s.stage, 16 * (w - G), lane);
+        const size_t rows_here = rows.batch - base < 64 ? rows.batch - base : 64;
+        if (w == 0) {
+            flight_lanes(s.stage, lane, out,
+                         rows.diag && (size_t)lane < rows_here ? rows.diag + (base + lane) * 5
+                                                               : nullptr);
+        } else if (w == 1) {
+            tactical_lanes(s.stage, lane, out);
+        } else if (w == 2) {
+            gunnery_lanes(s.stage, lane, out);
+        }
+        __syncthreads();
+        for (int i = tid; i < (int)rows_here * 24; i += kThreads)
+            rows.tactical[base * 24 + i] = out.tactical[i / 24][i % 24];
+        for (int i = tid; i < (int)rows_here * 15; i += kThreads)
+            rows.prior[base * 15 + i] = out.prior[i / 15][i % 15];
     }
     if (SCALARS) {
         constexpr int kWaves = kPoolWaves - G, kEach = (N + kWaves - 1) / kWaves;
