@@ -252,10 +252,12 @@ __device__ __forceinline__ void load_ranges(__amdgpu_buffer_rsrc_t obs,
 #pragma unroll
     for (int u = 0; u < kScanRays; ++u) {
         const int row = u / 2, head = row / 6, el = row % 6;
+        // A head's rows lie within the instruction's 12-bit offset, the heads
+        // 8,192 bytes apart: one scalar offset instead of one for each load.
         rg[u] = __builtin_bit_cast(
-            float, __builtin_amdgcn_raw_buffer_load_b32(
-                       el < 4 ? obs : upper, 4 * (48 + lane),
-                       4 * ((16 * head + el) * 128 + 64 * (u % 2)), kNontemporal));
+            float, __builtin_amdgcn_raw_buffer_load_b32(el < 4 ? obs : upper,
+                                                        4 * (48 + lane) + 4 * (el * 128 + 64 * (u % 2)),
+                                                        8192 * head, kNontemporal));
     }
 }
 
@@ -408,7 +410,12 @@ __device__ __forceinline__ void closest_fields(int ray, unsigned min_bits, const
 }
 
 // onboard_features.cuh:184-234 for one environment, on one wave (24 rays per
-// lane, no workgroup barrier).
+// lane, no workgroup barrier).  In a batch that fills the chip the scans are
+// three quarters of its instructions, and their number bounds the kernel: the
+// closest return takes about 150 and the corridor and cluster about 450 in an
+// open scene (250 and 500 before the offsets became the key of the closest
+// return, its slot search an early exit and the loads' offsets immediate:
+// 25.9 -> 24.9 us at 32,768 environments, 16.1 -> 15.0 at 16,384).
 //   * The reference maps non-finite ranges to 0 / +-1000 first; both fail
 //     the 0.35 < r < 11.5 window, as NaN does, so the raw value is tested.
 //     The reference skips rays outside the window (:193, :218), and so does
@@ -441,31 +448,30 @@ __device__ __forceinline__ void scan_env(float (&rg)[kScanRays], const RayPlanes
                                          __amdgpu_buffer_rsrc_t next_upper, int lane,
                                          u32x2 *list, ScanResult &out, int need) {
     // Closest return, straight from the ranges: each lane's minimum over its
-    // 16 slots of elevation rows 0..3 as bits (positive floats order like
-    // their bits; a ray outside the window counts as 11.5, the window's
-    // exclusive upper bound, so it never wins), the wave's minimum, then the
-    // first slot (slots are in ray order) and its first lane holding exactly
-    // that range: the reference's first minimum in scan order.
-    constexpr unsigned kWindowTop = 0x41380000u;  // 11.5f
-    unsigned min_bits = kWindowTop;
+    // 16 slots of elevation rows 0..3 as window offsets (they order like the
+    // ranges; everything outside the window is at or above kWindowSpan, so
+    // it never wins), the wave's minimum, then the first slot (slots are in
+    // ray order) and its first lane holding exactly that range: the
+    // reference's first minimum in scan order.
+    unsigned min_bits = kWindowSpan + kWindowLo;
     int min_ray = -1;
     if (need & kNeedClosest) {
-        unsigned lane_min = kWindowTop;
+        unsigned lane_min = kWindowSpan;
 #pragma unroll
-        for (int u = 0; u < kScanRays; ++u) {
-            if ((u / 2) % 6 >= 4) continue;
-            lane_min = min(lane_min, rg[u] > 0.35f ? __float_as_uint(rg[u]) : kWindowTop);
-        }
-        min_bits = wave_min_u32(lane_min);
-        if (min_bits != kWindowTop) {
-            // Visiting slots from the last to the first leaves the first slot
-            // (in ray order) that holds the range, at its first lane.
+        for (int u = 0; u < kScanRays; ++u)
+            if ((u / 2) % 6 < 4) lane_min = min(lane_min, window_offset(rg[u]));
+        const unsigned wave_low = wave_min_u32(lane_min);
+        if (wave_low != kWindowSpan) {
+            min_bits = wave_low + kWindowLo;
 #pragma unroll
-            for (int u = kScanRays - 1; u >= 0; --u) {
+            for (int u = 0; u < kScanRays; ++u) {
                 if ((u / 2) % 6 >= 4) continue;
                 const uint64_t hit =
                     __builtin_amdgcn_ballot_w64(__float_as_uint(rg[u]) == min_bits);
-                if (hit) min_ray = 64 * u + (int)__builtin_ctzll(hit);
+                if (hit) {
+                    min_ray = 64 * u + (int)__builtin_ctzll(hit);
+                    break;
+                }
             }
         }
     }
@@ -1539,7 +1545,8 @@ __device__ __forceinline__ void park_scan(float *park, const ScanResult &s) {
 // LiDAR channels of the scan rays.  The 32-byte result is parked in the
 // environment's own prior row (60 bytes), which phase 2 reads before it
 // writes the 15 prior values there: no scratch memory is needed.
-__global__ __launch_bounds__(kBlockThreads) void actor_scan_kernel(OnboardRows rows) {
+__global__ __launch_bounds__(kBlockThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void actor_scan_kernel(OnboardRows rows) {
     __shared__ RayPlanes rays;
     __shared__ u32x2 lists[kWavesPerBlock][kListCap + 64];  // + a spare entry per lane
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1608,14 +1615,16 @@ __global__ __launch_bounds__(kBlockThreads) void actor_scan_kernel(OnboardRows r
 // scanning waves.  Measured on one box, us, scenes as the generator makes
 // them / cluttered (two launches before, the scan and the control kernel;
 // one group; two; four):
-//    1,000  16.1 / 18.2   9.4 / 11.2  12.5 / 15.3       --
-//    8,192  20.5 / 23.3  11.5 / 14.2  12.9 / 16.3  15.8 / 18.6
-//   12,288  21.2 / 24.5  18.9 / 22.6  15.6 / 19.0  18.6 / 21.1
-//   16,384  22.3 / 25.3  21.5 / 25.6  15.9 / 19.3  20.5 / 22.9
-//   17,000  34.6 / 38.3       --      22.5 / 26.9  21.2 / 23.6
-//   32,768  42.8 / 46.2       --      31.0 / 37.6  27.1 / 29.7
-//   39,999  55.8 / 59.3  46.8 / 55.4  37.8 / 46.0  37.5 / 41.8
-//   65,536  78.5 / 82.0  73.6 / 87.1  57.3 / 67.8  49.0 / 54.2
+//    1,000  16.1 / 18.2   9.4 / 11.2  12.5 / 15.3  12.2 / 14.8
+//    8,192  20.5 / 23.3  11.5 / 14.2  12.9 / 16.3  14.6 / 17.5
+//   12,288  21.2 / 24.5  18.9 / 22.6  15.6 / 19.0  17.0 / 19.5
+//   16,384  22.3 / 25.3  21.5 / 25.6  15.9 / 19.3  18.9 / 21.4
+//   17,000  34.6 / 38.3       --      22.5 / 26.9  19.2 / 22.0
+//   32,768  42.8 / 46.2       --      31.0 / 37.6  25.9 / 28.4
+//   39,999  55.8 / 59.3  46.8 / 55.4  37.8 / 46.0  36.4 / 40.7
+//   65,536  78.5 / 82.0  73.6 / 87.1  57.3 / 67.8  47.3 / 52.2
+// (before the scan became lighter: one group 1,000 9.4 -> 8.9, two 16,384
+// 15.9 -> 15.0, four 32,768 25.9 -> 24.9 and 65,536 47.3 -> 45.4).
 // (Equal shares over two rounds lose: 39,999 at 40 each 40.2 / 45.2, since a
 // CU's last workgroup alone runs faster than two.)
 constexpr size_t kOneGroupMax = 8192, kTwoGroupMax = 16384;
@@ -1982,10 +1991,10 @@ void actor_control_kernel(OnboardRows rows) {
 //     count, every scanner takes its result off it.  The waves of a workgroup
 //     are resident together and no scanner waits for a flight wave, so the
 //     wait ends.
-struct PoolEntry {
+struct alignas(16) PoolEntry {
+    float r[9], py;
     unsigned env;
     int need;
-    float r[9], py;
 };
 
 template <int G>
@@ -2088,11 +2097,8 @@ __device__ __forceinline__ void onboard_block(const OnboardRows &rows, size_t ba
         for (;;) {
             ScanFrame f;
 #pragma unroll
-            for (int i = 0; i < 9; ++i)
-                f.r[i] = __builtin_bit_cast(
-                    float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s.pool[t].r[i])));
-            f.py = __builtin_bit_cast(
-                float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s.pool[t].py)));
+            for (int i = 0; i < 9; ++i) f.r[i] = s.pool[t].r[i];
+            f.py = s.pool[t].py;
             const int t_next = take();
             const bool has_next = t_next < count;
             int next_slot = slot, next_need = kNeedNone;
