@@ -240,7 +240,8 @@ __device__ __forceinline__ unsigned min_same_qx(unsigned v) {
 }
 
 // LV: floats per LiDAR load (4, 2 or 1 from the row alignment).
-// CV: bytes per camera load (16, 8, 4 or 1 from the row alignment).
+// CV: bytes per camera load (16, 8, 4 or 1 from the row alignment; 0 without
+// cameras).
 // DIAG: also write the per-environment diagnostics (no reference
 // counterpart): LiDAR sector minimum / first argmin / valid count and camera
 // quadrant minimum byte / nonzero count, from the same loads.
@@ -264,7 +265,9 @@ __global__ __launch_bounds__(kBlockThreads) void features_kernel(Rows rows) {
     // 0.4 us slower there).
     __shared__ float quads[DIAG ? 16 : 1];
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const bool has_cameras = DEPTH || rows.cameras != nullptr;
+    // A test at run time although it always holds where CV is not 0: without
+    // the branch the camera loads take 81 instead of 66 registers.
+    const bool has_cameras = DEPTH || (CV != 0 && rows.cameras != nullptr);
 
     for (size_t env = xcd_contiguous(blockIdx.x, gridDim.x); env < rows.batch;
          env += gridDim.x) {
@@ -491,6 +494,7 @@ void launch_lv(const Rows &rows, int cv, unsigned blocks, unsigned lds, hipStrea
     case 16: features_kernel<LV, 16, DIAG><<<blocks, kBlockThreads, lds, stream>>>(rows); break;
     case 8: features_kernel<LV, 8, DIAG><<<blocks, kBlockThreads, lds, stream>>>(rows); break;
     case 4: features_kernel<LV, 4, DIAG><<<blocks, kBlockThreads, lds, stream>>>(rows); break;
+    case 0: features_kernel<LV, 0, DIAG><<<blocks, kBlockThreads, lds, stream>>>(rows); break;
     default: features_kernel<LV, 1, DIAG><<<blocks, kBlockThreads, lds, stream>>>(rows); break;
     }
 }
@@ -504,23 +508,36 @@ void launch_diag(const Rows &rows, int lv, int cv, unsigned blocks, unsigned lds
 }
 
 // Workgroups in flight per CU.  Its registers let the plain kernel hold 7
-// per CU; on the streaming layouts fewer keep HBM busier (16,384
+// per CU; on large streaming batches fewer keep HBM busier (16,384
 // environments, identical outputs): rows laid out as the reference's batch
 // 4 per CU (85.76 -> 83.99 us; 3 per CU 91.9 us), strided replay records 5
-// per CU (353.9 -> 348.1 us for 65,536 records).  Indexed gathers, fp32
-// depth cameras and the diagnostics variant keep their resource limit
-// (4 per CU measured 91.9 -> 94.8, 208.0 -> 210.3 and 94.2 -> 116.2 us).
-// The cap is dynamic LDS the kernel does not use: a workgroup then takes
-// more than 1 / (n + 1) of the CU's LDS, so n fit.
+// per CU (353.9 -> 348.1 us for 65,536 records).  A batch of a few rounds
+// gains more from starting at once than from the cap, which leaves its last
+// round nearly empty: below kCapFrom it keeps the resource limit, and up to
+// kCapFewer 5 per CU.  Batch rows, us at 4 / 5 per CU / uncapped:
+//    1,100   9.66   8.57   8.52     4,099  22.86  22.44  22.70
+//    1,375  10.49   9.78   9.67     5,120  27.29  27.01  27.23
+//    2,048  13.58  13.30  12.96     5,800  30.42  30.05  30.34
+//    3,000  17.84  17.33  17.26     7,000  35.71  35.75  36.07
+// (records alike: 1,100 9.66 / 8.59 / 8.56, 7,000 35.80 / 35.83 / 35.92.)
+// Without cameras half as many bytes are in flight per workgroup and the cap
+// only costs: 16,384 environments 53.9 us at 4 per CU, 46.8 at 5, 45.6 at the
+// 7 of the kernel that also serves cameras, and 44.5 at the 8 that its own
+// instantiation's 60 registers allow (4,099: 15.3, 14.2, 13.2, 12.8).
+// Indexed gathers, fp32 depth cameras and the diagnostics variant keep their
+// resource limit (4 per CU measured 91.9 -> 94.8, 208.0 -> 210.3 and 94.2 ->
+// 116.2 us).  The cap is dynamic LDS the kernel does not use: a workgroup
+// then takes more than 1 / (n + 1) of the CU's LDS, so n fit.
+constexpr size_t kCapFrom = 4096, kCapFewer = 6144;
 constexpr unsigned kLdsPerCu = 160 * 1024;
 constexpr unsigned kStageLds = 16 * kStagePitch * sizeof(f32x4);
 
 unsigned occupancy_lds(const Rows &rows) {
-    if (rows.depth || rows.diag || rows.index) return 0;
+    if (rows.depth || rows.diag || rows.index || !rows.cameras || rows.batch < kCapFrom) return 0;
     const bool batch_rows = rows.obs_stride == kObsDim * sizeof(float) &&
                             rows.mission_stride == 10 * sizeof(float) &&
                             rows.camera_stride == 16384;
-    const unsigned per_cu = batch_rows ? 4 : 5;
+    const unsigned per_cu = batch_rows && rows.batch >= kCapFewer ? 4 : 5;
     const unsigned total = (kLdsPerCu / (per_cu + 1) + 1 + 1023) / 1024 * 1024;
     return total - kStageLds;
 }
@@ -534,7 +551,7 @@ int launch_features(const Rows &rows, hipStream_t stream) {
     // Float rows are 4-byte aligned (checked by the callers); the LiDAR block
     // starts 192 bytes into the row.
     const int lv = vector_bytes(rows.obs + kLidarOffset * sizeof(float), rows.obs_stride, 16) / 4;
-    const int cv = rows.cameras ? vector_bytes(rows.cameras, rows.camera_stride, 16) : 16;
+    const int cv = rows.cameras ? vector_bytes(rows.cameras, rows.camera_stride, 16) : 0;
     const unsigned blocks = rows.batch > kMaxBlocks ? kMaxBlocks : (unsigned)rows.batch;
     // Report errors of this launch only: a failure left on the thread by an
     // unrelated earlier runtime call (e.g. selecting a missing device) is
