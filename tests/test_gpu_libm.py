@@ -5,11 +5,12 @@
   evaluates each sine/cosine pair of one angle through sincosf, so its
   results equal those of the separate calls the reference makes
   (onboard_features.cuh:18,49,119-120,210-211,325,469).
-* (float)atan2((double)y, (double)x), the controller's atan2 for the angles
+* atan2_float (csrc/onboard_math.h), the controller's atan2 for the angles
   that reach its angle wraps, is correctly rounded on 8.4e6 arguments, and
   equals the host libm's atan2f (the oracle's) on the arguments that reach
   the wraps' discontinuity exactly: equal, opposite and zero components and
-  results near +-pi (tests/csrc/check_atan2.hip).
+  results near +-pi; directions half a turn apart wrap to the side that the
+  correctly rounded angles give (tests/csrc/check_atan2.hip).
 * One v_mfma_f32_16x16x32_f16 instruction drops the bits of a product that
   lie more than 2^-24 below the largest product of its group (one lane's
   eight k values) before it rounds the sum, and over random blocks its error
@@ -49,10 +50,12 @@ def test_wrap_angles_match_the_host_atan2f():
     proc = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert proc.returncode == 0, proc.stdout + proc.stderr
     # "<n> checked, <a> differ from double atan2, <m> exact-angle arguments,
-    #  <b> differ from atan2f, <c> other arguments differ from atan2f"
+    #  <b> differ from atan2f, <c> other arguments differ from atan2f,
+    #  <p> opposite pairs, <w> wrap to the other side"
     words = proc.stdout.split("\n")[-2].split()
     assert int(words[0]) > 8_000_000 and words[2] == "0", proc.stdout
     assert int(words[7]) > 2_000_000 and words[10] == "0", proc.stdout
+    assert int(words[20]) > 130_000 and words[23] == "0", proc.stdout
 
 
 @pytest.mark.gpu

@@ -4,8 +4,10 @@ on the GPU by tests/csrc/check_onboard_math.hip over 2^21 arguments each.
 Bounds, in ulp of the float result.  One rounding of a double evaluation is
 0.5.  A tail of at most a tenth of the result is evaluated in single with
 about five roundings, 2.5 ulp of a value whose ulp is at most an eighth of the
-result's: 0.3 more for atan2's q^3 and sine's r^3 terms (and the cosine of
-the same remainder), 0.1 for atanh (its tail is at most 0.01).  The tangent
+result's: 0.3 more for the sine's r^3 term (and the cosine of the same
+remainder), 0.1 for atanh (its tail is at most 0.01).  atan2 is double
+throughout, within 2^-51 of the angle before its one rounding
+(check_atan2.hip holds that it is the correctly rounded one).  The tangent
 adds its cosine's tail (0.02, so 0.05), and the cosine near a zero its
 remainder's 2^-41 over the ulp of 2^-16 where its result is measured (0.25).
 The half turn's sine is single throughout and in ulp of 1: the distance to
@@ -25,7 +27,7 @@ import pytest
 EXE = Path(__file__).resolve().parent / "csrc" / "bin" / "check_onboard_math"
 
 BOUND = {"quotient": 0.501, "divisor": 0.5, "square_root": 0.501, "hypotenuse": 0.501,
-         "atan2": 0.85, "direction_s": 0.501, "direction_c": 0.501, "atanh": 0.6, "cos": 1.05,
+         "atan2": 0.501, "direction_s": 0.501, "direction_c": 0.501, "atanh": 0.6, "cos": 1.05,
          "sin_half_turn": 1.9, "tan": 0.9, "wrap": 0.501}
 
 

@@ -10,7 +10,7 @@
 // The leading terms are in double, which issues at the rate of single, and
 // the polynomials' tails, which are at most a tenth of the result, in single
 // (their coefficients are literals of the instruction; a double coefficient
-// takes two scalar moves).  Errors are 0.5 to 0.6 ulp of a float, where the
+// takes two scalar moves), except where an ulp can flip a sign (atan2).  Errors are 0.5 to 0.6 ulp of a float, where the
 // single-precision library functions are up to an ulp or two off
 // (tests/csrc/check_onboard_math.hip).  Polynomials interpolate the power
 // series' tails at Chebyshev nodes (coefficients computed with 60 digits).
@@ -92,10 +92,15 @@ __device__ __forceinline__ float hypotenuse(float xf, float yf) {
     return h;
 }
 
-// atan2 of any two floats.  The smaller magnitude over the larger, brought
-// below tan(pi/8) by the addition theorem ((z - 1) / (z + 1), plus pi/4), an
-// odd polynomial, and a whole number of pi/4.  Exact angles (equal or zero
-// components) come out as the float nearest to them.
+// atan2 of any two floats, as one rounding of a double value within 2^-51: the
+// angles reach wrap_angle's discontinuity, where the side that an angle rounds
+// to decides the sign of the wrapped difference.  The smaller magnitude over
+// the larger, brought below tan(pi/8) by the addition theorem ((z - 1) / (z +
+// 1), plus pi/4), an odd polynomial, and a whole number of pi/4.  The
+// polynomial is the interpolant of (atan q - q) / q^3 in t = q^2 at 11
+// Chebyshev nodes of [0, 1.0001 tan^2(pi/8)], within 2^-56 of q.  With 8 terms
+// in single it was up to 0.85 ulp off, and the difference of two angles half a
+// turn apart changed sign for one pair of small integers in 350.
 template <bool TAME>
 __device__ __forceinline__ float atan2_float(float yf, float xf) {
     const float ay = __builtin_fabsf(yf), ax = __builtin_fabsf(xf);
@@ -108,15 +113,18 @@ __device__ __forceinline__ float atan2_float(float yf, float xf) {
     const double r = recip46(den);
     double q = num * r;
     q = __builtin_fma(__builtin_fma(-den, q, num), r, q);
-    const float qf = (float)q, t = qf * qf;
-    float p = __builtin_fmaf(t, 0x1.0df7a02661596p-5f, -0x1.edbfaee18e70fp-5f);
-    p = __builtin_fmaf(t, p, 0x1.377de082fa570p-4f);
-    p = __builtin_fmaf(t, p, -0x1.7415affa08e33p-4f);
-    p = __builtin_fmaf(t, p, 0x1.c7196338febe7p-4f);
-    p = __builtin_fmaf(t, p, -0x1.249240d9941d8p-3f);
-    p = __builtin_fmaf(t, p, 0x1.999999885befbp-3f);
-    p = __builtin_fmaf(t, p, -0x1.555555555260ep-2f);
-    const double v = q + (double)(qf * t * p);
+    const double t = q * q;
+    double p = __builtin_fma(t, -0x1.3a2b7a07caea9p-6, 0x1.41603647c7a7cp-5);
+    p = __builtin_fma(t, p, -0x1.a098bb6ba4941p-5);
+    p = __builtin_fma(t, p, 0x1.dfe61e80903d2p-5);
+    p = __builtin_fma(t, p, -0x1.10fa75382537fp-4);
+    p = __builtin_fma(t, p, 0x1.3b1262d95579ep-4);
+    p = __builtin_fma(t, p, -0x1.745d0b26b83e7p-4);
+    p = __builtin_fma(t, p, 0x1.c71c7185314cbp-4);
+    p = __builtin_fma(t, p, -0x1.24924924360cbp-3);
+    p = __builtin_fma(t, p, 0x1.999999999934ap-3);
+    p = __builtin_fma(t, p, -0x1.5555555555555p-2);
+    const double v = __builtin_fma(q * t, p, q);
     // Quarter turns: pi/4 for the upper octant, then reflected at pi/4 and
     // at pi/2.
     float k = upper ? 1.0f : 0.0f;
