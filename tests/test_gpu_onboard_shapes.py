@@ -1,7 +1,7 @@
 """The onboard and actor-input entries' workgroup shapes (csrc/onboard.hip): a
 row's outputs do not depend on the batch it comes in.  Every batch size around
-a shape's bounds (a group of 16, one, two and four groups, equal shares, the
-two-stream form) against the rows of a batch in another shape, bit for bit,
+a shape's bounds (the least share of 8, one workgroup per CU and two, one, two
+and four groups of 16, the two-stream form) against the rows of a batch in another shape, bit for bit,
 and each shape on the generator's non-finite and signed-zero rows."""
 from __future__ import annotations
 
@@ -14,7 +14,8 @@ from turbinator_c_amd import synth
 
 pytestmark = pytest.mark.gpu
 
-SIZES = (1, 15, 16, 17, 31, 33, 1000, 8191, 8192, 8193, 16383, 16384, 16385, 20011, 32767, 32768)
+SIZES = (1, 7, 8, 9, 15, 16, 17, 31, 33, 1000, 2048, 2049, 4095, 4097, 5000, 8191, 8192, 8193,
+         9000, 16383, 16384, 16385, 20011, 32767, 32768)
 
 
 @pytest.fixture(scope="module")
@@ -70,7 +71,7 @@ def test_special_rows_in_every_shape(torch_cuda, hip, n):
             f"special {n}")
 
 
-@pytest.mark.parametrize("n", [1, 16, 17, 3071, 3072, 3073])
+@pytest.mark.parametrize("n", [1, 16, 17, 512, 513, 2500, 3071, 3072, 3073])
 def test_actor_rows_do_not_depend_on_the_batch(torch_cuda, hip, tiled, n):
     torch = torch_cuda
     obs, mission = tiled

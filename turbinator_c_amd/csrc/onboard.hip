@@ -1608,27 +1608,37 @@ void actor_scan_kernel(OnboardRows rows) {
     }
 }
 
-// The onboard entry's workgroups: one group of 16 environments up to
-// kOneGroupMax (two workgroups on every CU), two up to kTwoGroupMax, four
-// above, in equal shares while that is one round of kRoundBlocks.  Fewer
-// groups are shorter chains, more share the ray table, the launch and the
-// scanning waves.  Measured on one box, us, scenes as the generator makes
-// them / cluttered (two launches before, the scan and the control kernel;
-// one group; two; four):
-//    1,000  16.1 / 18.2   9.4 / 11.2  12.5 / 15.3  12.2 / 14.8
-//    8,192  20.5 / 23.3  11.5 / 14.2  12.9 / 16.3  14.6 / 17.5
-//   12,288  21.2 / 24.5  18.9 / 22.6  15.6 / 19.0  17.0 / 19.5
-//   16,384  22.3 / 25.3  21.5 / 25.6  15.9 / 19.3  18.9 / 21.4
-//   17,000  34.6 / 38.3       --      22.5 / 26.9  19.2 / 22.0
-//   32,768  42.8 / 46.2       --      31.0 / 37.6  25.9 / 28.4
-//   39,999  55.8 / 59.3  46.8 / 55.4  37.8 / 46.0  36.4 / 40.7
-//   65,536  78.5 / 82.0  73.6 / 87.1  57.3 / 67.8  47.3 / 52.2
-// (before the scan became lighter: one group 1,000 9.4 -> 8.9, two 16,384
-// 15.9 -> 15.0, four 32,768 25.9 -> 24.9 and 65,536 47.3 -> 45.4).
-// (Equal shares over two rounds lose: 39,999 at 40 each 40.2 / 45.2, since a
-// CU's last workgroup alone runs faster than two.)
-constexpr size_t kOneGroupMax = 8192, kTwoGroupMax = 16384;
-constexpr size_t kRoundBlocks = 512;  // workgroups resident at once: two per CU
+// The onboard entry's workgroups take equal shares of the batch, at least
+// kMinShare environments: one workgroup for each CU up to 4,096 environments,
+// two above, as many as are resident at once.  A share of up to 16 runs as one
+// group, up to 32 as two, above that as four (whose flight chains take one
+// lane per environment), and batches above 32,768 take further rounds.  Fewer
+// environments are shorter chains and fewer scans for a workgroup's waves,
+// more share the ray table and the launch.  What the scans cost depends on the
+// scene and the missions: where every environment is scanned through a
+// cluttered corridor they are nine tenths of the time, and shares of 16 left
+// most CUs idle (64 environments on four).  Measured on one box, us, scenes as
+// the generator makes them / cluttered with every mission a slalom (two
+// launches, a scan and a control kernel; 16, 32 or 64 environments per
+// workgroup; these shares):
+//       64  15.5 / 22.0   7.9 / 26.6   7.9 / 21.2
+//    1,000  15.8 / 23.2   8.8 / 28.0   8.5 / 22.4
+//    2,560  17.7 / 28.6   9.0 / 28.4   8.7 / 23.6
+//    4,096  17.9 / 28.8   9.1 / 28.6   (the same)
+//    6,000  19.0 / 35.6  10.4 / 33.1  10.1 / 29.1
+//    9,000  20.2 / 42.5  13.4 / 56.0  12.7 / 40.5
+//   12,000  20.9 / 74.0  14.4 / 57.1  13.5 / 49.0
+//   16,384  21.0 / 74.4  14.9 / 57.7  (the same)
+//   17,000  34.1 / 69.9  (already equal shares)  16.7 / 54.7
+//   32,768  44.8 / 106   22.9 / 87.0  (the same)
+// Shares below 8 gain for the smallest batches when all are scanned (4 each:
+// 64 8.1 / 14.6) and lose from 2,048 (9.6 / 18.0; 3,000 15.1 / 29.9).  Of the
+// groups, one / two / four: 8,192 environments 10.6 / 12.9 / 14.6, 16,384 20.2
+// / 14.9 / 16.4, 17,000 -- / 22.5 / 16.7.
+// (Equal shares over two rounds lose: 39,999 at 40 each cluttered 45.2 us for
+// 40.7, since a CU's last workgroup alone runs faster than two.)
+constexpr unsigned kMinShare = 8;
+constexpr size_t kCus = 256, kRoundBlocks = 512;  // workgroups resident at once: two per CU
 constexpr int kPoolWaves = kControlThreads / 64;
 
 // The inputs of N environments in LDS: obs[0..47], mission[0..9], the scan
@@ -2158,6 +2168,13 @@ void onboard_kernel(OnboardRows rows, unsigned share) {
     onboard_block<G, false>(rows, base, lds);
 }
 
+// Environments per workgroup of a batch that one round of workgroups takes.
+size_t share_of(size_t batch) {
+    const size_t blocks = batch <= 16 * kCus ? kCus : kRoundBlocks;
+    const size_t share = (batch + blocks - 1) / blocks;
+    return share < kMinShare ? kMinShare : share;
+}
+
 // A grid of `want` workgroups.
 dim3 wide_grid(size_t want) {
     return dim3((unsigned)(want < kControlGridX ? want : kControlGridX),
@@ -2185,16 +2202,14 @@ extern "C" int tb_hip_onboard_tactical_prior_device(const float *obs, const floa
     rows.batch = batch_size;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     (void)hipGetLastError();
-    if (batch_size <= kOneGroupMax) {
-        onboard_kernel<1><<<wide_grid((batch_size + 15) / 16), kControlThreads, 0, s>>>(rows, 16);
-    } else if (batch_size <= kTwoGroupMax) {
-        onboard_kernel<2><<<wide_grid((batch_size + 31) / 32), kControlThreads, 0, s>>>(rows, 32);
-    } else {
-        const size_t share = batch_size < 64 * kRoundBlocks
-                                 ? (batch_size + kRoundBlocks - 1) / kRoundBlocks : 64;
-        onboard_kernel<4><<<wide_grid((batch_size + share - 1) / share), kControlThreads, 0, s>>>(
-            rows, (unsigned)share);
-    }
+    const size_t want = share_of(batch_size), share = want < 64 ? want : 64;
+    const dim3 grid = wide_grid((batch_size + share - 1) / share);
+    if (share <= 16)
+        onboard_kernel<1><<<grid, kControlThreads, 0, s>>>(rows, (unsigned)share);
+    else if (share <= 32)
+        onboard_kernel<2><<<grid, kControlThreads, 0, s>>>(rows, (unsigned)share);
+    else
+        onboard_kernel<4><<<grid, kControlThreads, 0, s>>>(rows, (unsigned)share);
     return hipGetLastError() == hipSuccess;
 }
 
@@ -2340,26 +2355,48 @@ __device__ __forceinline__ void actor_planes_block(const ActorRows &rows, size_t
     }
 }
 
+// The onboard features and scalars of one workgroup's environments: SPREAD a
+// share below 16, else 16 (a constant: the end of a share held in registers
+// cost the full workgroups 0.2 us and beside plane workgroups up to 4%).
+template <bool SPREAD>
+__device__ __forceinline__ void actor_share(OnboardRows &rows, size_t block, unsigned share,
+                                            OnboardLds<1> &lds) {
+    const size_t base = block * (SPREAD ? share : 16);
+    if (base >= rows.batch) return;
+    if (SPREAD && rows.batch - base > share) rows.batch = base + share;
+    onboard_block<1, true>(rows, base, lds);
+}
+
 // The whole preparation of a small batch in one launch: the first
-// `onboard_blocks` workgroups take 16 environments' onboard features and
-// scalars each (the longest chains start first), the others one
+// `onboard_blocks` workgroups take a share of the environments' onboard
+// features and scalars each (the longest chains start first), the others one
 // environment's planes each.
+template <bool SPREAD>
 __global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void actor_one_kernel(OnboardRows rows, ActorRows planes, unsigned onboard_blocks) {
     __shared__ OnboardLds<1> lds;
     if (blockIdx.x < onboard_blocks)
-        onboard_block<1, true>(rows, (size_t)blockIdx.x * 16, lds);
+        actor_share<SPREAD>(rows, blockIdx.x, kMinShare, lds);
     else
         actor_planes_block(planes, blockIdx.x - onboard_blocks);
 }
 
 // The onboard features and scalars alone, for any batch.
+template <bool SPREAD>
 __global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
-void actor_onboard_kernel(OnboardRows rows) {
+void actor_onboard_kernel(OnboardRows rows, unsigned share) {
     __shared__ OnboardLds<1> lds;
-    const size_t base = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 16;
-    if (base >= rows.batch) return;
-    onboard_block<1, true>(rows, base, lds);
+    actor_share<SPREAD>(rows, (size_t)blockIdx.y * gridDim.x + blockIdx.x, share, lds);
+}
+
+void launch_actor_onboard(const OnboardRows &rows, hipStream_t s) {
+    const size_t share = share_of(rows.batch);
+    if (share < 16)
+        actor_onboard_kernel<true><<<wide_grid((rows.batch + share - 1) / share), kControlThreads,
+                                     0, s>>>(rows, (unsigned)share);
+    else
+        actor_onboard_kernel<false><<<wide_grid((rows.batch + 15) / 16), kControlThreads, 0, s>>>(
+            rows, 16);
 }
 
 // From kOverlapMinBatch environments the scan and control kernels run beside
@@ -2388,6 +2425,13 @@ void actor_onboard_kernel(OnboardRows rows) {
 //    1,500   56.5   41.1   63.2      3,500   97.1   97.6   97.3
 //                                    4,096  112.8  116.4  112.5
 constexpr size_t kOverlapMinBatch = 3072;
+// In that one launch the onboard workgroups take 8 environments each while the
+// plane workgroups leave CUs idle, and 16 above, where they would hold more of
+// the CUs' places (both planes, generated scenes / cluttered slaloms, us;
+// three launches before, 16 and 8 each): 64 19.6 / 26.3, 8.0 / 26.9, 7.6 /
+// 21.6; 512 28.4 / 35.5, 13.2 / 31.5, 12.6 / 25.6; 700 32.8 / 39.8, 15.8 /
+// 33.5, 16.5 / 27.1; 3,071 86.8 / 86.8, 84.1 / 84.5, 87.3 / 89.2.
+constexpr size_t kSpreadMax = 512;
 constexpr int kMaxDevices = 64;
 
 struct SideStream {
@@ -2470,15 +2514,20 @@ extern "C" int tb_hip_actor_inputs_device(const float *obs, const float *mission
     ar.lidar = lidar_channels;
     ar.luma = camera_luma;
     ar.batch = batch_size;
-    const dim3 onboard_grid = wide_grid((batch_size + 15) / 16);
     if (!planes) {
-        actor_onboard_kernel<<<onboard_grid, kControlThreads, 0, s>>>(rows);
+        launch_actor_onboard(rows, s);
         return hipGetLastError() == hipSuccess;
     }
     if (batch_size < kOverlapMinBatch) {
-        const unsigned onboard_blocks = (unsigned)((batch_size + 15) / 16);
-        actor_one_kernel<<<onboard_blocks + (unsigned)batch_size, kControlThreads, 0, s>>>(
-            rows, ar, onboard_blocks);
+        const bool spread = batch_size <= kSpreadMax;
+        const unsigned n = (unsigned)batch_size, share = spread ? kMinShare : 16,
+                       onboard_blocks = (n + share - 1) / share;
+        if (spread)
+            actor_one_kernel<true><<<onboard_blocks + n, kControlThreads, 0, s>>>(rows, ar,
+                                                                                 onboard_blocks);
+        else
+            actor_one_kernel<false><<<onboard_blocks + n, kControlThreads, 0, s>>>(rows, ar,
+                                                                                  onboard_blocks);
         return hipGetLastError() == hipSuccess;
     }
     SideStream *side = side_stream(s);
@@ -2506,7 +2555,7 @@ extern "C" int tb_hip_actor_inputs_device(const float *obs, const float *mission
         actor_control_kernel<<<wide_grid((batch_size + 63) / 64), kControlThreads, 0, beside>>>(
             rows);
     } else {
-        actor_onboard_kernel<<<onboard_grid, kControlThreads, 0, beside>>>(rows);
+        launch_actor_onboard(rows, beside);
     }
     const int ok = hipGetLastError() == hipSuccess;
     if (side && (hipEventRecord(side->join, side->stream) != hipSuccess ||
