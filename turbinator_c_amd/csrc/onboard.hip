@@ -1635,10 +1635,22 @@ void actor_scan_kernel(OnboardRows rows) {
 // 64 8.1 / 14.6) and lose from 2,048 (9.6 / 18.0; 3,000 15.1 / 29.9).  Of the
 // groups, one / two / four: 8,192 environments 10.6 / 12.9 / 14.6, 16,384 20.2
 // / 14.9 / 16.4, 17,000 -- / 22.5 / 16.7.
-// (Equal shares over two rounds lose: 39,999 at 40 each cluttered 45.2 us for
-// 40.7, since a CU's last workgroup alone runs faster than two.)
 constexpr unsigned kMinShare = 8;
 constexpr size_t kCus = 256, kRoundBlocks = 512;  // workgroups resident at once: two per CU
+
+// Above one round of 64 environments in every workgroup the last round holds
+// the rest.  Up to half a round of it goes over all CUs in equal shares, one
+// workgroup each; in shares of 64 it left most of them idle, and a workgroup
+// alone on its CU took as long as before (us, as generated / cluttered
+// slaloms; two launches, shares of 64, equal shares of the rest):
+//   34,000  54.4 / 118.7   33.1 / 133.6   29.6 / 89.9
+//   39,999  59.3 / 133.2   33.6 / 135.1   32.2 / 110.5
+//   45,000  62.3 / 144.4   35.1 / 136.3   35.1 / 126.3
+//   70,000  99.3 / 221.4   52.0 / 207.4   51.0 / 176.3
+// (65,600, 64 above two rounds: 95.6 / 211.4, 45.8 / 201.9, 47.2 / 169.3.)
+// (Equal shares over both rounds lose: 39,999 at 40 each cluttered 45.2 us for
+// 40.7, since a CU's last workgroup alone runs faster than two.)
+constexpr size_t kRoundRows = 64 * kRoundBlocks, kRestRows = 64 * kCus;
 constexpr int kPoolWaves = kControlThreads / 64;
 
 // The inputs of N environments in LDS: obs[0..47], mission[0..9], the scan
@@ -2157,12 +2169,23 @@ __device__ __forceinline__ void onboard_block(const OnboardRows &rows, size_t ba
     }
 }
 
-// `share` environments per workgroup, at most 16 G.
-template <int G>
+// `share` environments per workgroup, at most 16 G; with REST (G = 4) those
+// after the batch's whole rounds of 64 each.
+template <int G, bool REST = false>
 __global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void onboard_kernel(OnboardRows rows, unsigned share) {
     __shared__ OnboardLds<G> lds;
-    const size_t base = ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * share;
+    size_t block = (size_t)blockIdx.y * gridDim.x + blockIdx.x, first = 0;
+    if constexpr (REST) {
+        const size_t whole = rows.batch / kRoundRows * kRoundBlocks;
+        if (block < whole) {
+            share = 64;
+        } else {
+            first = 64 * whole;
+            block -= whole;
+        }
+    }
+    const size_t base = first + block * share;
     if (base >= rows.batch) return;
     if (rows.batch - base > share) rows.batch = base + share;  // this workgroup's end
     onboard_block<G, false>(rows, base, lds);
@@ -2202,6 +2225,13 @@ extern "C" int tb_hip_onboard_tactical_prior_device(const float *obs, const floa
     rows.batch = batch_size;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     (void)hipGetLastError();
+    const size_t rest = batch_size % kRoundRows;
+    if (batch_size > kRoundRows && rest != 0 && rest < kRestRows) {
+        const size_t share = (rest + kCus - 1) / kCus;
+        onboard_kernel<4, true><<<wide_grid((batch_size - rest) / 64 + (rest + share - 1) / share),
+                                  kControlThreads, 0, s>>>(rows, (unsigned)share);
+        return hipGetLastError() == hipSuccess;
+    }
     const size_t want = share_of(batch_size), share = want < 64 ? want : 64;
     const dim3 grid = wide_grid((batch_size + share - 1) / share);
     if (share <= 16)
