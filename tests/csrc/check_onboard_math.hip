@@ -64,10 +64,49 @@ static uint32_t next32(void) {  // xorshift64*
     rng ^= rng >> 27;
     return (uint32_t)((rng * 2685821657736338717ull) >> 32);
 }
+static uint64_t hard_rng = 0x2545f4914f6cdd1dull;  // its own: the other arguments stay
+static uint32_t hard32(void) {
+    const uint64_t kept = rng;
+    rng = hard_rng;
+    const uint32_t v = next32();
+    hard_rng = rng;
+    rng = kept;
+    return v;
+}
 static float unit(void) { return (float)(next32() >> 8) / 16777216.0f; }
 static float sign(void) { return next32() & 1 ? -1.0f : 1.0f; }
 // Log-uniform magnitude in [2^lo, 2^hi), random sign.
 static float spread(int lo, int hi) { return sign() * ldexpf(1.0f + unit(), lo + (int)(next32() % (unsigned)(hi - lo))); }
+
+// x, y whose quotient lies within 2^-47 of a rounding boundary: x 2^25 = +-1
+// (mod y), so that x / y is 1 / (2^25 y) beside an odd multiple of 2^-25.
+static void hard_quotient(float *x, float *y) {
+    for (;;) {
+        const uint64_t d = (1u << 23) | (hard32() >> 9) | 1u;
+        uint64_t inv = 1, base = (d + 1) / 2;  // 1 / 2 (mod y), to the 25th power
+        for (int e = 25; e; e >>= 1) {
+            if (e & 1) inv = inv * base % d;
+            base = base * base % d;
+        }
+        const uint64_t n = hard32() & 1 ? inv : d - inv;
+        if (2 * n < d) continue;  // the quotient is to lie in [1/2, 1)
+        *x = (float)n;
+        *y = (float)d;
+        return;
+    }
+}
+// x = m^2 - s with an odd 25-bit m and a small s: its root lies within |s| 2^-49
+// of a rounding boundary.  s = 1 (mod 8) has a square root modulo 2^26.
+static float hard_square(void) {
+    const int64_t s = 8 * ((int64_t)(hard32() % 64) - 32) + 1;
+    int64_t m = 1;
+    for (int b = 3; b < 26; ++b)
+        if ((m * m - s) & ((int64_t)1 << b)) m += (int64_t)1 << (b - 1);
+    m &= (1 << 26) - 1;
+    if (m >= 1 << 25) m = (1 << 26) - m;
+    if (m < 1 << 24) m = (1 << 25) - m;
+    return (float)(m * m - s);
+}
 
 static const long double kTwoPi = 6.283185307179586476925286766559005768L;
 
@@ -124,7 +163,9 @@ int main(void) {
             b[i] = spread(-20, 13);
             if (kind == QUOTIENT || kind == DIVISOR) b[i] = fabsf(b[i]);
             if (kind == DIVISOR && i % 64 == 0) a[i] = spread(-126, 0) * 0x1p-20f;  // subnormal quotients
+            if ((kind == QUOTIENT || kind == DIVISOR) && i % 16 == 1) hard_quotient(&a[i], &b[i]);
             if (kind == ROOT) a[i] = i % 64 ? fabsf(spread(-40, 26)) : 0.0f;
+            if (kind == ROOT && i % 16 == 1) a[i] = hard_square();
             if (kind == ATANH) a[i] = sign() * (i % 2 ? 0.9999f * unit() : fminf(ldexpf(unit(), -(int)(next32() % 20)), 0.9999f));
             if (kind == ATANH && i % 1024 == 0) a[i] = sign() * 0.0f;
             if (kind == SIN_PI) a[i] = unit();
@@ -182,7 +223,7 @@ int main(void) {
             off += !same;
             if (!same) fprintf(stderr, "%s(%g, %g) = %g, library %g\n", kNames[kind], a[i], b[i], g[i], want);
         }
-        printf("%s %zu %.3f %zu %zu\n", kNames[kind], n, worst, differ, off);
+        printf("%s %zu %.9f %zu %zu\n", kNames[kind], n, worst, differ, off);
     }
     CHECK(hipFree(da));
     CHECK(hipFree(db));

@@ -34,27 +34,34 @@ __device__ __forceinline__ float above_zero(float x) {
     return __builtin_fmaxf(x, __builtin_bit_cast(float, 1u));
 }
 
-// 1 / y within 2^-46 (the hardware value, 2^-23, refined once) or 2^-52.
-// For y not 0, infinite or NaN.
-__device__ __forceinline__ double recip46(double y) {
+// 1 / y within 2^-48 (the hardware value, 2^-24, refined once) or 2^-52 (by
+// the cubic iteration, one operation more).  For y not 0, infinite or NaN.
+__device__ __forceinline__ double recip48(double y) {
     const double r = __builtin_amdgcn_rcp(y);
     return __builtin_fma(__builtin_fma(-y, r, 1.0), r, r);
 }
 __device__ __forceinline__ double recip52(double y) {
-    const double r = recip46(y);
-    return __builtin_fma(__builtin_fma(-y, r, 1.0), r, r);
+    const double r = __builtin_amdgcn_rcp(y), e = __builtin_fma(-y, r, 1.0);
+    return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// 1 / sqrt(x) within 2^-44, for positive normal x.
-__device__ __forceinline__ double rsqrt44(double x) {
+// 1 / sqrt(x) within 2^-47 (the hardware value, 2^-24, refined once) or 2^-52,
+// for positive normal x.
+__device__ __forceinline__ double rsqrt47(double x) {
     const double r = __builtin_amdgcn_rsq(x);
     return __builtin_fma(r * 0.5, __builtin_fma(-x * r, r, 1.0), r);
 }
+__device__ __forceinline__ double rsqrt52(double x) {
+    const double r = __builtin_amdgcn_rsq(x), e = __builtin_fma(-x * r, r, 1.0);
+    return __builtin_fma(r * e, __builtin_fma(e, 0.375, 0.5), r);
+}
 
-// x / y for y not 0.
+// The IEEE quotient x / y for y not 0: the product of x and the reciprocal is
+// within 1.5 2^-52 of x / y, and no quotient of two floats lies closer than
+// 2^-49 to a rounding boundary.
 template <bool TAME>
 __device__ __forceinline__ float quotient(float x, float y) {
-    const float q = (float)((double)x * recip46((double)y));
+    const float q = (float)((double)x * recip52((double)y));
     if constexpr (TAME) return q;
     const bool limit = !(__builtin_fabsf(y) < __builtin_huge_valf());
     const float l = x / y;
@@ -62,8 +69,6 @@ __device__ __forceinline__ float quotient(float x, float y) {
 }
 
 // The IEEE quotients by one divisor y > 0 (infinity included: quotients 0).
-// The product of x and the reciprocal is within 1.5 2^-52 of x / y, and no
-// quotient of two floats lies closer than 2^-49 to a rounding boundary.
 struct Divisor {
     double r;
     __device__ __forceinline__ explicit Divisor(float y)
@@ -71,10 +76,11 @@ struct Divisor {
     __device__ __forceinline__ float operator()(float x) const { return (float)((double)x * r); }
 };
 
-// sqrt(x), x >= 0.
+// The IEEE square root, x >= 0: within 1.5 2^-52 before its rounding, and no
+// root of a float lies closer than 2^-51 to a rounding boundary.
 template <bool TAME>
 __device__ __forceinline__ float square_root(float x) {
-    const float s = (float)((double)x * rsqrt44((double)above_zero(x)));
+    const float s = (float)((double)x * rsqrt52((double)above_zero(x)));
     if constexpr (TAME) return s;
     const bool limit = !(x < __builtin_huge_valf());
     return limit ? x : s;  // infinity or NaN
@@ -85,7 +91,7 @@ template <bool TAME>
 __device__ __forceinline__ float hypotenuse(float xf, float yf) {
     const double x = above_zero(__builtin_fabsf(xf)), y = yf;
     const double h2 = __builtin_fma(y, y, x * x);
-    const float h = (float)(h2 * rsqrt44(h2));
+    const float h = (float)(h2 * rsqrt47(h2));
     if constexpr (TAME) return h;
     const bool limit = !(__builtin_fabsf(xf) + __builtin_fabsf(yf) < __builtin_huge_valf());
     if (__builtin_amdgcn_ballot_w64(limit)) return limit ? hypotf(xf, yf) : h;
@@ -110,7 +116,7 @@ __device__ __forceinline__ float atan2_float(float yf, float xf) {
     const double h = hf, l = lf;
     const double diff = l - h, sum = l + h;
     const double num = upper ? diff : l, den = upper ? sum : h;
-    const double r = recip46(den);
+    const double r = recip48(den);
     double q = num * r;
     q = __builtin_fma(__builtin_fma(-den, q, num), r, q);
     const double t = q * q;
@@ -148,7 +154,7 @@ struct Direction {
 __device__ __forceinline__ Direction direction(float yf, float xf) {
     const double y = yf;
     const double x = __builtin_copysignf(above_zero(__builtin_fabsf(xf)), xf);
-    const double r = rsqrt44(__builtin_fma(y, y, x * x));
+    const double r = rsqrt47(__builtin_fma(y, y, x * x));
     return Direction{(float)(y * r), (float)(x * r)};
 }
 
@@ -164,7 +170,7 @@ __device__ __forceinline__ float atanh_float(float xf) {
     const double p = __builtin_amdgcn_ldexp(1.0, (int)k);
     const double minus = 1.0 - p, plus = 1.0 + p;
     const double num = __builtin_fma(x, plus, minus), den = __builtin_fma(x, minus, plus);
-    const double s = num * recip46(den);
+    const double s = num * recip48(den);
     const float sf = (float)s, t = sf * sf;
     float c = __builtin_fmaf(t, 0x1.ddf01984cfbd1p-4f, 0x1.245ba6a054aeep-3f);
     c = __builtin_fmaf(t, c, 0x1.9999ecc082d44p-3f);
@@ -228,7 +234,7 @@ __device__ __forceinline__ float tan_float(float xf) {
     const float tf = (float)t;
     const double c = __builtin_fma(t, -0.5, 1.0) + (double)cos_tail(tf);
     const double s = x + (double)sin_tail(xf, tf);
-    return (float)(s * recip46(c));
+    return (float)(s * recip48(c));
 }
 
 // atan2(sin(d), cos(d)): d less its whole turns.  d is a float, so it never
