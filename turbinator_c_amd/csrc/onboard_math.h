@@ -217,15 +217,13 @@ __device__ __forceinline__ float cos_float(float xf) {
     return f;
 }
 
-// sin(pi h) for h in [0, 1], as the cosine of the distance to pi/2.
+// sin(p h) for h in [0, 1] and the float p nearest to pi: 1 - 2 sin^2 of half
+// the distance of p h to pi/2, which is at most pi/4.
 __device__ __forceinline__ float sin_half_turn(float h) {
-    const float y = __builtin_fmaf(h, 0x1.921fb6p+1f, -0x1.921fb6p+0f), t = y * y;
-    float p = __builtin_fmaf(t, 0x1.155c2cdb344aep-29f, -0x1.27bbdf424ae4fp-22f);
-    p = __builtin_fmaf(t, p, 0x1.a0197101a3aa5p-16f);
-    p = __builtin_fmaf(t, p, -0x1.6c16c0b9cb32ap-10f);
-    p = __builtin_fmaf(t, p, 0x1.555555550eee7p-5f);
-    p = __builtin_fmaf(t, p, -0.5f);
-    return __builtin_fmaf(t, p, 1.0f);
+    const double a = __builtin_fma((double)h, 0x1.921fb6p+0, -0x1.921fb54442d18p-1);
+    const float af = (float)a;
+    const double s = a + (double)sin_tail(af, af * af);
+    return (float)__builtin_fma(s * -2.0, s, 1.0);
 }
 
 // tan(x) for |x| <= 0.75.
