@@ -17,10 +17,10 @@
 
 namespace om = onboard_math;
 
-enum { QUOTIENT, DIVISOR, ROOT, HYPOT, ATAN2, DIR_S, DIR_C, ATANH, COS, SIN_PI, TAN, WRAP, KINDS };
+enum { QUOTIENT, DIVISOR, ROOT, HYPOT, ATAN2, DIR_S, DIR_C, ATANH, COS, SIN_PI, TAN, WRAP, COS2, KINDS };
 static const char *const kNames[KINDS] = {"quotient", "divisor", "square_root", "hypotenuse",
                                           "atan2", "direction_s", "direction_c", "atanh", "cos",
-                                          "sin_half_turn", "tan", "wrap"};
+                                          "sin_half_turn", "tan", "wrap", "cosine_product"};
 
 template <bool TAME>
 __device__ float eval(int kind, float a, float b) {
@@ -36,6 +36,7 @@ __device__ float eval(int kind, float a, float b) {
     case COS: return om::cos_float<TAME>(a);
     case SIN_PI: return om::sin_half_turn(a);
     case TAN: return om::tan_float(a);
+    case COS2: return om::cosine_product(a, b);
     default: return om::wrap_angle<TAME>(a);
     }
 }
@@ -125,6 +126,7 @@ static long double truth(int kind, float a, float b) {
     case COS: return cosl(a);
     case SIN_PI: return sinl((long double)0x1.921fb6p+1f * a);
     case TAN: return tanl(a);
+    case COS2: return sqrtl((1.0L - (long double)a * a) * (1.0L - (long double)b * b));
     default: return remainderl(a, kTwoPi);
     }
 }
@@ -169,6 +171,10 @@ int main(void) {
             if (kind == ATANH) a[i] = sign() * (i % 2 ? 0.9999f * unit() : fminf(ldexpf(unit(), -(int)(next32() % 20)), 0.9999f));
             if (kind == ATANH && i % 1024 == 0) a[i] = sign() * 0.0f;
             if (kind == SIN_PI) a[i] = unit();
+            if (kind == COS2) {
+                a[i] = sign() * 0.35f * unit();
+                b[i] = sign() * 0.44f * unit();
+            }
             if (kind == TAN) a[i] = sign() * 0.75f * unit();
             if (kind == WRAP && i % 4 == 0) a[i] = sign() * 3.14159265f * (1.0f + ldexpf(sign() * unit(), -(int)(next32() % 24)));
             if ((kind == ATAN2 || kind == DIR_S || kind == DIR_C) && i % 8 == 0) {

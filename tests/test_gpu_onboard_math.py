@@ -12,7 +12,7 @@ adds its cosine's tail (0.02, so 0.05), and the cosine near a zero its
 remainder's 2^-41 over the ulp of 2^-16 where its result is measured (0.25).
 The half turn's sine is measured in ulp of 1, where its rounding is at most
 0.25; it is 1 - 2 s^2, and the tail of s, at most 0.08 with 2.5 ulp of single,
-adds 4 s 1.9e-8, at most 0.45.
+adds 4 s 1.9e-8, at most 0.45.  The cosine product is double throughout.
 The quotients and the square root are the IEEE ones, so exactly within half an
 ulp; one in 16 of their arguments has its result within 2^-47 (of a root within
 2^-41) of a rounding boundary.  For tame arguments both forms give the same bits, and
@@ -30,7 +30,7 @@ EXE = Path(__file__).resolve().parent / "csrc" / "bin" / "check_onboard_math"
 
 BOUND = {"quotient": 0.5, "divisor": 0.5, "square_root": 0.5, "hypotenuse": 0.501,
          "atan2": 0.501, "direction_s": 0.501, "direction_c": 0.501, "atanh": 0.6, "cos": 1.05,
-         "sin_half_turn": 0.75, "tan": 0.9, "wrap": 0.501}
+         "sin_half_turn": 0.75, "tan": 0.9, "wrap": 0.501, "cosine_product": 0.501}
 
 
 @pytest.mark.gpu

@@ -1246,11 +1246,8 @@ __device__ __forceinline__ ArmOutputs<QUAD> flight_values(const ChainInputs<QUAD
                                             -max_sin_inner, max_sin_inner);
         inner_cmd[i] = ob_clamp<TAME>(asinf(sin_in), -inner_limit * 0.90f, inner_limit * 0.90f);
         // cos(yaw_alpha) cos(inner_cmd), both arcsines (|sin_in| <= 0.44, so
-        // the limit on inner_cmd is never met): one square root of the
-        // product of the two squared cosines, which is at least 0.70.
-        const float nominal_cos =
-            fmaxf(__builtin_amdgcn_sqrtf(__builtin_fmaf(-sin_alpha, sin_alpha, 1.0f) *
-                                         __builtin_fmaf(-sin_in, sin_in, 1.0f)), 0.70f);
+        // the limit on inner_cmd is never met).
+        const float nominal_cos = fmaxf(onboard_math::cosine_product(sin_alpha, sin_in), 0.70f);
         const float lift_thrust = quotient<TAME>(fmaxf(fz_cmd, 0.0f), nominal_cos);
         const float target_thrust = land_idle ? idle_thrust : lift_thrust;
         const float u_des = ob_clamp<TAME>(

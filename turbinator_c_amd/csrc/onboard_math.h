@@ -226,6 +226,14 @@ __device__ __forceinline__ float sin_half_turn(float h) {
     return (float)__builtin_fma(s * -2.0, s, 1.0);
 }
 
+// cos(asin s) cos(asin t) for |s|, |t| <= 0.9: one square root of the product
+// of the two squared cosines.
+__device__ __forceinline__ float cosine_product(float sf, float tf) {
+    const double s = sf, t = tf;
+    const double p = __builtin_fma(-s, s, 1.0) * __builtin_fma(-t, t, 1.0);
+    return (float)(p * rsqrt47(p));
+}
+
 // tan(x) for |x| <= 0.75.
 __device__ __forceinline__ float tan_float(float xf) {
     const double x = xf, t = x * x;
