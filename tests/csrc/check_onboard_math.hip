@@ -183,6 +183,11 @@ int main(void) {
                 a[i] = sign() * (pick == 1 ? 0.0f : m);
                 b[i] = sign() * (pick == 2 ? 0.0f : m);
             }
+            if ((kind == HYPOT || kind == ATAN2 || kind == DIR_S || kind == DIR_C) && i % 32 == 5) {
+                // zeros and the least floats
+                a[i] = ldexpf((float)(hard32() % 4), -149) * (hard32() & 1 ? -1.0f : 1.0f);
+                b[i] = ldexpf((float)(hard32() % 4), -149) * (hard32() & 1 ? -1.0f : 1.0f);
+            }
         }
         for (size_t k = 0; k < tail; ++k) {
             a[tame_n + k] = special[k / ns];
@@ -204,15 +209,12 @@ int main(void) {
             const long double want = truth(kind, a[i], b[i]);
             // An ulp of the result; near a zero, of the magnitude below which
             // only the absolute error counts: the cosine's remainder is
-            // within 2^-41, the half turn's sine is added to 8, and a
-            // direction's zero component comes out as the least float over
-            // the other one.
+            // within 2^-41, and the half turn's sine is added to 8.
             const float w = fabsf((float)want);
             const float floor_mag = kind == COS ? 0x1p-16f
                                     : kind == WRAP ? 0x1p-20f
                                     : kind == SIN_PI ? 1.0f
-                                    : kind == DIR_S || kind == DIR_C ? 0x1p-100f
-                                                                     : 0x1p-126f;
+                                    : 0x1p-126f;
             const float mag = w > floor_mag ? w : floor_mag;
             const double ulp = (double)nextafterf(mag, inf) - (double)mag;
             const double e = (double)fabsl((long double)t[i] - want) / ulp;

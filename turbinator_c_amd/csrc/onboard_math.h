@@ -86,10 +86,16 @@ __device__ __forceinline__ float square_root(float x) {
     return limit ? x : s;  // infinity or NaN
 }
 
-// sqrt(x^2 + y^2); (0, 0) gives the least positive float, not 0.
+// |x| or 2^-500: what a sum of squares takes in place of an exact zero, so that
+// it can be divided by; it is far below the least float's share.
+__device__ __forceinline__ double above_tiny(float x) {
+    return __builtin_fmax((double)__builtin_fabsf(x), 0x1p-500);
+}
+
+// sqrt(x^2 + y^2).
 template <bool TAME>
 __device__ __forceinline__ float hypotenuse(float xf, float yf) {
-    const double x = above_zero(__builtin_fabsf(xf)), y = yf;
+    const double x = above_tiny(xf), y = yf;
     const double h2 = __builtin_fma(y, y, x * x);
     const float h = (float)(h2 * rsqrt47(h2));
     if constexpr (TAME) return h;
@@ -152,8 +158,7 @@ struct Direction {
     float s, c;
 };
 __device__ __forceinline__ Direction direction(float yf, float xf) {
-    const double y = yf;
-    const double x = __builtin_copysignf(above_zero(__builtin_fabsf(xf)), xf);
+    const double y = yf, x = __builtin_copysign(above_tiny(xf), (double)xf);
     const double r = rsqrt47(__builtin_fma(y, y, x * x));
     return Direction{(float)(y * r), (float)(x * r)};
 }
