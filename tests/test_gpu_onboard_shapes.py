@@ -58,6 +58,35 @@ def test_onboard_rows_do_not_depend_on_the_batch(torch_cuda, hip, tiled, diag):
             assert bool(same.all()), (n, k, torch.nonzero(~same)[:5].tolist())
 
 
+@pytest.mark.parametrize("n", [9000, 17000, 33000])
+def test_one_wild_arm_input(torch_cuda, hip, n):
+    """Ordinary environments with one arm input that is NaN, infinite or large:
+    a quad's lanes each read one arm, a lane of the largest batches all four,
+    and both must take the environment for the same kind of input."""
+    torch = torch_cuda
+    print(f"[gpu-case] onboard one wild arm input {n}", flush=True)
+    b = synth.make_batch(4096, seed=77, threads=16)
+    obs, e = in_window(b.obs), np.arange(4096)
+    wild = np.array([np.nan, np.inf, -np.inf, 1.2e4, -3.0e5], np.float32)
+    obs[e, 16 + e % 16] = wild[e // 16 % 5]
+    d_obs, d_mission = torch.from_numpy(obs).cuda(), torch.from_numpy(b.mission).cuda()
+    rows = torch.arange(n, device="cuda") % 4096
+
+    def run(o, m):
+        out = [torch.full((o.shape[0], w), 7.0, device="cuda") for w in (24, 15)]
+        s = torch.cuda.current_stream()
+        assert hip.onboard_tactical_prior_device(o, m, *out, None, o.shape[0], s) == 1
+        assert hip.synchronize(s) == 1
+        return out
+
+    small = run(d_obs, d_mission)
+    large = run(d_obs[rows].contiguous(), d_mission[rows].contiguous())
+    for k in range(2):
+        same = large[k].view(torch.int32) == small[k][rows].view(torch.int32)
+        assert bool(same.all()), (n, k, int((~same).any(1).sum()), torch.nonzero(~same)[:5].tolist())
+    compare(run_onboard(torch, hip, obs, b.mission), oracle.onboard(obs, b.mission), "wild arm")
+
+
 @pytest.mark.parametrize("n", [1, 47, 1024, 10000, 17000])
 def test_special_rows_in_every_shape(torch_cuda, hip, n):
     b = synth.make_batch(n, seed=500 + n, variant=synth.SPECIAL, threads=16)

@@ -730,26 +730,36 @@ __device__ __forceinline__ ChainInputs<QUAD> chain_inputs(const float *obs, cons
     return in;
 }
 
-// Whether a value that the lane reads is infinite, NaN or not below
-// onboard_math::kTameMax: unless the sum of their squares is below its square.
+// Whether an input of the environment is infinite, NaN or not below
+// onboard_math::kTameMax: unless for every arm the sum of its inputs' and the
+// shared inputs' squares is below its square.  The same flag in a quad's lanes
+// and in one lane per environment: ob_direction's results depend on it.
 template <bool QUAD>
 __device__ __forceinline__ bool wild_inputs(const ChainInputs<QUAD> &in) {
-    float s = 0.0f;
+    float shared = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 13; ++i) s = __builtin_fmaf(in.head[i], in.head[i], s);
+    for (int i = 0; i < 13; ++i) shared = __builtin_fmaf(in.head[i], in.head[i], shared);
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int k = 0; k < 6; ++k) shared = __builtin_fmaf(in.tail[k], in.tail[k], shared);
 #pragma unroll
-        for (int i = 0; i < kArms<QUAD>; ++i) s = __builtin_fmaf(in.arm[k][i], in.arm[k][i], s);
+    for (int i = 0; i < 10; ++i) shared = __builtin_fmaf(in.m[i], in.m[i], shared);
+    int wild = 0;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) s = __builtin_fmaf(in.tail[k], in.tail[k], s);
+    for (int i = 0; i < kArms<QUAD>; ++i) {
+        float s = shared;
 #pragma unroll
-    for (int i = 0; i < 10; ++i) s = __builtin_fmaf(in.m[i], in.m[i], s);
-    return !(s < onboard_math::kTameMax * onboard_math::kTameMax);
+        for (int k = 0; k < 4; ++k) s = __builtin_fmaf(in.arm[k][i], in.arm[k][i], s);
+        wild |= !(s < onboard_math::kTameMax * onboard_math::kTameMax);
+    }
+    if constexpr (QUAD) {
+        wild |= dpp_partner<0xB1>(wild);
+        wild |= dpp_partner<0x4E>(wild);
+    }
+    return wild != 0;
 }
 
-// Sine and cosine of atan2(y, x) from the components; a wild lane's are those
-// of the rounded angle, as the reference forms them: what they multiply may
+// Sine and cosine of atan2(y, x) from the components; a wild environment's are
+// those of the rounded angle, as the reference forms them: what they multiply may
 // be infinite or near the largest float, and then it matters that the sine of
 // a float near pi is about 1e-7 and not the exact value.
 template <bool TAME>
