@@ -42,8 +42,9 @@ int tb_cuda_synchronize(void *stream);
 typedef struct tb_cuda_feature_batch tb_cuda_feature_batch;
 
 /* Replaces cuda_features.h:26 (features.cu:27-44).  Makes `device_id`
- * current on the calling thread, creates a non-blocking stream and device
- * staging buffers for `max_batch` environments.  NULL when max_batch is 0 or
+ * current on the calling thread, creates a non-blocking stream and staging
+ * buffers for `max_batch` environments (pinned host memory up to 256, device
+ * memory above).  NULL when max_batch is 0 or
  * above 1024, when the device cannot be selected, or on any allocation
  * failure (partial state is released). */
 tb_cuda_feature_batch *tb_cuda_feature_batch_create(int device_id, size_t max_batch);

@@ -37,3 +37,23 @@ def test_host_object_equals_device_entry(torch_cuda, hip, max_batch):
                                        np.ascontiguousarray(b.cameras[rows]), count, got) == 1
             assert (got[count] == 7.0).all()
             assert np.array_equal(got[:count].view(np.uint32), want[rows]), count
+
+
+def test_small_handles_take_no_device_memory(torch_cuda, hip):
+    """A handle whose every batch goes through its pinned rows has no device
+    buffers: eight of them would take 69 MB."""
+    torch = torch_cuda
+    b = synth.make_batch(256, seed=10, threads=16)
+    got = np.empty((256, 142), np.float32)
+    with hip.FeatureBatch.create(0, 256) as handle:  # the runtime's own first allocations
+        assert handle.extract_host(b.obs, b.mission, b.cameras, 256, got) == 1
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    handles = [hip.FeatureBatch.create(0, 256) for _ in range(8)]
+    try:
+        taken = free - torch.cuda.mem_get_info()[0]
+        print(f"[gpu-case] eight handles of 256: {taken} bytes of device memory", flush=True)
+        assert taken < 16 << 20, taken
+    finally:
+        for handle in handles:
+            handle.destroy()

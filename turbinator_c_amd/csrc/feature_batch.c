@@ -2,7 +2,7 @@
  * Host staging object of the sensor-feature boundary, in C11 over the HIP
  * runtime C API.  Behaviour follows the reference host object
  * src/cuda/features.cu:9-88: a handle owns one non-blocking stream and
- * device buffers for up to max_batch (<= 1024) environments; extraction
+ * staging buffers for up to max_batch (<= 1024) environments; extraction
  * copies the caller's host arrays in, runs the device entry, copies the 142
  * features out and waits.  Failures record "<stage>: <runtime message>" in
  * the handle; argument errors return 0 and leave the text untouched.
@@ -10,9 +10,10 @@
  * Batches of up to FB_STAGE_MAX environments go through pinned memory of the
  * handle instead: the call copies FB_STAGE_ROWS environments at a time into
  * it and launches the extraction on them, which reads the rows over PCIe and
- * writes its features there, while the next rows are copied.  That leaves
- * out four copy-engine transfers and the runtime's own staging of pageable
- * memory.
+ * writes its features there, while the next rows, if any, are copied.  That
+ * leaves out four copy-engine transfers and the runtime's own staging of
+ * pageable memory.  Handles of up to FB_STAGE_MAX environments hold no device
+ * buffers.
  */
 #include <hip/hip_runtime_api.h>
 #include <stdio.h>
@@ -27,7 +28,6 @@ enum {
     FB_CAMERA = 16384,
     FB_FEATURES = 142,
     FB_MAX_BATCH = 1024,
-    FB_ROW_BYTES = (FB_OBS + FB_MISSION + FB_FEATURES) * 4 + FB_CAMERA,
     /* Pageable copies -> pinned rows, 32 at a time, us on one box with the
      * arrays in the host's caches: 1 environment 38.9 -> 19.1, 16 65.7 ->
      * 33.8, 32 80.0 -> 51.9, 64 119.6 -> 76.7, 128 180.8 -> 124.9, 256 295.6
@@ -46,13 +46,28 @@ struct tb_cuda_feature_batch {
     float *mission;
     unsigned char *cameras;
     float *features;
-    /* Pinned rows of the first stage_max environments, field by field in the
-     * order obs, cameras, features, mission (each section 16-byte aligned),
-     * and their device address; stage_max 0 when there is none. */
+    /* Pinned rows of up to stage_max environments (staged_rows) and their
+     * device address; stage_max 0 when there are none.  The device buffers
+     * above are NULL when stage_max is max_batch. */
     size_t stage_max;
     unsigned char *staged, *staged_device;
     char error[192];
 };
+
+/* Byte offsets of the pinned rows' sections for n environments: obs at 0, and
+ * each section on 16 bytes. */
+typedef struct {
+    size_t cameras, features, mission, end;
+} fb_sections;
+
+static fb_sections staged_rows(size_t n) {
+    fb_sections s;
+    s.cameras = n * FB_OBS * sizeof(float);
+    s.features = s.cameras + n * FB_CAMERA;
+    s.mission = (s.features + n * FB_FEATURES * sizeof(float) + 15) & ~(size_t)15;
+    s.end = s.mission + n * FB_MISSION * sizeof(float);
+    return s;
+}
 
 /* The device entry reads (and so clears) the launch error itself; a refused
  * launch whose error is already cleared is reported as a launch failure
@@ -79,24 +94,29 @@ tb_cuda_feature_batch *tb_cuda_feature_batch_create(int device_id, size_t max_ba
         tb_cuda_feature_batch_destroy(batch);
         return NULL;
     }
-    if (hipMalloc((void **)&batch->obs, max_batch * FB_OBS * sizeof(float)) != hipSuccess ||
-        hipMalloc((void **)&batch->mission, max_batch * FB_MISSION * sizeof(float)) != hipSuccess ||
-        hipMalloc((void **)&batch->cameras, max_batch * FB_CAMERA) != hipSuccess ||
-        hipMalloc((void **)&batch->features, max_batch * FB_FEATURES * sizeof(float)) != hipSuccess) {
-        tb_cuda_feature_batch_destroy(batch);
-        return NULL;
-    }
-    /* Without pinned memory every batch takes the copies. */
     batch->stage_max = max_batch < FB_STAGE_MAX ? max_batch : FB_STAGE_MAX;
-    if (hipHostMalloc((void **)&batch->staged, batch->stage_max * FB_ROW_BYTES,
+    if (hipHostMalloc((void **)&batch->staged, staged_rows(batch->stage_max).end,
                       hipHostMallocDefault) != hipSuccess) {
         batch->staged = NULL;
         batch->stage_max = 0;
         (void)hipGetLastError();
     } else if (hipHostGetDevicePointer((void **)&batch->staged_device, batch->staged, 0) !=
                hipSuccess) {
+        (void)hipHostFree(batch->staged);
+        batch->staged = NULL;
         batch->stage_max = 0;
         (void)hipGetLastError();
+    }
+    /* Only batches above the pinned rows take the copies; without pinned
+     * memory every batch does. */
+    if (max_batch > batch->stage_max &&
+        (hipMalloc((void **)&batch->obs, max_batch * FB_OBS * sizeof(float)) != hipSuccess ||
+         hipMalloc((void **)&batch->mission, max_batch * FB_MISSION * sizeof(float)) != hipSuccess ||
+         hipMalloc((void **)&batch->cameras, max_batch * FB_CAMERA) != hipSuccess ||
+         hipMalloc((void **)&batch->features, max_batch * FB_FEATURES * sizeof(float)) !=
+             hipSuccess)) {
+        tb_cuda_feature_batch_destroy(batch);
+        return NULL;
     }
     return batch;
 }
@@ -120,23 +140,20 @@ const char *tb_cuda_feature_batch_error(const tb_cuda_feature_batch *batch) {
 
 static int extract_staged(tb_cuda_feature_batch *batch, const float *obs, const float *mission,
                           const unsigned char *cameras, size_t count, float *out_features) {
-    const size_t n = batch->stage_max;
-    const size_t cameras_at = n * FB_OBS * sizeof(float);
-    const size_t features_at = cameras_at + n * FB_CAMERA;
-    const size_t mission_at = features_at + n * FB_FEATURES * sizeof(float);
+    const fb_sections at = staged_rows(batch->stage_max);
     unsigned char *const host = batch->staged, *const device = batch->staged_device;
     hipError_t launch = hipSuccess;
     for (size_t first = 0; first < count && launch == hipSuccess; first += FB_STAGE_ROWS) {
         const size_t rows = count - first < FB_STAGE_ROWS ? count - first : FB_STAGE_ROWS;
         const size_t o = first * FB_OBS, m = first * FB_MISSION, c = first * FB_CAMERA;
         memcpy(host + o * sizeof(float), obs + o, rows * FB_OBS * sizeof(float));
-        memcpy(host + mission_at + m * sizeof(float), mission + m,
+        memcpy(host + at.mission + m * sizeof(float), mission + m,
                rows * FB_MISSION * sizeof(float));
-        memcpy(host + cameras_at + c, cameras + c, rows * FB_CAMERA);
+        memcpy(host + at.cameras + c, cameras + c, rows * FB_CAMERA);
         if (!tb_cuda_extract_features_device(
-                (const float *)device + o, (const float *)(device + mission_at) + m,
-                device + cameras_at + c,
-                (float *)(device + features_at) + first * FB_FEATURES, rows, batch->stream))
+                (const float *)device + o, (const float *)(device + at.mission) + m,
+                device + at.cameras + c,
+                (float *)(device + at.features) + first * FB_FEATURES, rows, batch->stream))
             launch = launch_status();
     }
     /* Also after a refused launch: the rows launched before it are read from
@@ -144,7 +161,7 @@ static int extract_staged(tb_cuda_feature_batch *batch, const float *obs, const 
     const hipError_t status = hipStreamSynchronize(batch->stream);
     if (launch != hipSuccess) return fb_fail(batch, "extract features", launch);
     if (status != hipSuccess) return fb_fail(batch, "synchronize features", status);
-    memcpy(out_features, host + features_at, count * FB_FEATURES * sizeof(float));
+    memcpy(out_features, host + at.features, count * FB_FEATURES * sizeof(float));
     return 1;
 }
 
