@@ -523,7 +523,9 @@ void launch_diag(const Rows &rows, int lv, int cv, unsigned blocks, unsigned lds
 // Without cameras half as many bytes are in flight per workgroup and the cap
 // only costs: 16,384 environments 53.9 us at 4 per CU, 46.8 at 5, 45.6 at the
 // 7 of the kernel that also serves cameras, and 44.5 at the 8 that its own
-// instantiation's 60 registers allow (4,099: 15.3, 14.2, 13.2, 12.8).
+// instantiation's 60 registers allow (4,099: 15.3, 14.2, 13.2, 12.8).  The
+// diagnostics variant holds 6 per CU by its LDS, but its instantiation without
+// cameras gains too (16,384 environments 57.7 -> 55.3 us, 4,096 16.0 -> 14.8).
 // Indexed gathers, fp32 depth cameras and the diagnostics variant keep their
 // resource limit (4 per CU measured 91.9 -> 94.8, 208.0 -> 210.3 and 94.2 ->
 // 116.2 us).  The cap is dynamic LDS the kernel does not use: a workgroup

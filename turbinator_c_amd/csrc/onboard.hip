@@ -115,14 +115,8 @@ __device__ __forceinline__ float finite_as(float x, float limit) {
     const float y = inf ? copysignf(limit, x) : x;
     return nan ? 0.0f : y;
 }
-template <bool TAME = false>
-__device__ __forceinline__ float ob_obs(float x) {
-    return TAME ? x : finite_as(x, 1000.0f);
-}
-template <bool TAME = false>
-__device__ __forceinline__ float ob_mission(float x) {
-    return TAME ? x : finite_as(x, 1.0f);
-}
+__device__ __forceinline__ float ob_obs(float x) { return finite_as(x, 1000.0f); }
+__device__ __forceinline__ float ob_mission(float x) { return finite_as(x, 1.0f); }
 // atan2 and the angle wrap.  ob_wrap is discontinuous where its two angles
 // differ by pi, and that is reached exactly by angles such as -3pi/4 and pi/4
 // (from equal or zero components), or pi and a yaw of +-0: there one ulp of
@@ -791,10 +785,10 @@ __device__ __forceinline__ void controller_inputs(ChainInputs<QUAD> &in) {
     for (int i = 0; i < 10; ++i) in.m[i] = ob_mission(in.m[i]);
 }
 
-// Two of them.
 struct Direction2 {
     float s0, c0, s1, c1;
 };
+// Two directions; on a quad lane 0 forms the first and the others the second.
 template <bool TAME, bool QUAD>
 __device__ __forceinline__ Direction2 directions(int a, float y0, float x0, float y1, float x1,
                                                  bool wild) {
@@ -903,10 +897,7 @@ __device__ __forceinline__ void tactical_values(const ChainInputs<QUAD> &in, boo
 }
 
 // The reference's last mapping (NaN -> 0, +-inf -> +-1).
-template <bool TAME>
-__device__ __forceinline__ float tactical_out(float x) {
-    return TAME ? x : finite_as(x, 1.0f);
-}
+__device__ __forceinline__ float tactical_out(float x) { return finite_as(x, 1.0f); }
 
 // The mission's flags (onboard_features.cuh:107-109, 126-136, 433-437).
 struct MissionFlags {
@@ -1819,8 +1810,7 @@ __device__ __forceinline__ void support_wave(const OnboardRows &rows, size_t bas
         else tactical_values<false, true>(in, wild, a, v);
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
-            const float x = quad_pick(a, v[k], v[6 + k], v[12 + k], v[18 + k]);
-            t[k] = tactical_out<false>(x);
+            t[k] = tactical_out(quad_pick(a, v[k], v[6 + k], v[12 + k], v[18 + k]));
         }
     }
 #pragma unroll
@@ -1899,7 +1889,7 @@ __device__ __forceinline__ void tactical_lanes(const Stage<64> &stage, int lane,
     if (__builtin_amdgcn_ballot_w64(wild) == 0) tactical_values<true, false>(in, wild, 0, v);
     else tactical_values<false, false>(in, wild, 0, v);
 #pragma unroll
-    for (int k = 0; k < 24; ++k) out.tactical[lane][k] = tactical_out<false>(v[k]);
+    for (int k = 0; k < 24; ++k) out.tactical[lane][k] = tactical_out(v[k]);
 }
 
 __device__ __forceinline__ void gunnery_lanes(const Stage<64> &stage, int lane, LaneRows &out) {
