@@ -155,12 +155,13 @@ def test_config_16384(torch_cuda, hip):
     check_h2(sub, want, "16384")
 
 
-@pytest.mark.parametrize("n", [300, 1024, 2048, 2560])
+@pytest.mark.parametrize("n", [300, 1024, 2048, 3071, 3072, 3500])
 def test_lidar_or_luma_alone(torch_cuda, hip, n):
-    """The scan kernel writes the channel planes of elevation rows 0..5 and
-    the plane kernel the other rows: each plane output requested alone, at a
-    one-stream batch and at one that overlaps the two streams, is complete
-    and bit-exact against numpy for every environment."""
+    """Each plane output requested alone is complete and bit-exact against
+    numpy for every environment: in the one launch of batches below 3,072, and
+    in the two-stream form from there, where the scan kernel writes the
+    channel planes of elevation rows 0..5 and the plane kernel the other rows
+    (without LiDAR channels the onboard kernel runs beside it)."""
     note(f"actor inputs, lidar or luma alone, {n} envs")
     b = synth.make_batch(n, seed=700 + n, threads=16)
     got = run_actor(torch_cuda, hip, b.obs, b.mission, None, lidar=True, luma=False)
@@ -186,32 +187,34 @@ def _device_batch(torch, n, seed):
 
 
 def test_mode_thresholds_and_null_stream(torch_cuda, hip):
-    """The entry picks its mode by batch: one stream below 1,792
-    environments, with the scan kernel writing its rows' LiDAR channels from
-    512; two streams from 1,792, with that split from 2,560.  Every call on
-    either side of each threshold must equal the 2,560-row call on their
-    common rows, bit for bit, and a call on the null stream must equal one on
-    a torch stream."""
+    """The entry picks its form by batch: one launch below 3,072 environments
+    (with 8 of them per onboard workgroup up to 512, 16 above), two streams
+    from there.  Every call on either side of each threshold must equal the
+    3,500-row call on their common rows, bit for bit, and two-stream calls on
+    the null stream must equal those on a torch stream.  Only the call's
+    stream is waited for, so work of the second stream that is not joined
+    back to it would show."""
     torch = torch_cuda
     names = ("proprio", "mission", "tactical", "prior", "lidar", "luma")
-    note("actor inputs: mode thresholds 512 / 1792 / 2560, null stream")
-    d_in, out = _device_batch(torch, 2560, seed=2560)
+    note("actor inputs: mode thresholds 512 / 3072, null stream")
+    d_in, out = _device_batch(torch, 3500, seed=2560)
     s = torch.cuda.current_stream()
     torch.cuda.synchronize()
-    full = _call_all(torch, hip, d_in, out, 2560, s, s)
-    for n in (511, 512, 1791, 1792, 2559):
+    full = _call_all(torch, hip, d_in, out, 3500, s, s)
+    for n in (511, 512, 513, 3071, 3072, 3073):
         for t in out:
             t.fill_(float("nan"))
         torch.cuda.synchronize()
         part = _call_all(torch, hip, d_in, out, n, s, s)
         for name, g, w in zip(names, full, part):
-            assert np.array_equal(g[:n], w), f"{name}: {n}-row call differs from 2560-row call"
-    for t in out:
-        t.fill_(float("nan"))
-    torch.cuda.synchronize()
-    null = _call_all(torch, hip, d_in, out, 2560, None, None)
-    for name, g, w in zip(names, null, full):
-        assert np.array_equal(g, w), f"{name}: null-stream call differs"
+            assert np.array_equal(g[:n], w), f"{name}: {n}-row call differs from 3500-row call"
+    for n in (3072, 3500):
+        for t in out:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        null = _call_all(torch, hip, d_in, out, n, None, None)
+        for name, g, w in zip(names, null, full):
+            assert np.array_equal(g, w[:n]), f"{name}: null-stream call of {n} rows differs"
 
 
 def test_concurrent_callers_on_their_own_streams(torch_cuda, hip):
@@ -287,13 +290,12 @@ def test_graph_capture_with_the_second_stream(torch_cuda, hip):
 
 
 def test_more_than_64_environments_per_scan_wave(torch_cuda, hip):
-    """As for the onboard entry: 263,144 rows tiled from 4,096 distinct
-    environments (the scan waves form a second group of 64 frames, and the
-    control kernel's workgroups, which also write the symlog scalars, loop
-    past their 4,096-workgroup cap); proprio, mission, tactical and prior
-    rows must equal the 4,096-row call's bit for bit, and so must the LiDAR
-    channels (the scan waves write those of their rays), compared on the
-    device.  Luma is left out (no scan wave writes it)."""
+    """263,144 rows tiled from 4,096 distinct environments: the persistent
+    scan waves form a second group of 64 frames, and the control kernel, which
+    also writes the symlog scalars, runs 4,112 workgroups; proprio, mission,
+    tactical and prior rows must equal the 4,096-row call's bit for bit, and so
+    must the LiDAR channels (the scan waves write those of their rays),
+    compared on the device.  Luma is left out (no scan wave writes it)."""
     torch = torch_cuda
     distinct, batch = 4096, 64 * 4096 + 1000
     note(f"actor inputs {batch} envs tiled from {distinct}")

@@ -306,10 +306,10 @@ MISSION_CLASSES = [(0.0, 0.0), (0.0, 1.0), (1.0, 0.0), (1.0, 0.5), (0.75, 0.0),
 
 @pytest.mark.parametrize("variant", [0, 3, 5, 6])
 def test_scan_uses_by_mission(torch_cuda, hip, variant):
-    """The scan kernel computes only what an environment's mission uses of
-    the scan (nothing, the closest return, or the corridor and cluster),
-    unless the diagnostics row is asked for.  On 9,000 environments (so most
-    scan waves take three, with their needs mixed) cycling through the
+    """The scan computes only what an environment's mission uses of it
+    (nothing, the closest return, or the corridor and cluster), unless the
+    diagnostics row is asked for.  On 9,000 environments (18 per workgroup, so
+    that a scanning wave takes several, with their needs mixed) cycling through the
     mission classes above, the call without diagnostics must equal the call
     with them bit for bit, and both the oracle."""
     note(f"onboard scan uses by mission, variant {variant}, 9000 envs")
@@ -335,21 +335,20 @@ def test_scan_uses_by_mission(torch_cuda, hip, variant):
     note(f"scan uses variant {variant}: {stats}")
 
 
-@pytest.mark.parametrize("n,classes", [(2560, "mixed"), (2561, "mixed"), (4097, "mixed"),
-                                       (10240, "mixed"), (16384, "slalom"), (16384, "dodge"),
-                                       (16384, "bwb"), (16385, "mixed")])
+@pytest.mark.parametrize("n,classes", [(2048, "mixed"), (2049, "mixed"), (4097, "mixed"),
+                                       (8192, "slalom"), (8193, "mixed"), (16384, "slalom"),
+                                       (16384, "dodge"), (16384, "bwb"), (16385, "mixed"),
+                                       (20000, "slalom"), (20000, "dodge"), (20000, "bwb"),
+                                       (33000, "slalom")])
 def test_pooled_scan_sizes(torch_cuda, hip, n, classes):
-    """The H2 entry's scan forms by batch: from 2,560 environments the scan
-    kernel shares each workgroup's environments out from a pool in LDS, with
-    at least 16 per workgroup and at most 256 workgroups: the smallest pooled
-    batch (160 workgroups of 16), one more (161 workgroups, 15 or 16 each)
-    and one more than a full grid of 16 (4,097: the first workgroup takes
-    17).  From 10,240 to 16,384 environments one kernel scans and controls
-    each workgroup's 64 environments: its smallest batch, and full batches
-    whose every mission uses the corridor scan or the closest return (the
-    pool holds every environment) or is a BWB mission that uses no scan
-    result (every controller wave runs the BWB blocks).  16,385 goes back to
-    two kernels.
+    """A workgroup's scanning waves take its environments from a pool in LDS.
+    The shapes by batch: up to 2,048 environments workgroups take 8 each, up
+    to 8,192 up to 16 (one group), to 16,384 up to 32 (two groups), above up
+    to 64 (four groups, the chains on one lane per environment), and above
+    32,768 a rest in smaller shares.  On either side of each bound mixed
+    missions, and full pools in every shape: all missions use the corridor
+    scan, all the closest return, or all are BWB missions that use no scan
+    result (the pool is empty and every support wave runs the BWB blocks).
     Without diagnostics the call must equal the call with them bit for bit,
     and both the oracle on a sample."""
     note(f"onboard pooled scan, {n} envs, {classes} missions")
@@ -363,7 +362,7 @@ def test_pooled_scan_sizes(torch_cuda, hip, n, classes):
             mission[cls == c, 5] = m5
     elif classes == "bwb":
         # BWB cruise (m4 > 0.75, m2 > 0.25) with m5 = 0.5 (lateral: no scan
-        # result used), so every controller wave runs the BWB blocks.
+        # result used), so every support wave runs the BWB blocks.
         mission[:, 2], mission[:, 4], mission[:, 5] = 0.5, 1.0, 0.5
     else:
         mission[:, 4], mission[:, 5] = (1.0, 0.0) if classes == "slalom" else (0.0, 1.0)
@@ -378,12 +377,12 @@ def test_pooled_scan_sizes(torch_cuda, hip, n, classes):
     note(f"pooled scan {n} {classes}: {stats}")
 
 
-@pytest.mark.parametrize("n", [2560, 10240, 16385])
+@pytest.mark.parametrize("n", [2049, 4097, 8193, 16385, 32769])
 def test_scan_forms_agree(torch_cuda, hip, n):
-    """The H2 entry changes form at these batches: a static share of the
-    environments per scan wave below 2,560, the pooled scan kernel from
-    there, one kernel for scan and control from 10,240 to 16,384, and the
-    pooled scan kernel again above.  The same n environments (missions
+    """The H2 entry changes its workgroups' shape at these batches: the least
+    share of 8 up to 2,048, two workgroups per CU from 4,097, two groups from
+    8,193, four groups with one lane per environment from 16,385, and a rest
+    beside whole rounds from 32,769.  The same n environments (missions
     cycling through every class) called as n - 1 and as n must give the same
     first n - 1 rows bit for bit, with and without diagnostics."""
     torch = torch_cuda
@@ -408,16 +407,17 @@ def test_scan_forms_agree(torch_cuda, hip, n):
 
 @pytest.mark.parametrize("variant", [synth.SPECIAL, synth.CLAMP_LIMITS, synth.TIED_MINIMA,
                                      synth.EDGE_QUARTERS, synth.NO_RETURN])
-def test_one_kernel_form_on_variants(torch_cuda, hip, variant):
-    """The one-kernel form (10,240 to 16,384 environments) on the generator's
-    adversarial variants (NaN / +-Inf / +-0 / 3e38 inputs, clamp limits,
-    tied minima, edge quarters, no returns), ranges scaled into the scan
-    window: 4,096 distinct environments tiled three times on the device must
-    give, row for row, the bits of the 4,096-row call (the pooled scan kernel
-    and the control kernel), with and without diagnostics."""
+@pytest.mark.parametrize("reps", [3, 5])
+def test_group_shapes_on_variants(torch_cuda, hip, variant, reps):
+    """The shapes of two groups (12,288 environments) and of four (20,480, one
+    lane per environment) on the generator's adversarial variants (NaN /
+    +-Inf / +-0 / 3e38 inputs, clamp limits, tied minima, edge quarters, no
+    returns), ranges scaled into the scan window: 4,096 distinct environments
+    tiled on the device must give, row for row, the bits of the 4,096-row
+    call (one group per workgroup), with and without diagnostics."""
     torch = torch_cuda
-    distinct, reps = 4096, 3
-    note(f"onboard one-kernel form, variant {variant}, {distinct * reps} envs")
+    distinct = 4096
+    note(f"onboard group shapes, variant {variant}, {distinct * reps} envs")
     b = synth.make_batch(distinct, seed=5300 + variant, variant=variant, threads=16)
     obs = torch.from_numpy(in_window(b.obs)).cuda()
     mission = torch.from_numpy(b.mission).cuda()
@@ -445,17 +445,15 @@ def test_one_kernel_form_on_variants(torch_cuda, hip, variant):
                 f"variant {variant} diag {with_diag}: rows differ"
 
 
-def test_more_than_64_environments_per_scan_wave(torch_cuda, hip):
-    """The onboard entry's scan takes up to 1,024 environments per workgroup
-    and round (256 workgroups), so a batch beyond 262,144 makes every
-    workgroup take a second round.  4,096 distinct environments are tiled on
-    the device
-    to 263,144 rows (4.4 GB of observations); every row must equal, bit for
-    bit, the same environment's row from the 4,096-row call, with and without
-    the diagnostics row."""
+def test_many_rounds_of_workgroups(torch_cuda, hip):
+    """A batch of nine rounds of workgroups: eight whole rounds of 32,768 and a
+    rest of 1,000 in equal shares.  4,096 distinct environments are tiled on
+    the device to 263,144 rows (4.4 GB of observations); every row must equal,
+    bit for bit, the same environment's row from the 4,096-row call, with and
+    without the diagnostics row."""
     torch = torch_cuda
     distinct, batch = 4096, 64 * 4096 + 1000
-    note(f"onboard {batch} envs tiled from {distinct} (second round)")
+    note(f"onboard {batch} envs tiled from {distinct}")
     b = synth.make_batch(distinct, seed=271, threads=16)
     obs = torch.from_numpy(in_window(b.obs)).cuda()
     mission = torch.from_numpy(b.mission).cuda()
