@@ -207,14 +207,10 @@ int main(void) {
         for (size_t i = 0; i < tame_n; ++i) {
             differ += memcmp(&t[i], &g[i], 4) != 0;
             const long double want = truth(kind, a[i], b[i]);
-            // An ulp of the result; near a zero, of the magnitude below which
-            // only the absolute error counts: the cosine's remainder is
-            // within 2^-41, and the half turn's sine is added to 8.
+            // An ulp of the result; the half turn's sine is added to 8, so an
+            // ulp of 1, and a wrapped angle's remainder is within 2^-42.
             const float w = fabsf((float)want);
-            const float floor_mag = kind == COS ? 0x1p-16f
-                                    : kind == WRAP ? 0x1p-20f
-                                    : kind == SIN_PI ? 1.0f
-                                    : 0x1p-126f;
+            const float floor_mag = kind == SIN_PI ? 1.0f : kind == WRAP ? 0x1p-20f : 0x1p-126f;
             const float mag = w > floor_mag ? w : floor_mag;
             const double ulp = (double)nextafterf(mag, inf) - (double)mag;
             const double e = (double)fabsl((long double)t[i] - want) / ulp;

@@ -200,13 +200,15 @@ __device__ __forceinline__ float cos_tail(float t) {
     return t * t * p;
 }
 
-// cos(x): the remainder of x by pi/2 (within 2^-41 up to
-// kTameMax) and the quadrant's function of it.
+// cos(x): the remainder of x by pi/2 (two terms, so that it is exact to 2^-52 of
+// itself near the zeros of the cosine up to kTameMax) and the quadrant's
+// function of it.
 template <bool TAME>
 __device__ __forceinline__ float cos_float(float xf) {
     const double x = xf;
     const double n = __builtin_rint(x * 0x1.45f306dc9c883p-1);  // 2 / pi
-    const double r = __builtin_fma(n, -0x1.921fb54442d18p+0, x);
+    const double r =
+        __builtin_fma(n, -0x1.1a62633145c07p-54, __builtin_fma(n, -0x1.921fb54442d18p+0, x));
     const int quadrant = (int)n;
     const double t = r * r;
     const float tf = (float)t;
