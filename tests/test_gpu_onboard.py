@@ -345,7 +345,7 @@ def test_pooled_scan_sizes(torch_cuda, hip, n, classes):
     The shapes by batch: up to 2,048 environments workgroups take 8 each, up
     to 8,192 up to 16 (one group), to 16,384 up to 32 (two groups), above up
     to 64 (four groups, the chains on one lane per environment), and above
-    32,768 a rest in smaller shares.  On either side of each bound mixed
+    32,768 a rest in shares of 32.  On either side of each bound mixed
     missions, and full pools in every shape: all missions use the corridor
     scan, all the closest return, or all are BWB missions that use no scan
     result (the pool is empty and every support wave runs the BWB blocks).
@@ -447,7 +447,7 @@ def test_group_shapes_on_variants(torch_cuda, hip, variant, reps):
 
 def test_many_rounds_of_workgroups(torch_cuda, hip):
     """A batch of nine rounds of workgroups: eight whole rounds of 32,768 and a
-    rest of 1,000 in equal shares.  4,096 distinct environments are tiled on
+    rest of 1,000 in shares of 32.  4,096 distinct environments are tiled on
     the device to 263,144 rows (4.4 GB of observations); every row must equal,
     bit for bit, the same environment's row from the 4,096-row call, with and
     without the diagnostics row."""

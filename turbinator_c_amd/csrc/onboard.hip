@@ -1637,18 +1637,21 @@ constexpr unsigned kMinShare = 8;
 constexpr size_t kCus = 256, kRoundBlocks = 512;  // workgroups resident at once: two per CU
 
 // Above one round of 64 environments in every workgroup the last round holds
-// the rest.  Up to half a round of it goes over all CUs in equal shares, one
-// workgroup each; in shares of 64 it left most of them idle, and a workgroup
-// alone on its CU took as long as before (us, as generated / cluttered
-// slaloms; two launches, shares of 64, equal shares of the rest):
-//   34,000  54.4 / 118.7   33.1 / 133.6   29.6 / 89.9
-//   39,999  59.3 / 133.2   33.6 / 135.1   32.2 / 110.5
-//   45,000  62.3 / 144.4   35.1 / 136.3   35.1 / 126.3
-//   70,000  99.3 / 221.4   52.0 / 207.4   51.0 / 176.3
-// (65,600, 64 above two rounds: 95.6 / 211.4, 45.8 / 201.9, 47.2 / 169.3.)
+// the rest.  A rest of up to one workgroup of 32 for each CU is shared out by
+// 32: in shares of 64 a few CUs kept the others waiting, which in scenes full
+// of scans took longer than two launches.  Smaller shares gain more there and
+// lose in open scenes, whose last workgroups start when the first of the
+// round before end; above 8,192 the same holds for shares of 32.  us, scenes
+// as generated / with a quarter of the returns within 12 m / cluttered, every
+// mission a slalom (two launches; shares of 64; the rest by 32; over all CUs):
+//   34,000  51.4 / 55.3 / 118.9  31.4 / 35.7 / 133.8  29.7 / 33.6 / 110.2  30.0 / 33.6 / 90.3
+//   39,999  54.8 / 58.3 / 133.0  32.7 / 37.0 / 135.3  32.2 / 36.4 / 112.0  33.3 / 37.8 / 110.8
+//   45,000  57.8 / 61.3 / 144.0  35.4 / 39.5 / 135.9  37.5 / 41.4 / 131.7  36.3 / 41.5 / 126.6
+//   70,000  89.8 / 93.4 / 220.6  50.0 / 55.7 / 207.1  49.6 / 55.0 / 185.3  50.9 / 56.0 / 176.8
 // (Equal shares over both rounds lose: 39,999 at 40 each cluttered 45.2 us for
 // 40.7, since a CU's last workgroup alone runs faster than two.)
-constexpr size_t kRoundRows = 64 * kRoundBlocks, kRestRows = 64 * kCus;
+constexpr unsigned kRestShare = 32;
+constexpr size_t kRoundRows = 64 * kRoundBlocks, kRestRows = kRestShare * kCus;
 constexpr int kPoolWaves = kControlThreads / 64;
 
 // The inputs of N environments in LDS: obs[0..47], mission[0..9], the scan
@@ -2166,23 +2169,19 @@ __device__ __forceinline__ void onboard_block(const OnboardRows &rows, size_t ba
     }
 }
 
-// `share` environments per workgroup, at most 16 G; with REST (G = 4) those
-// after the batch's whole rounds of 64 each.
+// `share` environments per workgroup, at most 16 G; with REST (G = 4) 64 in the
+// batch's whole rounds and kRestShare after them.
 template <int G, bool REST = false>
 __global__ __launch_bounds__(kControlThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void onboard_kernel(OnboardRows rows, unsigned share) {
     __shared__ OnboardLds<G> lds;
-    size_t block = (size_t)blockIdx.y * gridDim.x + blockIdx.x, first = 0;
+    const size_t block = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+    size_t base = block * share;
     if constexpr (REST) {
         const size_t whole = rows.batch / kRoundRows * kRoundBlocks;
-        if (block < whole) {
-            share = 64;
-        } else {
-            first = 64 * whole;
-            block -= whole;
-        }
+        share = block < whole ? 64 : kRestShare;
+        base = 64 * block - (block < whole ? 0 : (64 - kRestShare) * (block - whole));
     }
-    const size_t base = first + block * share;
     if (base >= rows.batch) return;
     if (rows.batch - base > share) rows.batch = base + share;  // this workgroup's end
     onboard_block<G, false>(rows, base, lds);
@@ -2223,10 +2222,9 @@ extern "C" int tb_hip_onboard_tactical_prior_device(const float *obs, const floa
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     (void)hipGetLastError();
     const size_t rest = batch_size % kRoundRows;
-    if (batch_size > kRoundRows && rest != 0 && rest < kRestRows) {
-        const size_t share = (rest + kCus - 1) / kCus;
-        onboard_kernel<4, true><<<wide_grid((batch_size - rest) / 64 + (rest + share - 1) / share),
-                                  kControlThreads, 0, s>>>(rows, (unsigned)share);
+    if (batch_size > kRoundRows && rest != 0 && rest <= kRestRows) {
+        const size_t blocks = (batch_size - rest) / 64 + (rest + kRestShare - 1) / kRestShare;
+        onboard_kernel<4, true><<<wide_grid(blocks), kControlThreads, 0, s>>>(rows, kRestShare);
         return hipGetLastError() == hipSuccess;
     }
     const size_t want = share_of(batch_size), share = want < 64 ? want : 64;
