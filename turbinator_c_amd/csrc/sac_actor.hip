@@ -790,6 +790,14 @@ void launch_shape(const ActArgs &a, hipStream_t s) {
 //               16,384 12.0 / 9.3 / 9.0, 16,500 14.4 / 12.8 / 15.7, 65,536 41.4 / 30.1 / 32.2
 //   hidden 256: 256 rows 7.7 / 9.4 / 12.3, 4,096 8.4 / 9.5 / 12.6, 8,192 14.8 / 9.7 / 12.7,
 //               16,384 28.9 / 19.1 / 14.3, 40,000 68.2 / 44.5 / 38.6
+// Between these widths the lines lie in the same places (80, 112, 144, 176, 208
+// and 240 measured at 256 to 65,536 rows: the shape taken is the fastest):
+//   hidden 112: 4,096 rows 4.9 / 6.3 / 8.2, 8,192 6.9 / 6.4 / 8.2, 16,384 11.3 / 8.9 / 8.4,
+//               16,500 13.3 / 12.2 / 15.2, 65,536 39.8 / 29.0 / 31.6
+//   hidden 144: 4,096 rows 6.9 / 8.2 / 10.5, 8,192 12.5 / 8.4 / 10.5, 16,384 23.7 / 15.8 / 10.8,
+//               16,500 28.7 / 22.2 / 19.8, 65,536 91.0 / 60.1 / 41.2
+//   hidden 208: 4,096 rows 7.6 / 9.1 / 12.0, 8,192 13.9 / 9.5 / 12.0, 16,384 26.4 / 17.8 / 12.7,
+//               16,500 32.0 / 25.1 / 23.1, 65,536 102 / 68.9 / 49.4
 constexpr size_t kOneGroupMax = 4096, kTwoGroupMax = 8192, kFullMax = 16384;
 
 template <int HT>
