@@ -59,6 +59,40 @@ def test_onboard_rows_do_not_depend_on_the_batch(torch_cuda, hip, tiled, diag):
             assert bool(same.all()), (n, k, torch.nonzero(~same)[:5].tolist())
 
 
+@pytest.mark.parametrize("small,large,most", [(8, 64, 1.3), (8192, 9000, 1.43),
+                                              (32768, 34000, 1.39)])
+def test_scans_are_shared_out(torch_cuda, hip, small, large, most):
+    """Where every environment is scanned through clutter, a batch a little
+    above a shape's bound must not take much longer than one at it: its
+    workgroups are spread over the CUs.  With 16, 32 and 64 environments in
+    every workgroup the larger batches took 1.46, 1.67 and 1.53 times the
+    smaller ones' time, in shares 1.14, 1.19 and 1.25; the bounds lie halfway.
+    Medians of alternating runs of one device, so that clocks cancel."""
+    torch = torch_cuda
+    print(f"[gpu-case] onboard times {small} / {large}", flush=True)
+    b = synth.make_batch(4096, seed=79, threads=16)
+    mission = b.mission.copy()
+    mission[:, 4], mission[:, 5] = 1.0, 0.0  # slalom
+    rows = torch.arange(large, device="cuda") % 4096
+    obs = torch.from_numpy(in_window(b.obs)).cuda()[rows].contiguous()
+    d_mission = torch.from_numpy(mission).cuda()[rows].contiguous()
+    out = [torch.empty((large, w), device="cuda") for w in (24, 15, 5)]
+    s = torch.cuda.current_stream()
+    times = {small: [], large: []}
+    for _ in range(15):
+        for n in times:
+            first, last = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            first.record(s)
+            for _ in range(100):
+                assert hip.onboard_tactical_prior_device(obs, d_mission, *out, n, s) == 1
+            last.record(s)
+            last.synchronize()
+            times[n].append(first.elapsed_time(last) * 10.0)
+    at = {n: float(np.median(t)) for n, t in times.items()}
+    print(f"[gpu-case] us {at}", flush=True)
+    assert at[large] < most * at[small], at
+
+
 @pytest.mark.parametrize("n", [9000, 17000, 33000])
 def test_one_wild_arm_input(torch_cuda, hip, n):
     """Ordinary environments with one arm input that is NaN, infinite or large:
